@@ -148,6 +148,8 @@ struct remc_ctx {
     int rec_max = 0;
     unsigned long long *d_slots = nullptr;
     int *d_err = nullptr;
+    uint32_t *h_pin = nullptr; // pinned host memory that read-backs go through (ReadBack)
+    size_t pin_words = 0;
     double *d_adj = nullptr; // adjoint scratch: bead gradients, tile partials, body forces, parameter gradients
     size_t adj_cap = 0;      // doubles held by d_adj
     int adj_target = 0;      // all-replica adjoint's workgroup target (0: tune on first use)
@@ -600,6 +602,9 @@ int finalize(remc_ctx *c)
         c->max_bodies = std::max(c->max_bodies, sy.n_bodies);
         c->max_body_beads = std::max(c->max_body_beads, sy.max_body);
     }
+    // the largest read-back: one replica's state, or the counters of all (and the error flag)
+    c->pin_words = std::max((size_t)6 * c->max_beads + (size_t)11 * c->max_bodies, (size_t)8 * R) + 8;
+    HIP_TRY(hipHostMalloc((void **)&c->h_pin, 4 * c->pin_words, hipHostMallocDefault));
     HIP_TRY(hipStreamSynchronize(s));
     c->synced_copies = 1;
     c->finalized = true;
@@ -645,18 +650,66 @@ int sync_copies(remc_ctx *c, int coop)
     return REMC_OK;
 }
 
-// Reads and clears the device error flag of the cooperative MC kernel.
-int check_err(remc_ctx *c)
+// Device arrays read back together: add() each (a null destination is left
+// out), then run() packs them into the context's pinned memory by one launch,
+// waits once and copies them out.
+struct ReadBack {
+    remc_ctx *c;
+    Gather g{};
+    void *out[GATHER_MAX];
+    explicit ReadBack(remc_ctx *c_) : c(c_) {}
+    // words: 32-bit words of the array
+    void add(void *dst, const void *src, size_t words)
+    {
+        if (!dst) return;
+        g.src[g.n] = (const uint32_t *)src;
+        out[g.n] = dst;
+        g.at[g.n + 1] = g.at[g.n] + (uint32_t)words;
+        ++g.n;
+    }
+    int run()
+    {
+        if (g.at[g.n] > c->pin_words) return fail(REMC_ERR_STATE, "read-back of %u words exceeds its buffer", g.at[g.n]);
+        HIP_TRY(launch_gather(g, c->h_pin, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        for (int k = 0; k < g.n; ++k) std::memcpy(out[k], c->h_pin + g.at[k], 4 * (size_t)(g.at[k + 1] - g.at[k]));
+        return REMC_OK;
+    }
+};
+
+// Reports the device error flag of the cooperative MC kernel (read as err) and clears it.
+int report_err(remc_ctx *c, int err)
 {
-    int err = 0;
-    HIP_TRY(hipMemcpyAsync(&err, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
     if (err) {
         int zero = 0;
         HIP_TRY(hipMemcpyAsync(c->d_err, &zero, sizeof(int), hipMemcpyHostToDevice, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
         return fail(REMC_ERR_DEVICE, "cooperative MC workgroups did not meet within the wait limit; replica state is invalid");
     }
+    return REMC_OK;
+}
+
+int check_err(remc_ctx *c)
+{
+    int err = 0;
+    ReadBack rb(c);
+    rb.add(&err, c->d_err, 1);
+    const int rc = rb.run();
+    return rc != REMC_OK ? rc : report_err(c, err);
+}
+
+// Full (noncrowder_only 0) or non-crowder energies of every replica into out:
+// the sum kernel writes the totals straight into the pinned read-back memory.
+int energies_out(remc_ctx *c, int noncrowder_only, double *out)
+{
+    const int R = (int)c->reps.size();
+    {
+        TimedLaunch t(c, 1);
+        HIP_TRY(launch_energy_full(c->params(), R, c->max_tiles, c->d_full_partials, (double *)c->h_pin, noncrowder_only,
+                                   0, c->full_split, c->stream));
+    }
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    std::memcpy(out, c->h_pin, sizeof(double) * R);
     return REMC_OK;
 }
 
@@ -1112,6 +1165,7 @@ int remc_ctx_destroy(remc_ctx *c)
                     c->d_ana};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    if (c->h_pin) (void)hipHostFree(c->h_pin);
     for (auto e : c->free_events) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1278,14 +1332,7 @@ int remc_energy_all(remc_ctx *c, double *out)
     CHECK_CTX(c);
     FINALIZE(c);
     if (!out) return fail(REMC_ERR_ARG, "null output");
-    const int R = (int)c->reps.size();
-    {
-        TimedLaunch t(c, 1);
-        HIP_TRY(launch_energy_full(c->params(), R, c->max_tiles, c->d_full_partials, c->d_out, 0, 0, c->full_split, c->stream));
-    }
-    HIP_TRY(hipMemcpyAsync(out, c->d_out, sizeof(double) * R, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REMC_OK;
+    return energies_out(c, 0, out);
 }
 
 int remc_energy_all_noalloc(remc_ctx *c, double *out)
@@ -1329,14 +1376,7 @@ int remc_energy_noncrowder_all(remc_ctx *c, double *out)
     CHECK_CTX(c);
     FINALIZE(c);
     if (!out) return fail(REMC_ERR_ARG, "null output");
-    const int R = (int)c->reps.size();
-    {
-        TimedLaunch t(c, 1);
-        HIP_TRY(launch_energy_full(c->params(), R, c->max_tiles, c->d_full_partials, c->d_out, 1, 0, c->full_split, c->stream));
-    }
-    HIP_TRY(hipMemcpyAsync(out, c->d_out, sizeof(double) * R, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REMC_OK;
+    return energies_out(c, 1, out);
 }
 
 int remc_mc_steps(remc_ctx *c, int nsteps)
@@ -1601,9 +1641,12 @@ int remc_get_energies(remc_ctx *c, double *out)
     CHECK_CTX(c);
     FINALIZE(c);
     if (!out) return fail(REMC_ERR_ARG, "null output");
-    HIP_TRY(hipMemcpyAsync(out, c->d_E, sizeof(double) * c->reps.size(), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return check_err(c);
+    int err = 0;
+    ReadBack rb(c);
+    rb.add(out, c->d_E, 2 * c->reps.size());
+    rb.add(&err, c->d_err, 1);
+    const int rc = rb.run();
+    return rc != REMC_OK ? rc : report_err(c, err);
 }
 
 int remc_get_temperatures(remc_ctx *c, double *out)
@@ -1611,9 +1654,9 @@ int remc_get_temperatures(remc_ctx *c, double *out)
     CHECK_CTX(c);
     FINALIZE(c);
     if (!out) return fail(REMC_ERR_ARG, "null output");
-    HIP_TRY(hipMemcpyAsync(out, c->d_T, sizeof(double) * c->reps.size(), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REMC_OK;
+    ReadBack rb(c);
+    rb.add(out, c->d_T, 2 * c->reps.size());
+    return rb.run();
 }
 
 int remc_get_counters(remc_ctx *c, remc_counters *out)
@@ -1623,9 +1666,11 @@ int remc_get_counters(remc_ctx *c, remc_counters *out)
     if (!out) return fail(REMC_ERR_ARG, "null output");
     const int R = (int)c->reps.size();
     std::vector<unsigned long long> cnt(3 * R), st(R);
-    HIP_TRY(hipMemcpyAsync(cnt.data(), c->d_cnt, 24 * R, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(st.data(), c->d_step, 8 * R, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    ReadBack rb(c);
+    rb.add(cnt.data(), c->d_cnt, (size_t)6 * R);
+    rb.add(st.data(), c->d_step, (size_t)2 * R);
+    const int rc = rb.run();
+    if (rc != REMC_OK) return rc;
     for (int r = 0; r < R; ++r) {
         out[r].accept = cnt[3 * r];
         out[r].accept_boltz = cnt[3 * r + 1];
@@ -1642,10 +1687,9 @@ int remc_get_ladder(remc_ctx *c, int sys_id, int *slot_replica)
     if (sys_id < 0 || sys_id >= (int)c->systems.size() || !slot_replica) return fail(REMC_ERR_ARG, "bad ladder request");
     int off = 0;
     for (int i = 0; i < sys_id; ++i) off += (int)c->systems[i].replicas.size();
-    HIP_TRY(hipMemcpyAsync(slot_replica, c->d_slot + off, sizeof(int) * c->systems[sys_id].replicas.size(),
-                           hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REMC_OK;
+    ReadBack rb(c);
+    rb.add(slot_replica, c->d_slot + off, c->systems[sys_id].replicas.size());
+    return rb.run();
 }
 
 int remc_get_state(remc_ctx *c, int replica, float *x, float *y, float *z, float *rx, float *ry, float *rz,
@@ -1657,18 +1701,15 @@ int remc_get_state(remc_ctx *c, int replica, float *x, float *y, float *z, float
     const HostSys &s = c->systems[c->reps[replica].sys];
     const size_t nb = s.n_beads, nm = s.n_bodies;
     const int bo = c->rep_bead_off[replica], mo = c->rep_body_off[replica];
-    hipStream_t st = c->stream;
     float *dst_b[6] = {x, y, z, rx, ry, rz};
     float *src_b[6] = {c->d_px, c->d_py, c->d_pz, c->d_rx, c->d_ry, c->d_rz};
-    for (int i = 0; i < 6; ++i)
-        if (dst_b[i]) HIP_TRY(hipMemcpyAsync(dst_b[i], src_b[i] + bo, 4 * nb, hipMemcpyDeviceToHost, st));
     float *dst_m[3] = {cx, cy, cz};
     float *src_m[3] = {c->d_cx, c->d_cy, c->d_cz};
-    for (int i = 0; i < 3; ++i)
-        if (dst_m[i]) HIP_TRY(hipMemcpyAsync(dst_m[i], src_m[i] + mo, 4 * nm, hipMemcpyDeviceToHost, st));
-    if (quat) HIP_TRY(hipMemcpyAsync(quat, c->d_quat + 4 * (size_t)mo, 32 * nm, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    return REMC_OK;
+    ReadBack rb(c);
+    for (int i = 0; i < 6; ++i) rb.add(dst_b[i], src_b[i] + bo, nb);
+    for (int i = 0; i < 3; ++i) rb.add(dst_m[i], src_m[i] + mo, nm);
+    rb.add(quat, c->d_quat + 4 * (size_t)mo, 8 * nm);
+    return rb.run();
 }
 
 int remc_set_state(remc_ctx *c, int replica, const float *x, const float *y, const float *z, const float *rx,
@@ -1780,10 +1821,12 @@ int remc_get_exchange_state(remc_ctx *c, int sys_id, uint64_t *round, int *offse
     if (sys_id < 0 || sys_id >= (int)c->systems.size()) return fail(REMC_ERR_ARG, "bad system %d", sys_id);
     unsigned long long rd = 0, sw = 0;
     int of = 0;
-    HIP_TRY(hipMemcpyAsync(&rd, c->d_exround + sys_id, 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(&of, c->d_exoff + sys_id, 4, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(&sw, c->d_exswaps + sys_id, 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    ReadBack rb(c);
+    rb.add(&rd, c->d_exround + sys_id, 2);
+    rb.add(&of, c->d_exoff + sys_id, 1);
+    rb.add(&sw, c->d_exswaps + sys_id, 2);
+    const int rc = rb.run();
+    if (rc != REMC_OK) return rc;
     if (round) *round = rd;
     if (offset) *offset = of;
     if (swaps) *swaps = sw;

@@ -138,6 +138,16 @@ hipError_t launch_centre_hist(const KParams &p, int sys_id, int n_bodies, int n_
                               int n_types, int nbin, double lo, double dr, unsigned long long *counts, hipStream_t s);
 hipError_t launch_gr_normalise(const unsigned long long *counts, const int *type_count, int n_types, int nbin, double lo,
                                double dr, double frames_over_volume, double *gr, hipStream_t s);
+// Up to GATHER_MAX device arrays read back by one launch: array k's words go to
+// dst[at[k]] .. dst[at[k + 1]) (32-bit words, packed without gaps), dst being
+// pinned host memory.
+constexpr int GATHER_MAX = 10;
+struct Gather {
+    const uint32_t *src[GATHER_MAX];
+    uint32_t at[GATHER_MAX + 1];
+    int n;
+};
+hipError_t launch_gather(const Gather &g, uint32_t *dst, hipStream_t s);
 size_t adjoint_ff_size();
 void adjoint_ff_fill(void *dst, const float *table, double lambda, double e0, double xi, double c_lj, double c_dh);
 

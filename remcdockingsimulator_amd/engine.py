@@ -234,12 +234,14 @@ class Engine:
     def state(self, replica):
         sa = self.systems[self.replica_sys[replica]]
         n, m = sa.n_beads, sa.n_bodies
-        b = [np.zeros(n, dtype=np.float32) for _ in range(6)]
-        c = [np.zeros(m, dtype=np.float32) for _ in range(3)]
-        q = np.zeros((m, 4), dtype=np.float64)
-        self._chk(self.lib.remc_get_state(self.ctx, replica, *[nat.fptr(a) for a in b + c], nat.dptr(q)),
-                  "remc_get_state")
-        return dict(pos=np.stack(b[:3], 1), rel=np.stack(b[3:], 1), center=np.stack(c, 1), quat=q)
+        b = np.empty((6, n), dtype=np.float32)
+        c = np.empty((3, m), dtype=np.float32)
+        q = np.empty((m, 4), dtype=np.float64)
+        pb, pc = b.ctypes.data, c.ctypes.data
+        self._chk(self.lib.remc_get_state(self.ctx, replica, *[pb + 4 * n * k for k in range(6)],
+                                          *[pc + 4 * m * k for k in range(3)], q.ctypes.data), "remc_get_state")
+        return dict(pos=np.ascontiguousarray(b[:3].T), rel=np.ascontiguousarray(b[3:].T),
+                    center=np.ascontiguousarray(c.T), quat=q)
 
     def set_state(self, replica, pos=None, rel=None, center=None, quat=None):
         def cols(a, k):
