@@ -351,6 +351,20 @@ int autotune_energy(remc_ctx *c)
     return REMC_OK;
 }
 
+// Grows the pinned memory to at least `bytes`.  Every call that uses it waits
+// for the device before it returns, so nothing in flight refers to it here.
+int pin_reserve(remc_ctx *c, size_t bytes)
+{
+    const size_t words = (bytes + 3) / 4;
+    if (words <= c->pin_words) return REMC_OK;
+    if (c->h_pin) HIP_TRY(hipHostFree(c->h_pin));
+    c->h_pin = nullptr;
+    c->pin_words = 0;
+    HIP_TRY(hipHostMalloc((void **)&c->h_pin, 4 * words, hipHostMallocDefault));
+    c->pin_words = words;
+    return REMC_OK;
+}
+
 int finalize(remc_ctx *c)
 {
     if (c->finalized) return REMC_OK;
@@ -603,8 +617,9 @@ int finalize(remc_ctx *c)
         c->max_body_beads = std::max(c->max_body_beads, sy.max_body);
     }
     // the largest read-back: one replica's state, or the counters of all (and the error flag)
-    c->pin_words = std::max((size_t)6 * c->max_beads + (size_t)11 * c->max_bodies, (size_t)8 * R) + 8;
-    HIP_TRY(hipHostMalloc((void **)&c->h_pin, 4 * c->pin_words, hipHostMallocDefault));
+    const int prc = pin_reserve(
+        c, 4 * (std::max((size_t)6 * c->max_beads + (size_t)11 * c->max_bodies, (size_t)8 * R) + 8));
+    if (prc != REMC_OK) return prc;
     HIP_TRY(hipStreamSynchronize(s));
     c->synced_copies = 1;
     c->finalized = true;
@@ -1879,18 +1894,59 @@ int remc_drms(remc_ctx *c, int sys_id, const float *ref_x, const float *ref_y, c
         beads_before += nm;
     }
     if (pairs <= 0.0) return fail(REMC_ERR_ARG, "system %d has fewer than two non-crowder bodies", sys_id);
-    const int tiles = (N + 255) / 256;
+    // scratch: the reference, then the partials; the reference goes up in one
+    // copy from pinned memory, the results come back into it
     const size_t fbytes = ((3 * (size_t)N * sizeof(float) + 255) / 256) * 256;
-    int rc = ana_reserve(c, fbytes + sizeof(double) * ((size_t)R * tiles + R));
+    const size_t units = drms_units(N, R);
+    int rc = ana_reserve(c, fbytes + sizeof(double) * (size_t)R * units);
+    if (rc == REMC_OK) rc = pin_reserve(c, fbytes + sizeof(double) * R);
     if (rc != REMC_OK) return rc;
-    float *rx = (float *)c->d_ana, *ry = rx + N, *rz = ry + N;
-    double *part = (double *)((char *)c->d_ana + fbytes), *dout = part + (size_t)R * tiles;
-    HIP_TRY(hipMemcpyAsync(rx, ref_x, sizeof(float) * N, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemcpyAsync(ry, ref_y, sizeof(float) * N, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemcpyAsync(rz, ref_z, sizeof(float) * N, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(launch_drms(c->params(), sys_id, N, R, rx, ry, rz, part, 1.0 / pairs, dout, c->stream));
-    HIP_TRY(hipMemcpyAsync(out, dout, sizeof(double) * R, hipMemcpyDeviceToHost, c->stream));
+    float *rx = (float *)c->d_ana, *ry = rx + N, *rz = ry + N, *hx = (float *)c->h_pin;
+    double *part = (double *)((char *)c->d_ana + fbytes), *hout = (double *)((char *)c->h_pin + fbytes);
+    std::memcpy(hx, ref_x, sizeof(float) * N);
+    std::memcpy(hx + N, ref_y, sizeof(float) * N);
+    std::memcpy(hx + 2 * (size_t)N, ref_z, sizeof(float) * N);
+    HIP_TRY(hipMemcpyAsync(rx, hx, 3 * sizeof(float) * N, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(launch_drms(c->params(), sys_id, N, R, rx, ry, rz, part, 1.0 / pairs, hout, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
+    std::memcpy(out, hout, sizeof(double) * R);
+    return REMC_OK;
+}
+
+// The histogram kernels of a system: body types, sites (may be null) and the
+// bodies per type (type_count) go up in one copy from pinned memory, the nh
+// counts or values of g(r) come back into it.
+static int centre_hist(remc_ctx *c, int sys_id, const int *body_type, const int *site_bead, const int *type_count,
+                       int n_types, int nbin, double lo, double hi, double frames_over_volume, uint64_t *counts, double *gr)
+{
+    const HostSys &s = c->systems[sys_id];
+    const int M = s.n_bodies, R = (int)s.replicas.size();
+    const size_t nh = (size_t)n_types * n_types * nbin;
+    const size_t ints = (site_bead ? 2 : 1) * (size_t)M + (type_count ? n_types : 0);
+    const size_t ib = (ints * sizeof(int) + 255) / 256 * 256;
+    int rc = ana_reserve(c, ib + sizeof(unsigned int) * nh * (size_t)hist_workgroups(M, R, (int)nh));
+    if (rc == REMC_OK) rc = pin_reserve(c, ib + 8 * nh);
+    if (rc != REMC_OK) return rc;
+    int *h = (int *)c->h_pin, *d = (int *)c->d_ana;
+    std::memcpy(h, body_type, sizeof(int) * M);
+    size_t at = M;
+    const int *dsite = nullptr, *dcount = nullptr;
+    if (site_bead) {
+        std::memcpy(h + at, site_bead, sizeof(int) * M);
+        dsite = d + at;
+        at += M;
+    }
+    if (type_count) {
+        std::memcpy(h + at, type_count, sizeof(int) * n_types);
+        dcount = d + at;
+    }
+    HIP_TRY(hipMemcpyAsync(d, h, sizeof(int) * ints, hipMemcpyHostToDevice, c->stream));
+    char *hout = (char *)c->h_pin + ib;
+    HIP_TRY(launch_centre_hist(c->params(), sys_id, M, R, d, dsite, n_types, nbin, lo, (hi - lo) / nbin,
+                               (unsigned int *)((char *)c->d_ana + ib), dcount, frames_over_volume,
+                               (unsigned long long *)hout, gr ? (double *)hout : nullptr, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    std::memcpy(gr ? (void *)gr : (void *)counts, hout, 8 * nh);
     return REMC_OK;
 }
 
@@ -1907,21 +1963,9 @@ int remc_centre_histogram(remc_ctx *c, int sys_id, const int *body_type, int n_t
     if (nh * sizeof(unsigned int) > 48 * 1024)
         return fail(REMC_ERR_LIMIT, "histogram of %zu bins exceeds the 12288-bin workgroup limit", nh);
     const HostSys &s = c->systems[sys_id];
-    const int M = s.n_bodies, R = (int)s.replicas.size();
-    for (int m = 0; m < M; ++m)
+    for (int m = 0; m < s.n_bodies; ++m)
         if (body_type[m] < -1 || body_type[m] >= n_types) return fail(REMC_ERR_ARG, "body %d has type %d", m, body_type[m]);
-    const size_t tbytes = ((sizeof(int) * (size_t)M + 255) / 256) * 256;
-    int rc = ana_reserve(c, tbytes + sizeof(unsigned long long) * nh);
-    if (rc != REMC_OK) return rc;
-    int *dtype = (int *)c->d_ana;
-    unsigned long long *dcounts = (unsigned long long *)((char *)c->d_ana + tbytes);
-    HIP_TRY(hipMemcpyAsync(dtype, body_type, sizeof(int) * M, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemsetAsync(dcounts, 0, sizeof(unsigned long long) * nh, c->stream));
-    HIP_TRY(launch_centre_hist(c->params(), sys_id, M, R, dtype, nullptr, n_types, nbin, lo, (hi - lo) / nbin, dcounts,
-                               c->stream));
-    HIP_TRY(hipMemcpyAsync(counts, dcounts, sizeof(unsigned long long) * nh, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REMC_OK;
+    return centre_hist(c, sys_id, body_type, nullptr, nullptr, n_types, nbin, lo, hi, 0.0, counts, nullptr);
 }
 
 int remc_radial_distribution(remc_ctx *c, int sys_id, const int *body_type, const int *site_bead, int n_types,
@@ -1947,26 +1991,9 @@ int remc_radial_distribution(remc_ctx *c, int sys_id, const int *body_type, cons
             (site_bead[m] < s.body_start[m] || site_bead[m] >= s.body_start[m + 1]))
             return fail(REMC_ERR_ARG, "site bead %d is not a bead of body %d", site_bead[m], m);
     }
-    auto up = [](size_t b) { return ((b + 255) / 256) * 256; };
-    const size_t tb = up(sizeof(int) * (size_t)M), sb = up(sizeof(int) * (size_t)M), cb = up(sizeof(int) * n_types);
-    const size_t hb = up(sizeof(unsigned long long) * nh);
-    int rc = ana_reserve(c, tb + sb + cb + hb + sizeof(double) * nh);
-    if (rc != REMC_OK) return rc;
-    char *base = (char *)c->d_ana;
-    int *dtype = (int *)base, *dsite = (int *)(base + tb), *dcount = (int *)(base + tb + sb);
-    unsigned long long *dhist = (unsigned long long *)(base + tb + sb + cb);
-    double *dgr = (double *)(base + tb + sb + cb + hb);
-    HIP_TRY(hipMemcpyAsync(dtype, body_type, sizeof(int) * M, hipMemcpyHostToDevice, c->stream));
-    if (site_bead) HIP_TRY(hipMemcpyAsync(dsite, site_bead, sizeof(int) * M, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemcpyAsync(dcount, type_count.data(), sizeof(int) * n_types, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemsetAsync(dhist, 0, sizeof(unsigned long long) * nh, c->stream));
-    const double dr = (hi - lo) / nbin, L = (double)s.box;
-    HIP_TRY(launch_centre_hist(c->params(), sys_id, M, R, dtype, site_bead ? dsite : nullptr, n_types, nbin, lo, dr,
-                               dhist, c->stream));
-    HIP_TRY(launch_gr_normalise(dhist, dcount, n_types, nbin, lo, dr, (double)R / (L * L * L), dgr, c->stream));
-    HIP_TRY(hipMemcpyAsync(gr, dgr, sizeof(double) * nh, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return REMC_OK;
+    const double L = (double)s.box;
+    return centre_hist(c, sys_id, body_type, site_bead, type_count.data(), n_types, nbin, lo, hi, (double)R / (L * L * L),
+                       nullptr, gr);
 }
 
 int remc_adjoint(remc_ctx *c, int replica, double *force_torque, double *dparams)

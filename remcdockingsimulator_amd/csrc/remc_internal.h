@@ -134,10 +134,13 @@ hipError_t launch_adjoint(const KParams &p, const void *adj_ff, const AdjPlan &a
                           double *force_torque, double *dparams, hipStream_t s);
 hipError_t launch_drms(const KParams &p, int sys_id, int n_beads, int n_rep, const float *rx, const float *ry,
                        const float *rz, double *partials, double inv_pairs, double *out, hipStream_t s);
+size_t drms_units(int n_beads, int n_rep); // partials of launch_drms per replica
+// part: hist_workgroups(...) x nh 32-bit counts; the result goes to gr when it
+// is given, else to counts
+int hist_workgroups(int n_bodies, int n_rep, int nh);
 hipError_t launch_centre_hist(const KParams &p, int sys_id, int n_bodies, int n_rep, const int *btype, const int *site,
-                              int n_types, int nbin, double lo, double dr, unsigned long long *counts, hipStream_t s);
-hipError_t launch_gr_normalise(const unsigned long long *counts, const int *type_count, int n_types, int nbin, double lo,
-                               double dr, double frames_over_volume, double *gr, hipStream_t s);
+                              int n_types, int nbin, double lo, double dr, unsigned int *part, const int *type_count,
+                              double frames_over_volume, unsigned long long *counts, double *gr, hipStream_t s);
 // Up to GATHER_MAX device arrays read back by one launch: array k's words go to
 // dst[at[k]] .. dst[at[k + 1]) (32-bit words, packed without gaps), dst being
 // pinned host memory.
