@@ -17,7 +17,7 @@ LIB = os.path.join(HERE, "libremc.so")
 SIM = os.path.join(HERE, "remc_sim")
 PDBGEN = os.path.join(HERE, "remc_pdbgen")
 
-SOURCES = ["remc_kernels.hip", "remc_analysis.hip", "remc_api.hip"]
+SOURCES = ["remc_kernels.hip", "remc_full.hip", "remc_analysis.hip", "remc_api.hip"]
 FACADE_SOURCES = ["host/remc_facade.cpp"]
 
 HIPCC_FLAGS = [

@@ -124,7 +124,7 @@ struct remc_ctx {
     // sizes
     int total_static_beads = 0, total_static_bodies = 0;
     int total_rep_beads = 0, total_rep_bodies = 0, total_slots = 0;
-    int max_beads = 0, max_tiles = 0;
+    int max_beads = 0;
     std::vector<int> rep_bead_off, rep_body_off;
 
     // device buffers
@@ -140,7 +140,10 @@ struct remc_ctx {
     int *d_slot = nullptr, *d_exoff = nullptr;
     double *d_ladder = nullptr;
     unsigned long long *d_exround = nullptr, *d_exswaps = nullptr;
-    double *d_full_partials = nullptr, *d_out = nullptr;
+    double *d_full_partials = nullptr;
+    int *d_border = nullptr;
+    int *d_grp = nullptr; // static summaries of the groups of 16 beads
+    int *d_fix = nullptr; // what k_fix makes of the conformations (scratch of the full-energy and adjoint kernels)
     float *d_plain_partials = nullptr;
     size_t plain_partials_cap = 0;
     remc_step_record *d_rec = nullptr;
@@ -157,7 +160,6 @@ struct remc_ctx {
     size_t ana_bytes = 0;
     DevFF devff{};
     double *noalloc_scratch = nullptr; // this device's `scratch` (remc_energy_all_noalloc)
-    int full_split = 0;      // full-energy partner sub-ranges per unit (0: the size rule; set at set-up)
     int fb_block = 0;        // force-biased kernel's workgroup size (0 = autotune on first use)
     bool run_refresh = false; // remc_run: energy refresh between the MC launch and the exchange
 
@@ -172,6 +174,7 @@ struct remc_ctx {
     bool mc_window = true;   // speculative windows of small moves allowed
     long long min_move_pairs = -1;
     int max_bodies = 0, max_body_beads = 0;
+    int max_body_waves = 0; // waves of k_adjoint_bodies for one replica
 
     // graph
     hipGraphExec_t graph = nullptr;
@@ -192,7 +195,7 @@ struct remc_ctx {
     {
         KParams p{};
         p.tc = d_tc; p.q = d_q; p.sig = d_sig; p.body = d_body;
-        p.bstart = d_bstart; p.bend = d_bend; p.bcrow = d_bcrow;
+        p.bstart = d_bstart; p.bend = d_bend; p.bcrow = d_bcrow; p.grp = d_grp; p.border = d_border;
         p.sys = d_sys; p.rep = d_rep; p.etab = d_etab; p.ff = devff;
         p.sstab = d_sstab; p.sigtab = sigtab;
         p.px = d_px; p.py = d_py; p.pz = d_pz; p.rx = d_rx; p.ry = d_ry; p.rz = d_rz;
@@ -294,62 +297,10 @@ struct EventPair {
     }
 };
 
-// Partner split of the full-energy kernels for each (replicas, bead tiles):
-// timed once per process and grid size, so every context of a process with
-// that size takes the same split and their energies agree bit for bit.
 std::mutex g_split_mu;
-std::map<std::pair<int, int>, int> g_split_cache;
 
-int autotune_energy(remc_ctx *c)
-{
-    const int R = (int)c->reps.size();
-    const std::pair<int, int> key(R, c->max_tiles);
-    {
-        std::lock_guard<std::mutex> lock(g_split_mu);
-        auto it = g_split_cache.find(key);
-        if (it != g_split_cache.end()) {
-            c->full_split = it->second;
-            return REMC_OK;
-        }
-    }
-    // each candidate on the live conformations (energies only, nothing
-    // written back), best of three; the size rule's choice is kept unless
-    // another split is at least 3% faster
-    const int def = full_split_default(R, c->max_tiles);
-    const int cand[3] = {1, 2, FULL_SPLIT_MAX};
-    float best_ms[3] = {0.f, 0.f, 0.f};
-    EventPair ev;
-    HIP_TRY(ev.create());
-    const KParams p = c->params();
-    for (int k = 0; k < 3; ++k) {
-        HIP_TRY(launch_energy_full(p, R, c->max_tiles, c->d_full_partials, c->d_out, 0, 0, cand[k], c->stream));
-        float best = 1e30f;
-        for (int rep = 0; rep < 3; ++rep) {
-            HIP_TRY(hipEventRecord(ev.a, c->stream));
-            HIP_TRY(launch_energy_full(p, R, c->max_tiles, c->d_full_partials, c->d_out, 0, 0, cand[k], c->stream));
-            HIP_TRY(hipEventRecord(ev.b, c->stream));
-            HIP_TRY(hipEventSynchronize(ev.b));
-            float ms = 0.f;
-            HIP_TRY(hipEventElapsedTime(&ms, ev.a, ev.b));
-            best = std::min(best, ms);
-        }
-        best_ms[k] = best;
-    }
-    float t_def = 1e30f;
-    for (int k = 0; k < 3; ++k)
-        if (cand[k] == def) t_def = best_ms[k];
-    int pick = def;
-    float t_pick = t_def;
-    for (int k = 0; k < 3; ++k)
-        if (best_ms[k] < 0.97f * t_def && best_ms[k] < t_pick) {
-            pick = cand[k];
-            t_pick = best_ms[k];
-        }
-    std::lock_guard<std::mutex> lock(g_split_mu);
-    auto ins = g_split_cache.emplace(key, pick); // a context set up meanwhile keeps its choice
-    c->full_split = ins.first->second;
-    return REMC_OK;
-}
+// 32-bit words of an adjoint of all replicas that comes back in pinned memory, at most
+constexpr size_t PIN_ADJ_WORDS = 1 << 18;
 
 // Grows the pinned memory to at least `bytes`.  Every call that uses it waits
 // for the device before it returns, so nothing in flight refers to it here.
@@ -374,7 +325,7 @@ int finalize(remc_ctx *c)
     HIP_TRY(hipSetDevice(c->device));
 
     // static layout
-    std::vector<int> tc, body, bstart, bend, bcrow;
+    std::vector<int> tc, body, bstart, bend, bcrow, grp, border;
     std::vector<float> q, sig;
     std::vector<DevSys> dsys;
     int bead_off = 0, body_off = 0, slot_off = 0;
@@ -388,6 +339,7 @@ int finalize(remc_ctx *c)
         d.rep_first = s.replicas.empty() ? 0 : s.replicas.front();
         d.n_rep = (int)s.replicas.size();
         d.slot_off = slot_off;
+        d.grp_off = (int)(grp.size() / 4);
         d.box = s.box > 0.f ? s.box : 0.f;
         d.inv_box = s.box > 0.f ? 1.0f / s.box : 0.f;
         dsys.push_back(d);
@@ -402,6 +354,23 @@ int finalize(remc_ctx *c)
                 sig.push_back(s.sigma[b]);
             }
         }
+        for (int g = 0; g < full_groups(s.n_beads); ++g) {
+            const int b0 = g * GROUP, b1 = std::min(b0 + GROUP, s.n_beads);
+            int kinds = 0, charged = 0;
+            for (int b = b0; b < b1; ++b) {
+                kinds |= (tc[bead_off + b] >> 8) ? GROUP_CROWDER : GROUP_CHAIN;
+                if (s.charge[b] != 0.f) charged |= 1 << (b - b0);
+            }
+            grp.insert(grp.end(), {body[bead_off + b0], body[bead_off + b1 - 1], kinds | (b1 - b0) << 8, charged});
+        }
+        for (int several = 1; several >= 0; --several)
+            for (int m = 0; m < s.n_bodies; ++m)
+                if ((s.body_start[m + 1] - s.body_start[m] > 1) == (several != 0)) {
+                    border.push_back(m);
+                    dsys.back().n_multi += several;
+                }
+        const int n_multi = dsys.back().n_multi;
+        c->max_body_waves = std::max(c->max_body_waves, n_multi + (s.n_bodies - n_multi + 63) / 64);
         bead_off += s.n_beads;
         body_off += s.n_bodies;
         slot_off += (int)s.replicas.size();
@@ -418,7 +387,7 @@ int finalize(remc_ctx *c)
     c->rep_body_off.assign(R, 0);
     std::vector<float> px, py, pz, rx, ry, rz, cx, cy, cz;
     std::vector<double> quat, E(R, 0.0), T(R);
-    int rbo = 0, rmo = 0;
+    int rbo = 0, rmo = 0, rgo = 0;
     for (int r = 0; r < R; ++r) {
         const HostRep &h = c->reps[r];
         const HostSys &s = c->systems[h.sys];
@@ -426,6 +395,7 @@ int finalize(remc_ctx *c)
         d.sys = h.sys;
         d.bead_off = rbo;
         d.body_off = rmo;
+        d.grp_off = rgo;
         d.rng_id = (uint32_t)r;
         d.tstep = h.tstep;
         d.rot_ch = std::cos(h.rstep / 2.0);
@@ -447,6 +417,7 @@ int finalize(remc_ctx *c)
         T[r] = h.T;
         rbo += s.n_beads;
         rmo += s.n_bodies;
+        rgo += full_groups(s.n_beads);
     }
     c->total_rep_beads = rbo;
     c->total_rep_bodies = rmo;
@@ -475,13 +446,11 @@ int finalize(remc_ctx *c)
         c->devff.crow_k = (float)(lj_scale * s2 * s2 * s2);
     }
 
-    c->max_tiles = (c->max_beads + FULL_TILE - 1) / FULL_TILE;
-
     // When every non-crowder bead's sigma is its residue type's (as the
-    // reference's amino-acid table makes it), the MC kernel reads each type
-    // pair's (0.5 (sigma_i + sigma_j))^2 / box^2 from a table per system: the
-    // FP32 operations the kernel would form from the two sigmas, in the same
-    // order, so the numbers are the same.
+    // reference's amino-acid table makes it), the kernels read each type pair's
+    // (0.5 (sigma_i + sigma_j))^2 from tables per system (over box^2 for the MC
+    // kernel, then as it is): the FP32 operations the kernels would form from
+    // the two sigmas, in the same order, so the numbers are the same.
     {
         std::vector<float> sstab;
         bool by_type = true;
@@ -504,15 +473,16 @@ int finalize(remc_ctx *c)
             if (!by_type) break;
             const float ib = hs.box > 0.f ? 1.0f / hs.box : 0.f;
             const float ib2 = ib * ib;
-            for (int i = 0; i < REMC_NTYPES; ++i)
-                for (int j = 0; j < REMC_NTYPES; ++j) {
-                    float v = 0.f;
-                    if (seen[i] && seen[j]) {
-                        const float h = 0.5f * st[i] + 0.5f * st[j];
-                        v = (h * h) * ib2;
+            for (int scaled = 1; scaled >= 0; --scaled)
+                for (int i = 0; i < REMC_NTYPES; ++i)
+                    for (int j = 0; j < REMC_NTYPES; ++j) {
+                        float v = 0.f;
+                        if (seen[i] && seen[j]) {
+                            const float h = 0.5f * st[i] + 0.5f * st[j];
+                            v = scaled ? (h * h) * ib2 : h * h;
+                        }
+                        sstab.push_back(v);
                     }
-                    sstab.push_back(v);
-                }
         }
         c->sigtab = by_type ? 1 : 0;
         if (by_type) {
@@ -554,8 +524,10 @@ int finalize(remc_ctx *c)
     HIP_TRY(dalloc(&c->d_exround, c->systems.size()));
     HIP_TRY(dalloc(&c->d_exoff, c->systems.size()));
     HIP_TRY(dalloc(&c->d_exswaps, c->systems.size()));
-    HIP_TRY(dalloc(&c->d_full_partials, (size_t)R * full_units(c->max_tiles) * FULL_SPLIT_MAX));
-    HIP_TRY(dalloc(&c->d_out, (size_t)R));
+    HIP_TRY(dalloc(&c->d_full_partials, (size_t)R * full_units(R, c->max_beads)));
+    HIP_TRY(dalloc(&c->d_grp, grp.size()));
+    HIP_TRY(dalloc(&c->d_border, border.size()));
+    HIP_TRY(dalloc(&c->d_fix, fix_ints(px.size(), (size_t)rgo)));
     HIP_TRY(dalloc(&c->d_rec_start, (size_t)R));
 
     HIP_TRY(upload(c->d_tc, tc, s));
@@ -565,6 +537,8 @@ int finalize(remc_ctx *c)
     HIP_TRY(upload(c->d_bstart, bstart, s));
     HIP_TRY(upload(c->d_bend, bend, s));
     HIP_TRY(upload(c->d_bcrow, bcrow, s));
+    HIP_TRY(upload(c->d_grp, grp, s));
+    HIP_TRY(upload(c->d_border, border, s));
     HIP_TRY(upload(c->d_sys, dsys, s));
     HIP_TRY(upload(c->d_rep, drep, s));
     HIP_TRY(upload(c->d_etab, etab, s));
@@ -616,9 +590,11 @@ int finalize(remc_ctx *c)
         c->max_bodies = std::max(c->max_bodies, sy.n_bodies);
         c->max_body_beads = std::max(c->max_body_beads, sy.max_body);
     }
-    // the largest read-back: one replica's state, or the counters of all (and the error flag)
-    const int prc = pin_reserve(
-        c, 4 * (std::max((size_t)6 * c->max_beads + (size_t)11 * c->max_bodies, (size_t)8 * R) + 8));
+    // the largest read-back: one replica's state, the counters of all (and the
+    // error flag), or the adjoint of all
+    const size_t adj_words = 2 * (6 * (size_t)c->total_rep_bodies + 3 * (size_t)R);
+    const int prc = pin_reserve(c, 4 * (std::max({(size_t)6 * c->max_beads + (size_t)11 * c->max_bodies, (size_t)8 * R,
+                                                  adj_words <= PIN_ADJ_WORDS ? adj_words : 0}) + 8));
     if (prc != REMC_OK) return prc;
     HIP_TRY(hipStreamSynchronize(s));
     c->synced_copies = 1;
@@ -626,10 +602,10 @@ int finalize(remc_ctx *c)
 
     // initial energies of every replica
     KParams p = c->params();
-    HIP_TRY(launch_energy_full(p, R, c->max_tiles, c->d_full_partials, nullptr, 0, 1, 0, s));
+    HIP_TRY(launch_energy_full(p, R, c->max_beads, c->d_fix, c->d_full_partials, nullptr, 0, 1, s));
     HIP_TRY(hipStreamSynchronize(s));
     c->adj_target = 0; // the all-replica adjoint is tuned on its first call
-    return autotune_energy(c);
+    return REMC_OK;
 }
 
 #define CHECK_CTX(c)                                                   \
@@ -720,8 +696,8 @@ int energies_out(remc_ctx *c, int noncrowder_only, double *out)
     const int R = (int)c->reps.size();
     {
         TimedLaunch t(c, 1);
-        HIP_TRY(launch_energy_full(c->params(), R, c->max_tiles, c->d_full_partials, (double *)c->h_pin, noncrowder_only,
-                                   0, c->full_split, c->stream));
+        HIP_TRY(launch_energy_full(c->params(), R, c->max_beads, c->d_fix, c->d_full_partials, (double *)c->h_pin, noncrowder_only,
+                                   0, c->stream));
     }
     HIP_TRY(hipStreamSynchronize(c->stream));
     std::memcpy(out, c->h_pin, sizeof(double) * R);
@@ -1089,10 +1065,10 @@ int autotune_adjoint(remc_ctx *c)
         int rc = adjoint_scratch(c, a, R, c->total_rep_bodies);
         if (rc != REMC_OK) return rc;
         double *ft = c->d_adj + a.part_doubles + a.param_doubles, *dp = ft + 6 * (size_t)c->total_rep_bodies;
-        HIP_TRY(launch_adjoint(p, af.data(), a, 0, R, c->max_bodies, 0, stride, 0, c->d_adj, ft, dp, c->stream));
+        HIP_TRY(launch_adjoint(p, af.data(), a, 0, R, c->max_beads, c->max_body_waves, 0, stride, 0, c->d_fix, c->d_adj, ft, dp, c->stream));
         for (int rep = 0; rep < 3; ++rep) {
             HIP_TRY(hipEventRecord(ev.a, c->stream));
-            HIP_TRY(launch_adjoint(p, af.data(), a, 0, R, c->max_bodies, 0, stride, 0, c->d_adj, ft, dp, c->stream));
+            HIP_TRY(launch_adjoint(p, af.data(), a, 0, R, c->max_beads, c->max_body_waves, 0, stride, 0, c->d_fix, c->d_adj, ft, dp, c->stream));
             HIP_TRY(hipEventRecord(ev.b, c->stream));
             HIP_TRY(hipEventSynchronize(ev.b));
             float ms = 0.f;
@@ -1113,7 +1089,7 @@ int autotune_adjoint(remc_ctx *c)
     return REMC_OK;
 }
 
-int adjoint_range(remc_ctx *c, int first, int n, int max_beads, int max_bodies, int bead_base, size_t bead_stride,
+int adjoint_range(remc_ctx *c, int first, int n, int max_beads, int bead_base, size_t bead_stride,
                   int body_base, int n_bodies_out, double *force_torque, double *dparams, int target_wg = 0)
 {
     const AdjPlan a = adjoint_plan(n, max_beads, bead_stride, target_wg);
@@ -1123,8 +1099,16 @@ int adjoint_range(remc_ctx *c, int first, int n, int max_beads, int max_bodies, 
     const std::vector<unsigned char> af = adjoint_ff(c);
     {
         TimedLaunch t(c, 4);
-        HIP_TRY(launch_adjoint(c->params(), af.data(), a, first, n, max_bodies, bead_base, bead_stride, body_base,
-                               c->d_adj, ft, dp, c->stream));
+        HIP_TRY(launch_adjoint(c->params(), af.data(), a, first, n, max_beads, c->max_body_waves, bead_base, bead_stride,
+                               body_base, c->d_fix, c->d_adj, ft, dp, c->stream));
+    }
+    // up to a megabyte comes back packed in pinned memory; more is copied into
+    // the caller's by the runtime, which overlaps its staging
+    if (2 * (6 * (size_t)c->total_rep_bodies + 3 * c->reps.size()) <= PIN_ADJ_WORDS) {
+        ReadBack rb(c);
+        rb.add(force_torque, ft, 12 * (size_t)n_bodies_out);
+        rb.add(dparams, dp, 6 * (size_t)n);
+        return rb.run();
     }
     if (force_torque)
         HIP_TRY(hipMemcpyAsync(force_torque, ft, sizeof(double) * 6 * n_bodies_out, hipMemcpyDeviceToHost, c->stream));
@@ -1176,7 +1160,7 @@ int remc_ctx_destroy(remc_ctx *c)
                     c->d_sys, c->d_rep, c->d_px, c->d_py, c->d_pz, c->d_rx, c->d_ry, c->d_rz,
                     c->d_cx, c->d_cy, c->d_cz, c->d_quat, c->d_E, c->d_T, c->d_step, c->d_cnt,
                     c->d_slot, c->d_exoff, c->d_ladder, c->d_exround, c->d_exswaps, c->d_full_partials,
-                    c->d_out, c->d_plain_partials, c->d_rec, c->d_rec_start, c->d_slots, c->d_err, c->d_adj,
+                    c->d_fix, c->d_grp, c->d_border, c->d_plain_partials, c->d_rec, c->d_rec_start, c->d_slots, c->d_err, c->d_adj,
                     c->d_ana};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -1361,13 +1345,16 @@ int remc_energy_all_noalloc(remc_ctx *c, double *out)
                                     "remc_energy_all, ...); remc_energy_all_noalloc allocates nothing");
     if (!c->noalloc_scratch) return fail(REMC_ERR_STATE, "no scratch address for device %d", c->device);
     const int R = (int)c->reps.size();
-    const size_t stride = (size_t)full_units(c->max_tiles) * FULL_SPLIT_MAX;
-    const size_t need = stride * (size_t)R + (size_t)R;
-    if (need > REMC_NOALLOC_DOUBLES)
+    // the documented need: four partials per unit of a 256-bead tile schedule
+    // (the launch's own units are fewer, checked below)
+    const size_t tiles = ((size_t)c->max_beads + 255) / 256, stride = 4 * tiles * (tiles / 2 + 1);
+    const size_t need = stride * (size_t)R + (size_t)R, own = (size_t)R * full_units(R, c->max_beads) + (size_t)R;
+    if (need > REMC_NOALLOC_DOUBLES || own > REMC_NOALLOC_DOUBLES)
         return fail(REMC_ERR_LIMIT, "remc_energy_all_noalloc needs %zu doubles of scratch for %d replicas of up to %d "
-                                    "beads; its static scratch holds %zu", need, R, c->max_beads, REMC_NOALLOC_DOUBLES);
-    double *partials = c->noalloc_scratch, *dout = partials + stride * (size_t)R;
-    HIP_TRY(launch_energy_full(c->params(), R, c->max_tiles, partials, dout, 0, 0, c->full_split, c->stream));
+                                    "beads; its static scratch holds %zu", std::max(need, own), R, c->max_beads,
+                    REMC_NOALLOC_DOUBLES);
+    double *partials = c->noalloc_scratch, *dout = partials + own - R;
+    HIP_TRY(launch_energy_full(c->params(), R, c->max_beads, c->d_fix, partials, dout, 0, 0, c->stream));
     HIP_TRY(hipMemcpyAsync(out, dout, sizeof(double) * R, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     return REMC_OK;
@@ -1380,7 +1367,7 @@ int remc_refresh_energies(remc_ctx *c)
     const int R = (int)c->reps.size();
     {
         TimedLaunch t(c, 1);
-        HIP_TRY(launch_energy_full(c->params(), R, c->max_tiles, c->d_full_partials, nullptr, 0, 1, c->full_split, c->stream));
+        HIP_TRY(launch_energy_full(c->params(), R, c->max_beads, c->d_fix, c->d_full_partials, nullptr, 0, 1, c->stream));
     }
     HIP_TRY(hipStreamSynchronize(c->stream));
     return REMC_OK;
@@ -1587,8 +1574,7 @@ int remc_run(remc_ctx *c, int rounds, int steps_per_round)
         hipError_t e1 = launch_mc(p, (int)c->reps.size(), steps_per_round, c->mc_block, c->mc_coop, c->stream);
         // with the refresh, the exchange reads full energies, as the reference's does
         if (e1 == hipSuccess && c->run_refresh)
-            e1 = launch_energy_full(p, (int)c->reps.size(), c->max_tiles, c->d_full_partials, nullptr, 0, 1,
-                                    c->full_split, c->stream);
+            e1 = launch_energy_full(p, (int)c->reps.size(), c->max_beads, c->d_fix, c->d_full_partials, nullptr, 0, 1, c->stream);
         hipError_t e2 = launch_exchange(p, (int)c->systems.size(), c->stream);
         hipError_t e3 = hipStreamEndCapture(c->stream, &g);
         if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
@@ -2003,7 +1989,7 @@ int remc_adjoint(remc_ctx *c, int replica, double *force_torque, double *dparams
     CHECK_REP(c, replica);
     if (!force_torque && !dparams) return fail(REMC_ERR_ARG, "null outputs");
     const HostSys &s = c->systems[c->reps[replica].sys];
-    return adjoint_range(c, replica, 1, s.n_beads, s.n_bodies, c->rep_bead_off[replica], (size_t)s.n_beads,
+    return adjoint_range(c, replica, 1, s.n_beads, c->rep_bead_off[replica], (size_t)s.n_beads,
                          c->rep_body_off[replica], s.n_bodies, force_torque, dparams);
 }
 
@@ -2016,7 +2002,7 @@ int remc_adjoint_all(remc_ctx *c, double *force_torque, double *dparams)
         const int rc = autotune_adjoint(c);
         if (rc != REMC_OK) return rc;
     }
-    return adjoint_range(c, 0, (int)c->reps.size(), c->max_beads, c->max_bodies, 0, (size_t)c->total_rep_beads, 0,
+    return adjoint_range(c, 0, (int)c->reps.size(), c->max_beads, 0, (size_t)c->total_rep_beads, 0,
                          c->total_rep_bodies, force_torque, dparams, c->adj_target);
 }
 

@@ -27,13 +27,15 @@ struct DevSys {
     int bead_off, n_beads, body_off, n_bodies;
     int max_body, rep_first, n_rep, slot_off;
     float box, inv_box;
-    int pad0, pad1;
+    int grp_off; // groups of 16 beads of the systems before it
+    int n_multi; // bodies of several beads
 };
 
 struct DevRep {
     int sys, bead_off, body_off;
     uint32_t rng_id;
-    float tstep, pad;
+    float tstep;
+    int grp_off; // groups of 16 beads of the replicas before it
     double rot_ch, rot_sh;
     double rstep; // rotate step (rad)
 };
@@ -59,10 +61,12 @@ struct KParams {
     const int *bstart;
     const int *bend;
     const int *bcrow;
+    const int *border; // the system's bodies (local), those of several beads first
+    const int *grp; // per group of 16 beads (sys.grp_off + g): first body, last body, kinds of beads | beads << 8, mask of charged beads
     const DevSys *sys;
     const DevRep *rep;
     const float *etab;
-    const float *sstab; // per system: (0.5 (sigma_i + sigma_j))^2 / box^2 of type pairs (when sigtab)
+    const float *sstab; // per system: (0.5 (sigma_i + sigma_j))^2 of type pairs, over box^2 and as it is (when sigtab)
     int sigtab;         // 1: every non-crowder bead's sigma is its type's
     DevFF ff;
     // dynamic
@@ -111,11 +115,18 @@ hipError_t launch_mc_fb(const KParams &p, int n_rep, int nsteps, int block, int 
 hipError_t mc_fb_max_active_per_cu(const KParams &p, int block, int *out);
 size_t mc_fb_dynamic_lds(const KParams &p);
 hipError_t mc_max_active_per_cu(const KParams &p, int block, int *out);
-// split: partner sub-ranges per full-energy unit (1, 2 or FULL_SPLIT_MAX;
-// anything else takes full_split_default, a rule on the grid's size)
-hipError_t launch_energy_full(const KParams &p, int n_rep, int max_tiles, double *partials, double *out,
-                              int noncrowder_only, int write_E, int split, hipStream_t s);
-int full_split_default(int n_rep, int max_tiles);
+// full energies of n_rep replicas of at most max_beads beads: fix holds
+// fix_ints(...) ints (scratch), partials n_rep x full_units(...) doubles
+hipError_t launch_energy_full(const KParams &p, int n_rep, int max_beads, int *fix, double *partials, double *out,
+                              int noncrowder_only, int write_E, hipStream_t s);
+int full_units(int n_rep, int max_beads);
+constexpr int GROUP = 16;                          // beads of a column group of the all-pairs kernels
+constexpr int GROUP_CHAIN = 1, GROUP_CROWDER = 2; // kinds of beads present (KParams::grp)
+__host__ __device__ inline int full_groups(int beads) { return (beads + GROUP - 1) / GROUP; }
+// k_fix's output: coordinates as fractions of the box of all replicas, then
+// (16-byte aligned) the groups' ranges
+__host__ __device__ inline size_t fix_centres(size_t beads) { return (3 * beads + 3) / 4 * 4; }
+inline size_t fix_ints(size_t beads, size_t groups) { return fix_centres(beads) + 4 * groups; }
 hipError_t launch_energy_plain(const KParams &p, int replica, int n_beads, int block, float *partials, hipStream_t s);
 hipError_t launch_exchange(const KParams &p, int n_sys, hipStream_t s);
 // adjoint launch plan for n_rep replicas of at most max_beads beads whose
@@ -130,8 +141,8 @@ struct AdjPlan {
 // sub-ranges are cut only while the launch holds fewer
 AdjPlan adjoint_plan(int n_rep, int max_beads, size_t bead_stride, int target_wg = 0);
 hipError_t launch_adjoint(const KParams &p, const void *adj_ff, const AdjPlan &a, int rep_first, int n_rep,
-                          int max_bodies, int bead_base, size_t bead_stride, int body_base, double *scratch,
-                          double *force_torque, double *dparams, hipStream_t s);
+                          int max_beads, int body_waves, int bead_base, size_t bead_stride, int body_base, int *fix,
+                          double *scratch, double *force_torque, double *dparams, hipStream_t s);
 hipError_t launch_drms(const KParams &p, int sys_id, int n_beads, int n_rep, const float *rx, const float *ry,
                        const float *rz, double *partials, double inv_pairs, double *out, hipStream_t s);
 size_t drms_units(int n_beads, int n_rep); // partials of launch_drms per replica
@@ -154,12 +165,11 @@ hipError_t launch_gather(const Gather &g, uint32_t *dst, hipStream_t s);
 size_t adjoint_ff_size();
 void adjoint_ff_fill(void *dst, const float *table, double lambda, double e0, double xi, double c_lj, double c_dh);
 
-constexpr int FULL_TILE = 256;
-// full-energy work units per replica of a system with `tiles` bead tiles:
-// row tile x offset 0..tiles/2 of the half-window tile schedule
-__host__ __device__ inline int full_units(int tiles) { return tiles * (tiles / 2 + 1); }
-// largest number of partner sub-ranges a full-energy unit is cut into
-constexpr int FULL_SPLIT_MAX = 4;
+// full energy: tiles of 64 beads; column tiles of a workgroup (at most),
+// workgroups a launch aims at
+__host__ __device__ inline int full_tiles(int beads) { return (beads + 63) / 64; }
+constexpr int FULL_PER_MAX = 32;
+constexpr int FULL_WG = 2048;
 constexpr int SPEC_MAX = 16;     // largest body (beads) a speculative window slot takes
 static_assert(SPEC_MAX > 1, "a window slot's thread 1 forms its rotation");
 constexpr int REMC_MAX_COOP = 8; // workgroups per replica in the cooperative MC kernel

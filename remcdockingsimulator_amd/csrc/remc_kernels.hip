@@ -10,12 +10,6 @@
 //   k_mc_fb<BLOCK,CACHE>  force-biased (smart) MC steps: 1-8 workgroups per
 //                      replica (large moves split), one-bead crowder moves in
 //                      windows.
-//   k_adjoint_*        gradient of one replica's energy: per-body force and
-//                      torque, d/d(lambda, e0, xi).
-//   k_energy_full      batched full energy, every replica in one launch,
-//                      256-bead tiles, half-window tile schedule (each
-//                      unordered tile pair once), Kahan FP32 per thread,
-//                      FP64 per tile; k_sum_partials adds tiles in fixed order.
 //   k_energy_plain     the reference-shaped kernel (E_TiledKernel,
 //                      CudaFunctions.cu:455-685): (G,G) grid of B-bead tiles,
 //                      lower triangle culled, FP32 partial per tile, diagonal
@@ -35,6 +29,7 @@
 
 #include "remc_internal.h"
 #include "remc_math.h"
+#include "remc_pair.h"
 
 namespace remc {
 
@@ -45,44 +40,6 @@ template <typename T>
 __device__ __forceinline__ T lds_ld(const T *ptr)
 {
     return *(const __attribute__((address_space(3))) T *)ptr;
-}
-
-__device__ __forceinline__ float min_image(float d, float box, float inv_box)
-{
-    return __builtin_fmaf(-box, __builtin_rintf(d * inv_box), d);
-}
-
-// Energy of one non-crowder pair from squared distance.  eij4 = 4 E_ij (the
-// table holds the factor 4, so LJ = E (4 x6 (x6 - 1)) costs one FMA: scaling by
-// 4 is exact, the result is the same bits as forming 4 x6 (x6 - 1) and E).
-// SKIP_UNCHARGED: the Debye-Hueckel term is formed under a branch on qq != 0.
-// Four residue types of twenty carry a charge, so where the charge product
-// is the same for a whole wave (one partner bead per wave in the full energy,
-// one moved bead per wave in the MC pair loops) most waves skip the exp2 and
-// its multiplies.  The skipped term is +-0, so the sum is the same number;
-// coincident beads still give NaN from the LJ part (r2 = 0: rinv = inf,
-// x6 = inf, inf*inf - inf) and hence the 1e30 cap.  The plain per-replica
-// kernel forms every term.
-template <bool SKIP_UNCHARGED = true>
-__device__ __forceinline__ float pair_lj_dh(float r2, float eij4, float sij2, float qq, const DevFF &ff)
-{
-    float rinv = __builtin_amdgcn_rsqf(r2);
-    float s2 = sij2 * (rinv * rinv);
-    float x6 = s2 * s2 * s2;
-    float base = __builtin_fmaf(x6, x6, -x6);           // x6 (x6 - 1)
-    bool flip = (eij4 > 0.0f) & (x6 > 0.5f);            // r < 2^(1/6) sigma
-    float e = eij4 * (flip ? base + 0.5f : -base);      // E (LJ + 2) when flipped, else -E LJ
-    if (!SKIP_UNCHARGED || qq != 0.0f) {
-        float r = r2 * rinv;
-        // keeps the exp2 inside the branch (otherwise it is hoisted above it
-        // and the branch becomes a select)
-        if (SKIP_UNCHARGED) asm volatile("" : "+v"(r));
-        e = e + qq * __builtin_amdgcn_exp2f(r * ff.k_dh) * rinv;
-    }
-    // coincident beads (r2 = 0: rinv = inf, r = 0 * inf) give NaN; the cap
-    // (IEEE minNum returns the number) turns it, like any overflow, into 1e30
-    // so compensated sums stay finite
-    return fminf(e, 1e30f);
 }
 
 // pair_lj_dh of an uncharged pair (qq = 0) without the Debye-Hueckel branch,
@@ -113,16 +70,6 @@ __device__ __forceinline__ float pair_lj_dh_k(float r2, float eij4, float sij2, 
     return fminf(e, 1e30f);
 }
 
-// Crowder term C (sigma_c / r)^6 inside the cutoff as crow_k (1/r^2)^3.  r2 = 0
-// (coincident beads) gives inf, capped like the pair term; no clamp is needed
-// since no zero multiplies the infinity.
-__device__ __forceinline__ float pair_crowder(float r2, const DevFF &ff)
-{
-    const float rc = __builtin_amdgcn_rcpf(r2);
-    const float rc3 = rc * rc * rc;
-    return r2 < ff.crow_cut2 ? fminf(ff.crow_k * rc3, 1e30f) : 0.0f;
-}
-
 // pair_crowder with the squared cutoff and the constant given (in the length
 // unit of r2).
 __device__ __forceinline__ float pair_crowder_u(float r2, float cut2, float ck)
@@ -151,13 +98,6 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float v)
     float t = s + y;
     c = (t - s) - y;
     s = t;
-}
-
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
 }
 
 // --------------------------------------------------------------------------
@@ -290,31 +230,6 @@ struct StepDraw {
 };
 constexpr int DRAW_BATCH = 64;
 
-// 64-bit DPP move of a double (both halves with the same control word).
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ double dpp_f64(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    const int l2 = __builtin_amdgcn_update_dpp(0, lo, CTRL, ROW_MASK, 0xf, true);
-    const int h2 = __builtin_amdgcn_update_dpp(0, hi, CTRL, ROW_MASK, 0xf, true);
-    return __hiloint2double(h2, l2);
-}
-
-// Sum over the 64 lanes of a wave in a fixed order, with DPP row shifts and
-// row broadcasts (no LDS traffic); the result is uniform.
-__device__ __forceinline__ double wave_sum_dpp(double v)
-{
-    v += dpp_f64<0x111, 0xf>(v); // row_shr:1
-    v += dpp_f64<0x112, 0xf>(v); // row_shr:2
-    v += dpp_f64<0x114, 0xf>(v); // row_shr:4
-    v += dpp_f64<0x118, 0xf>(v); // row_shr:8: lane 15 of each row holds the row sum
-    v += dpp_f64<0x142, 0xa>(v); // row_bcast:15: rows 1 and 3 add the previous row's sum
-    v += dpp_f64<0x143, 0xc>(v); // row_bcast:31: rows 2 and 3 add lane 31
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
-    return __hiloint2double(hi, lo);
-}
-
 // Squared distance in units of the box between box-scaled positions (x/box):
 // the minimum image of a scaled difference d is d - rint(d).
 __device__ __forceinline__ float dist2_unit(float xj, float yj, float zj, float4 a)
@@ -323,14 +238,6 @@ __device__ __forceinline__ float dist2_unit(float xj, float yj, float zj, float4
     dx -= __builtin_rintf(dx);
     dy -= __builtin_rintf(dy);
     dz -= __builtin_rintf(dz);
-    return __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-}
-
-__device__ __forceinline__ float dist2(float xj, float yj, float zj, float4 a, const DevSys &S)
-{
-    const float dx = min_image(xj - a.x, S.box, S.inv_box);
-    const float dy = min_image(yj - a.y, S.box, S.inv_box);
-    const float dz = min_image(zj - a.z, S.box, S.inv_box);
     return __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
 }
 
@@ -433,7 +340,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
 
     for (int k = tid; k < REMC_NTYPES * REMC_NTYPES; k += BLOCK) {
         s_etab[k] = p.etab[k];
-        s_et2[k] = make_float2(p.etab[k], p.sigtab ? p.sstab[(size_t)R.sys * (REMC_NTYPES * REMC_NTYPES) + k] : 0.0f);
+        s_et2[k] = make_float2(p.etab[k], p.sigtab ? p.sstab[(size_t)2 * R.sys * (REMC_NTYPES * REMC_NTYPES) + k] : 0.0f);
     }
     if (tid == 0) s_abort = 0;
 
@@ -2553,132 +2460,6 @@ int mc_static_lds(int block)
 }
 
 // --------------------------------------------------------------------------
-// batched full energy
-// --------------------------------------------------------------------------
-// One workgroup per (row tile a, offset bo) unit of the half-window tile
-// schedule: tile a against tile (a + bo) mod G for bo = 0..G/2 (the last
-// offset only for a < G/2 when G is even), so every unordered tile pair is
-// visited once.  Unit x = a (G/2 + 1) + bo of each replica writes one FP64
-// partial (0 for the skipped units); k_sum_partials adds them in a fixed
-// order.  When the grid is small (a few replicas of a thousand beads) each
-// unit's partner tile is further cut into `split` equal sub-ranges, one
-// workgroup each, so that every SIMD holds several waves.
-__global__ __launch_bounds__(FULL_TILE) void k_energy_full(KParams p, int stride, int split, double *partials,
-                                                           int noncrowder_only)
-{
-    __shared__ float s_etab[REMC_NTYPES * REMC_NTYPES];
-    __shared__ float s_x[FULL_TILE], s_y[FULL_TILE], s_z[FULL_TILE], s_q[FULL_TILE], s_s[FULL_TILE];
-    __shared__ int s_tc[FULL_TILE], s_body[FULL_TILE];
-    __shared__ double s_red[FULL_TILE / 64];
-
-    const int tid = threadIdx.x;
-    const int x = blockIdx.x / split, sub = blockIdx.x % split, r = blockIdx.y;
-    const DevRep R = p.rep[r];
-    const DevSys S = p.sys[R.sys];
-    const int N = S.n_beads;
-    const int G = (N + FULL_TILE - 1) / FULL_TILE;
-    const int h = G / 2;
-    if (x >= full_units(G)) return; // whole workgroup leaves before any barrier
-    const int a = x / (h + 1), bo = x % (h + 1);
-    if ((G % 2 == 0) && bo == h && bo > 0 && a >= h) {
-        if (tid == 0) partials[(size_t)r * stride + blockIdx.x] = 0.0;
-        return;
-    }
-    const DevFF ff = p.ff;
-    for (int k = tid; k < REMC_NTYPES * REMC_NTYPES; k += FULL_TILE) s_etab[k] = p.etab[k];
-
-    const float *gx = p.px + R.bead_off, *gy = p.py + R.bead_off, *gz = p.pz + R.bead_off;
-    const int *tcs = p.tc + S.bead_off, *bodies = p.body + S.bead_off;
-    const float *qs = p.q + S.bead_off, *sgs = p.sig + S.bead_off;
-
-    const int i = a * FULL_TILE + tid;
-    const bool vi = i < N;
-    const float xi = vi ? gx[i] : 0.f, yi = vi ? gy[i] : 0.f, zi = vi ? gz[i] : 0.f;
-    const int tci = vi ? tcs[i] : 0, bi = vi ? bodies[i] : -1;
-    const float qi = vi ? qs[i] * ff.c_dh : 0.f, si = vi ? sgs[i] : 0.f;
-    const bool ci = (tci >> 8) != 0;
-    const float *erow = s_etab + (tci & 0xff) * REMC_NTYPES;
-
-    float acc = 0.0f, comp = 0.0f;
-    {
-        const int b = (a + bo) % G;
-        const int sw = FULL_TILE / split;
-        const int j0 = b * FULL_TILE + sub * sw;
-        const int jt = j0 + tid;
-        if (tid < sw && jt < N) {
-            s_x[tid] = gx[jt]; s_y[tid] = gy[jt]; s_z[tid] = gz[jt];
-            s_q[tid] = qs[jt]; s_s[tid] = sgs[jt]; s_tc[tid] = tcs[jt]; s_body[tid] = bodies[jt];
-        }
-        __syncthreads();
-        // partner sub-range [j0, j0 + nj): only loaded entries are read
-        const int nj = vi ? min(sw, N - j0) : 0;
-        const int kstart = (bo == 0) ? max(tid + 1 - sub * sw, 0) : 0;
-        for (int k = kstart; k < nj; ++k) {
-            if (s_body[k] == bi) continue;
-            const int tcj = s_tc[k];
-            const bool cj = (tcj >> 8) != 0;
-            if (noncrowder_only && (ci || cj)) continue;
-            float dx = min_image(s_x[k] - xi, S.box, S.inv_box);
-            float dy = min_image(s_y[k] - yi, S.box, S.inv_box);
-            float dz = min_image(s_z[k] - zi, S.box, S.inv_box);
-            float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-            float e;
-            if (ci || cj) {
-                e = pair_crowder(r2, ff);
-            } else {
-                const float sij = 0.5f * (si + s_s[k]);
-                e = pair_lj_dh(r2, erow[tcj & 0xff], sij * sij, qi * s_q[k], ff);
-            }
-            kahan_add(acc, comp, e);
-        }
-    }
-    double v = wave_sum((double)acc - (double)comp);
-    if ((tid & 63) == 0) s_red[tid >> 6] = v;
-    __syncthreads();
-    if (tid == 0) {
-        double t = 0.0;
-        for (int w = 0; w < FULL_TILE / 64; ++w) t += s_red[w];
-        partials[(size_t)r * stride + blockIdx.x] = t;
-    }
-}
-
-// one wave per replica: lane l adds units l, l+64, ... in order, then a
-// fixed butterfly across the wave (the same total on every call)
-__global__ __launch_bounds__(64) void k_sum_partials(KParams p, int stride, int split, const double *partials,
-                                                     double *out, int write_E)
-{
-    const int r = blockIdx.x, lane = threadIdx.x;
-    const DevSys S = p.sys[p.rep[r].sys];
-    const int U = full_units((S.n_beads + FULL_TILE - 1) / FULL_TILE) * split;
-    double t = 0.0;
-    for (int x = lane; x < U; x += 64) t += partials[(size_t)r * stride + x];
-    t = wave_sum(t);
-    if (lane == 0) {
-        if (out) out[r] = t;
-        if (write_E) p.E[r] = t;
-    }
-}
-
-int full_split_default(int n_rep, int max_tiles)
-{
-    const long long units = (long long)full_units(max_tiles) * n_rep;
-    return units >= 2048 ? 1 : units >= 1024 ? 2 : FULL_SPLIT_MAX;
-}
-
-hipError_t launch_energy_full(const KParams &p, int n_rep, int max_tiles, double *partials, double *out,
-                              int noncrowder_only, int write_E, int split, hipStream_t s)
-{
-    if (n_rep <= 0) return hipSuccess;
-    const int max_units = full_units(max_tiles);
-    if (split != 1 && split != 2 && split != FULL_SPLIT_MAX) split = full_split_default(n_rep, max_tiles);
-    const int stride = max_units * FULL_SPLIT_MAX;
-    hipLaunchKernelGGL(k_energy_full, dim3(max_units * split, n_rep), dim3(FULL_TILE), 0, s, p, stride, split,
-                       partials, noncrowder_only);
-    hipLaunchKernelGGL(k_sum_partials, dim3(n_rep), dim3(64), 0, s, p, stride, split, partials, out, write_E);
-    return hipGetLastError();
-}
-
-// --------------------------------------------------------------------------
 // reference-shaped plain kernel (one replica, FP32 tiles, host FP64 sum)
 // --------------------------------------------------------------------------
 template <int B>
@@ -2818,265 +2599,6 @@ hipError_t launch_gather(const Gather &g, uint32_t *dst, hipStream_t s)
     if (words == 0) return hipSuccess;
     hipLaunchKernelGGL(k_gather, dim3((words + 255) / 256), dim3(256), 0, s, g, dst);
     return hipGetLastError();
-}
-
-// --------------------------------------------------------------------------
-// adjoint: gradient of the full energy, every replica of a range in one launch
-//
-// k_adjoint_rows: one workgroup of ADJ_WAVES waves per (row tile of 64 beads,
-// partner sub-range, replica).  The sub-range is staged through LDS in chunks
-// of ADJ_BLOCK beads; wave w takes the staged beads w, w + ADJ_WAVES, ...
-// against its lane's row bead, so every staged value is read as a broadcast.
-// A lane accumulates in FP64, from FP32 pair derivatives (the same branches as
-// the pair term), dE/dx_i of its row bead and the parameter derivatives
-// dE/dlambda = sum dE/dE_ij (T_ij - e0), dE/de0 = -lambda sum dE/dE_ij and
-// dE/dxi = sum DH r / xi^2 over the unordered pairs it owns.  The waves' row
-// gradients are added through LDS in wave order and written once per
-// (sub-range, bead), their parameter sums once per workgroup.
-// k_adjoint_bodies: one wave per (replica, body) adds each bead's sub-range
-// partials in sub-range order, forms F = -sum dE/dx_i and the torque
-// sum rel_i x F_i about the body centre with fixed-order wave sums; the first
-// wave of each replica adds the parameter partials.  The result does not
-// depend on scheduling.  Sub-ranges are only cut when the launch holds fewer
-// than ADJ_TARGET_WG (row tile, replica) workgroups.
-// --------------------------------------------------------------------------
-struct AdjFF {
-    float table[REMC_NTYPES * REMC_NTYPES]; // raw table T_ij
-    float lambda, e0, xi, c_lj, c_dh;
-};
-
-constexpr int ADJ_ROWS = 64;                 // row beads per workgroup (one per lane)
-constexpr int ADJ_WAVES = 4;                 // waves per workgroup
-constexpr int ADJ_BLOCK = 64 * ADJ_WAVES;    // staged partner beads per chunk
-constexpr int ADJ_TARGET_WG = 2048;          // workgroups a launch aims at
-
-__global__ __launch_bounds__(ADJ_BLOCK) void k_adjoint_rows(KParams p, AdjFF af, int rep_first, int tiles, int split,
-                                                            int sub_len, int bead_base, size_t bead_stride,
-                                                            double *part_grad, double *param_part)
-{
-    __shared__ float s_tab[REMC_NTYPES * REMC_NTYPES];
-    __shared__ float s_x[ADJ_BLOCK], s_y[ADJ_BLOCK], s_z[ADJ_BLOCK], s_q[ADJ_BLOCK], s_s[ADJ_BLOCK];
-    __shared__ int s_tc[ADJ_BLOCK], s_body[ADJ_BLOCK];
-    __shared__ double s_g[ADJ_WAVES - 1][3][ADJ_ROWS];
-    __shared__ double s_pp[ADJ_WAVES][3];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int tile = blockIdx.x / split, sub = blockIdx.x % split;
-    const int rr = blockIdx.y;
-    const DevRep R = p.rep[rep_first + rr];
-    const DevSys S = p.sys[R.sys];
-    const DevFF ff = p.ff;
-    const int N = S.n_beads;
-    const int j0 = sub * sub_len;
-    if (tile * ADJ_ROWS >= N || j0 >= N) return; // the whole workgroup, before any barrier
-    const int j1 = min(N, j0 + sub_len);
-    for (int k = tid; k < REMC_NTYPES * REMC_NTYPES; k += ADJ_BLOCK) s_tab[k] = af.table[k];
-    const float *gx = p.px + R.bead_off, *gy = p.py + R.bead_off, *gz = p.pz + R.bead_off;
-    const int *tcs = p.tc + S.bead_off, *bodies = p.body + S.bead_off;
-    const float *qs = p.q + S.bead_off, *sgs = p.sig + S.bead_off;
-    const int i = tile * ADJ_ROWS + lane;
-    const bool vi = i < N;
-    const float xi = vi ? gx[i] : 0.f, yi = vi ? gy[i] : 0.f, zi = vi ? gz[i] : 0.f;
-    const int tci = vi ? tcs[i] : 0, bi = vi ? bodies[i] : -1;
-    const float qi = vi ? qs[i] : 0.f, si = vi ? sgs[i] : 0.f;
-    const bool ci = (tci >> 8) != 0;
-    double gxa = 0.0, gya = 0.0, gza = 0.0, dl = 0.0, de0 = 0.0, dxi = 0.0;
-    const float inv_xi2 = 1.0f / (af.xi * af.xi);
-    for (int c0 = j0; c0 < j1; c0 += ADJ_BLOCK) {
-        const int nc = min(ADJ_BLOCK, j1 - c0);
-        __syncthreads(); // the previous chunk is consumed (first pass: the table is written)
-        if (tid < nc) {
-            const int jt = c0 + tid;
-            s_x[tid] = gx[jt]; s_y[tid] = gy[jt]; s_z[tid] = gz[jt];
-            s_q[tid] = qs[jt]; s_s[tid] = sgs[jt]; s_tc[tid] = tcs[jt]; s_body[tid] = bodies[jt];
-        }
-        __syncthreads();
-        if (vi) {
-            for (int k = wave; k < nc; k += ADJ_WAVES) {
-                if (s_body[k] == bi) continue;
-                const int tcj = s_tc[k];
-                const bool cj = (tcj >> 8) != 0;
-                const float dx = min_image(xi - s_x[k], S.box, S.inv_box);
-                const float dy = min_image(yi - s_y[k], S.box, S.inv_box);
-                const float dz = min_image(zi - s_z[k], S.box, S.inv_box);
-                const float r2 = fmaxf(__builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)), 1e-36f);
-                const float rinv = __builtin_amdgcn_rsqf(r2);
-                const float r = r2 * rinv;
-                float dedr;
-                if (ci || cj) {
-                    const float t = ff.crow_s2 * (rinv * rinv);
-                    const float t6 = t * t * t;
-                    dedr = r2 < ff.crow_cut2 ? -6.0f * ff.c_crow * t6 * rinv : 0.0f;
-                } else {
-                    const int ti = tci & 0xff, tj = tcj & 0xff;
-                    const float traw = s_tab[ti * REMC_NTYPES + tj];
-                    const float eij = af.lambda * (traw - af.e0);
-                    const float sij = 0.5f * (si + s_s[k]);
-                    const float s2 = sij * sij * (rinv * rinv);
-                    const float x6 = s2 * s2 * s2;
-                    const float base = 4.0f * x6 * (x6 - 1.0f);
-                    const float dbase = 4.0f * (2.0f * x6 - 1.0f) * (-6.0f * x6 * rinv);
-                    const bool flip = (eij > 0.0f) & (x6 > 0.5f);
-                    const float dlj = flip ? eij * dbase : -eij * dbase;
-                    const float dlj_de = flip ? base + 2.0f : -base;
-                    const float dh = af.c_dh * qi * s_q[k] * __builtin_amdgcn_exp2f(r * ff.k_dh) * rinv;
-                    const float ddh = -dh * (1.0f / af.xi + rinv);
-                    dedr = af.c_lj * dlj + ddh;
-                    // each unordered pair once for the parameter sums
-                    if (s_body[k] > bi) {
-                        const float de_deij = af.c_lj * dlj_de;
-                        dl += (double)(de_deij * (traw - af.e0));
-                        de0 += (double)(-de_deij * af.lambda);
-                        dxi += (double)(dh * r * inv_xi2);
-                    }
-                }
-                const float kf = dedr * rinv;
-                gxa += (double)(kf * dx);
-                gya += (double)(kf * dy);
-                gza += (double)(kf * dz);
-            }
-        }
-    }
-    if (wave > 0) {
-        s_g[wave - 1][0][lane] = gxa;
-        s_g[wave - 1][1][lane] = gya;
-        s_g[wave - 1][2][lane] = gza;
-    }
-    const double v0 = wave_sum_dpp(dl), v1 = wave_sum_dpp(de0), v2 = wave_sum_dpp(dxi);
-    if (lane == 0) {
-        s_pp[wave][0] = v0;
-        s_pp[wave][1] = v1;
-        s_pp[wave][2] = v2;
-    }
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-        for (int w = 0; w < ADJ_WAVES - 1; ++w) {
-            gxa += s_g[w][0][lane];
-            gya += s_g[w][1][lane];
-            gza += s_g[w][2][lane];
-        }
-        if (vi) {
-            double *pg = part_grad + 3 * ((size_t)sub * bead_stride + (size_t)(R.bead_off - bead_base) + i);
-            pg[0] = gxa;
-            pg[1] = gya;
-            pg[2] = gza;
-        }
-        if (lane < 3) {
-            double t = 0.0;
-#pragma unroll
-            for (int w = 0; w < ADJ_WAVES; ++w) t += s_pp[w][lane];
-            param_part[3 * (((size_t)rr * tiles + tile) * split + sub) + lane] = t;
-        }
-    }
-}
-
-// One wave per (replica, body): the lanes stride over the body's beads, then
-// wave sums (fixed order, so every call gives the same bits); the first wave of
-// workgroup (0, replica) also adds the replica's parameter partials.
-__global__ __launch_bounds__(256) void k_adjoint_bodies(KParams p, int rep_first, int tiles, int split, int sub_len,
-                                                        int bead_base, size_t bead_stride, int body_base,
-                                                        const double *part_grad, const double *param_part,
-                                                        double *force_torque, double *dparams)
-{
-    const int rr = blockIdx.y;
-    const DevRep R = p.rep[rep_first + rr];
-    const DevSys S = p.sys[R.sys];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int N = S.n_beads;
-    const int nsub = (N + sub_len - 1) / sub_len, ntile = (N + ADJ_ROWS - 1) / ADJ_ROWS;
-    if (blockIdx.x == 0 && wave == 0) {
-        double t0 = 0.0, t1 = 0.0, t2 = 0.0;
-        for (int a = lane; a < ntile * nsub; a += 64) {
-            const int tile = a / nsub, sub = a - tile * nsub;
-            const double *pp = param_part + 3 * (((size_t)rr * tiles + tile) * split + sub);
-            t0 += pp[0];
-            t1 += pp[1];
-            t2 += pp[2];
-        }
-        t0 = wave_sum_dpp(t0);
-        t1 = wave_sum_dpp(t1);
-        t2 = wave_sum_dpp(t2);
-        if (lane == 0) {
-            dparams[3 * rr + 0] = t0;
-            dparams[3 * rr + 1] = t1;
-            dparams[3 * rr + 2] = t2;
-        }
-    }
-    const int m = blockIdx.x * (blockDim.x >> 6) + wave;
-    if (m >= S.n_bodies) return;
-    const int b0 = p.bstart[S.body_off + m], b1 = p.bend[S.body_off + m];
-    const float *rx = p.rx + R.bead_off, *ry = p.ry + R.bead_off, *rz = p.rz + R.bead_off;
-    const double *pg = part_grad + 3 * (size_t)(R.bead_off - bead_base);
-    double F[3] = {0.0, 0.0, 0.0}, T[3] = {0.0, 0.0, 0.0};
-    for (int i = b0 + lane; i < b1; i += 64) {
-        double g0 = 0.0, g1 = 0.0, g2 = 0.0;
-        for (int s = 0; s < nsub; ++s) {
-            const double *q = pg + 3 * ((size_t)s * bead_stride + i);
-            g0 += q[0];
-            g1 += q[1];
-            g2 += q[2];
-        }
-        const double f0 = -g0, f1 = -g1, f2 = -g2;
-        F[0] += f0; F[1] += f1; F[2] += f2;
-        const double ax = rx[i], ay = ry[i], az = rz[i];
-        T[0] += ay * f2 - az * f1;
-        T[1] += az * f0 - ax * f2;
-        T[2] += ax * f1 - ay * f0;
-    }
-    for (int k = 0; k < 3; ++k) {
-        F[k] = wave_sum_dpp(F[k]);
-        T[k] = wave_sum_dpp(T[k]);
-    }
-    if (lane == 0) {
-        double *o = force_torque + 6 * ((size_t)(R.body_off - body_base) + m);
-        for (int k = 0; k < 3; ++k) {
-            o[k] = F[k];
-            o[3 + k] = T[k];
-        }
-    }
-}
-
-AdjPlan adjoint_plan(int n_rep, int max_beads, size_t bead_stride, int target_wg)
-{
-    AdjPlan a{};
-    a.tiles = (max_beads + ADJ_ROWS - 1) / ADJ_ROWS;
-    const long long target = target_wg > 0 ? target_wg : ADJ_TARGET_WG;
-    const long long units = (long long)n_rep * a.tiles;
-    const long long want = units >= target ? 1 : (target + units - 1) / units;
-    const long long per = (max_beads + want - 1) / want;
-    a.sub_len = (int)std::max<long long>(ADJ_ROWS, (per + ADJ_ROWS - 1) / ADJ_ROWS * ADJ_ROWS);
-    a.split = (max_beads + a.sub_len - 1) / a.sub_len;
-    a.part_doubles = 3 * (size_t)a.split * bead_stride;
-    a.param_doubles = 3 * (size_t)n_rep * a.tiles * a.split;
-    return a;
-}
-
-hipError_t launch_adjoint(const KParams &p, const void *adj_ff, const AdjPlan &a, int rep_first, int n_rep,
-                          int max_bodies, int bead_base, size_t bead_stride, int body_base, double *scratch,
-                          double *force_torque, double *dparams, hipStream_t s)
-{
-    if (n_rep <= 0) return hipSuccess;
-    double *part_grad = scratch, *param_part = scratch + a.part_doubles;
-    const AdjFF af = *(const AdjFF *)adj_ff;
-    hipLaunchKernelGGL(k_adjoint_rows, dim3(a.tiles * a.split, n_rep), dim3(ADJ_BLOCK), 0, s, p, af, rep_first,
-                       a.tiles, a.split, a.sub_len, bead_base, bead_stride, part_grad, param_part);
-    hipLaunchKernelGGL(k_adjoint_bodies, dim3((max_bodies + 3) / 4, n_rep), dim3(256), 0, s, p, rep_first, a.tiles,
-                       a.split, a.sub_len, bead_base, bead_stride, body_base, part_grad, param_part, force_torque,
-                       dparams);
-    return hipGetLastError();
-}
-
-size_t adjoint_ff_size() { return sizeof(AdjFF); }
-
-void adjoint_ff_fill(void *dst, const float *table, double lambda, double e0, double xi, double c_lj, double c_dh)
-{
-    AdjFF *a = (AdjFF *)dst;
-    for (int k = 0; k < REMC_NTYPES * REMC_NTYPES; ++k) a->table[k] = table[k];
-    a->lambda = (float)lambda;
-    a->e0 = (float)e0;
-    a->xi = (float)xi;
-    a->c_lj = (float)c_lj;
-    a->c_dh = (float)c_dh;
 }
 
 } // namespace remc
