@@ -193,7 +193,7 @@ __device__ __forceinline__ void walk_group(OP &op, const Beads &B, int g, const 
     const int b0 = B.g[4 * g], b1 = B.g[4 * g + 1], kc = B.g[4 * g + 2], chm = B.g[4 * g + 3];
     const int kinds = kc & 0xff, cnt = kc >> 8, j = g * GROUP;
     if (kinds & r.kinds & GROUP_CHAIN) {
-        if (((kinds | r.kinds) & GROUP_CROWDER) == 0 && !diag && (b1 < r.b0 || b0 > r.b1)) {
+        if (((kinds | r.kinds) & GROUP_CROWDER) == 0 && !diag && (b1 < r.b0 || b0 > r.b1) && !op.general()) {
             op.contact(j, cnt, chm, b0 > r.b1);
             return;
         }
@@ -226,8 +226,7 @@ __device__ __forceinline__ void walk_group(OP &op, const Beads &B, int g, const 
 
 // What the kernels below read of the conformation, made once a call:
 //   fix[k * p.copy_beads + b], k = 0..2: coordinate k of replica bead b as a
-//     fraction of its box in units of 2^-32, modulo 1 (a float's product with
-//     2^32/L is exact to 2^-20 of a unit in FP64 for any |x| < 2^12 boxes);
+//     fraction of its box;
 //   then per replica and group of 16 beads (R.grp_off groups before the
 //   replica's) the middle of the range of their coordinates and half its
 //   diagonal, 4 floats.
@@ -241,14 +240,9 @@ __global__ __launch_bounds__(256) void k_fix(KParams p, int rep_first, int *fix)
     const size_t i = (size_t)R.bead_off + min(b, S.n_beads - 1);
     const float x = p.px[i], y = p.py[i], z = p.pz[i];
     if (on && S.box > 0.f) {
-        const double u = 4294967296.0 / (double)S.box;
-        const float src[3] = {x, y, z};
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const double t = (double)src[k] * u;
-            const double w = t - 4294967296.0 * rint(t * (1.0 / 4294967296.0)); // [-2^31, 2^31]
-            fix[k * p.copy_beads + i] = (int)(unsigned)(long long)rint(w);
-        }
+        fix[i] = fix_coord(x, S.unit);
+        fix[p.copy_beads + i] = fix_coord(y, S.unit);
+        fix[2 * p.copy_beads + i] = fix_coord(z, S.unit);
     }
     // lanes past the last bead repeat it
     const float lx = row16<false>(x), ly = row16<false>(y), lz = row16<false>(z);
@@ -275,7 +269,15 @@ static void launch_fix(const KParams &p, int rep_first, int n_rep, int max_beads
 // 32 x 1300 beads: 55 -> 33 us; 64 x 11000 beads: 2.64 -> 1.77 ms (40.5M contact
 // pairs a replica at 24 VALU instructions a wave's 64 of them, 92% of the issue
 // slots; 256-bead tiles staged in LDS took 35 and lost a quarter to padding).
-template <bool TAB, bool PBC>
+// A system of up to FULL_SMALL beads forms its contact pairs from float
+// differences, as the MC kernels form their energies.  A few dilute chains'
+// energy is what is left of terms that nearly cancel, so that a total of other
+// terms than the moves' would show as much of its rounding as of the energy.
+// Such a launch is all latency: 8 replicas of 100 beads take 16.0 us in this form
+// and 15.7 in the other, of 250 beads 17.4 and 17.7.
+constexpr int FULL_SMALL = 256;
+
+template <bool TAB, bool PBC, bool SMALL>
 struct EnergyOp {
     const Beads &B;
     const float *gx, *gy, *gz; // positions, types and groups, for reads by lane
@@ -290,10 +292,12 @@ struct EnergyOp {
     float qu, kdh;      // the row's charge times the Debye-Hueckel coefficient, and the exponent scale, in the unit of
                         // contact distances
     float u2, u2l;      // 1 A^2 in the unit squared (high and low part)
+    float q;            // the row's charge times the Debye-Hueckel coefficient
     bool free_only;     // non-crowder pairs only
     double acc;
 
     __device__ __forceinline__ bool crowders() const { return !free_only; }
+    __device__ __forceinline__ bool general() const { return SMALL; }
     struct Term {
         float r2, x6, e4, e;
     };
@@ -368,10 +372,18 @@ struct EnergyOp {
             load_columns<TAB, PBC, 1>(B, j + k, &c);
             if ((c.tc >> 8) != 0) continue; // uniform
             const bool on = B.body[j + k] != r.body && !r.crow && (!diag || j + k > r.i);
-            Term t = term(c);
-            flip(t);
-            if (chm & (1 << k)) charged(t, c.q);
-            acc += (double)(on ? fminf(t.e, 1e30f) : 0.0f);
+            float e;
+            if (SMALL) {
+                const float sij = 0.5f * (s + B.s[j + k]);
+                e = pair_lj_dh(dist2(B.x[j + k], B.y[j + k], B.z[j + k], make_float4(r.x, r.y, r.z, 0.f), S), erow[c.tc].x,
+                               sij * sij, q * c.q, ff);
+            } else {
+                Term t = term(c);
+                flip(t);
+                if (chm & (1 << k)) charged(t, c.q);
+                e = fminf(t.e, 1e30f);
+            }
+            acc += (double)(on ? e : 0.0f);
         }
     }
     __device__ __forceinline__ void crowder(int j, bool diag)
@@ -401,9 +413,6 @@ __device__ __forceinline__ Beads replica_beads(const KParams &p, const DevRep &R
             (Uniform<float>)(fix + fix_centres(p.copy_beads) + 4 * (size_t)R.grp_off)};
 }
 
-// Units of contact distances per Angstrom.
-__device__ __forceinline__ double units(const DevSys &S) { return S.box > 0.f ? 4294967296.0 / (double)S.box : 1.0; }
-
 // The type table of the contact pairs in LDS: scale e_ij, sigma_ij^2 in the
 // unit squared (u2) as high and low part, w_ij.
 __device__ __forceinline__ void load_table(float4 *s_et, const KParams &p, int sys, const float *e, float scale, double u2,
@@ -430,7 +439,7 @@ __global__ __launch_bounds__(COLS) void k_energy_full(KParams p, const int *fix,
     const Beads B = replica_beads(p, R, S, fix);
     const float *gx = p.px + R.bead_off, *gy = p.py + R.bead_off, *gz = p.pz + R.bead_off;
     const int *tcs = p.tc + S.bead_off, *bodies = p.body + S.bead_off;
-    const double unit = units(S), u2 = unit * unit;
+    const double unit = S.unit, u2 = unit * unit; // of contact distances, per Angstrom
     const float u2h = (float)u2, u2l = (float)(u2 - (double)u2h);
     const float4 *gc = (const float4 *)(fix + fix_centres(p.copy_beads)) + R.grp_off;
     load_table(s_et, p, R.sys, p.etab, 1.0f, u2, nullptr);
@@ -438,7 +447,7 @@ __global__ __launch_bounds__(COLS) void k_energy_full(KParams p, const int *fix,
     // this workgroup's column tiles, of all row tiles' in order
     const long long all = (long long)T * (h + 1);
     const int u0 = (int)(all * blockIdx.x / gridDim.x), u1 = (int)(all * (blockIdx.x + 1) / gridDim.x);
-    auto walk = [&](auto tab, auto pbc) {
+    auto walk = [&](auto tab, auto pbc, auto small) {
         double sum = 0.0;
         for (int u = u0; u < u1;) {
             const int a = u / (h + 1), bo0 = u % (h + 1), end = min(h + 1, bo0 + (u1 - u));
@@ -449,10 +458,10 @@ __global__ __launch_bounds__(COLS) void k_energy_full(KParams p, const int *fix,
             const int i = row.on ? row.i : N - 1;
             const RowFix rf = load_row_fix(row, fix + R.bead_off, fix + p.copy_beads + R.bead_off,
                                            fix + 2 * p.copy_beads + R.bead_off, N);
-            EnergyOp<decltype(tab)::value, decltype(pbc)::value> op{
+            EnergyOp<decltype(tab)::value, decltype(pbc)::value, decltype(small)::value> op{
                 B, gx, gy, gz, tcs, gc, row, rf, S, ff, s_et + row.type * TSTRIDE, p.sig[S.bead_off + i],
                 (float)((double)(p.q[S.bead_off + i] * ff.c_dh) * unit), (float)((double)ff.k_dh / unit), u2h, u2l,
-                noncrowder_only != 0, 0.0};
+                p.q[S.bead_off + i] * ff.c_dh, noncrowder_only != 0, 0.0};
             for (int k = (ROWS / GROUP) * bo0 + wave; k < (ROWS / GROUP) * bo1; k += WAVES) {
                 int t = a + k / (ROWS / GROUP);
                 if (t >= T) t -= T;
@@ -465,8 +474,9 @@ __global__ __launch_bounds__(COLS) void k_energy_full(KParams p, const int *fix,
     };
     using T1 = std::true_type;
     using T0 = std::false_type;
-    const double v = wave_sum_dpp(S.box > 0.f ? (p.sigtab ? walk(T1{}, T1{}) : walk(T0{}, T1{}))
-                                              : (p.sigtab ? walk(T1{}, T0{}) : walk(T0{}, T0{})));
+    const double v = wave_sum_dpp(N <= FULL_SMALL ? walk(T0{}, T0{}, T1{})
+                                  : S.box > 0.f   ? (p.sigtab ? walk(T1{}, T1{}, T0{}) : walk(T0{}, T1{}, T0{}))
+                                                  : (p.sigtab ? walk(T1{}, T0{}, T0{}) : walk(T0{}, T0{}, T0{})));
     if (lane == 0) s_red[wave] = v;
     __syncthreads();
     if (tid == 0) {
@@ -560,6 +570,7 @@ struct AdjointOp {
     double ux, uy, uz, pl, pe, px, ax, ay, az;
 
     __device__ __forceinline__ bool crowders() const { return true; }
+    __device__ __forceinline__ bool general() const { return false; }
     struct Term {
         float dx, dy, dz, r2, inv2, x6, kf, u, t0, dhr;
     };
@@ -711,7 +722,7 @@ __global__ __launch_bounds__(COLS) void k_adjoint_rows(KParams p, AdjFF af, int 
     const int j1 = min(N, j0 + sub_len);
     const Beads B = replica_beads(p, R, S, fix);
     const float *gx = p.px + R.bead_off, *gy = p.py + R.bead_off, *gz = p.pz + R.bead_off;
-    const double unit = units(S), u2 = unit * unit;
+    const double unit = S.unit, u2 = unit * unit; // of contact distances, per Angstrom
     const float u2h = (float)u2, u2l = (float)(u2 - (double)u2h);
     const float4 *gc = (const float4 *)(fix + fix_centres(p.copy_beads)) + R.grp_off;
     load_table(s_et, p, R.sys, af.e, 24.0f * af.c_lj, u2, af.t0);

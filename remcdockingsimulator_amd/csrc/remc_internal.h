@@ -29,6 +29,7 @@ struct DevSys {
     float box, inv_box;
     int grp_off; // groups of 16 beads of the systems before it
     int n_multi; // bodies of several beads
+    double unit; // 2^32 / box (1 without a box): units of fixed-point distances per Angstrom
 };
 
 struct DevRep {

@@ -65,6 +65,16 @@ __device__ __forceinline__ float dist2(float xj, float yj, float zj, float4 a, c
     return __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
 }
 
+// A coordinate as a 32-bit fraction of the box (unit = 2^32/L units per
+// Angstrom), modulo 1: the difference of two, taken in 32 bits, wraps to the
+// nearest image.  x unit + 1.5 2^52 has a unit of 1 in its last place, so the
+// low word of the sum is x unit rounded to a whole number, modulo 2^32 (for any
+// |x| < 2^19 boxes).
+__device__ __forceinline__ int fix_coord(float x, double unit)
+{
+    return __double2loint(__builtin_fma((double)x, unit, 6755399441055744.0));
+}
+
 // 64-bit DPP move of a double (both halves with the same control word).
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ double dpp_f64(double v)
