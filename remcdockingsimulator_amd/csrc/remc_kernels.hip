@@ -42,32 +42,44 @@ __device__ __forceinline__ T lds_ld(const T *ptr)
     return *(const __attribute__((address_space(3))) T *)ptr;
 }
 
-// pair_lj_dh of an uncharged pair (qq = 0) without the Debye-Hueckel branch,
-// with (sigma/r)^2 from one reciprocal instead of a squared reciprocal root
-// (the two differ in the last bits; a difference en - eo is always formed
-// from one of the two forms).
-__device__ __forceinline__ float pair_lj(float r2, float eij4, float sij2)
+// The contact pairs of the large moves' passes, in parts: (sigma/r)^6 of an
+// uncharged pair from one reciprocal, of a charged one from the reciprocal root
+// that its Debye-Hueckel term needs (the two differ in the last bits; a
+// difference en - eo is always formed from one of the two forms), and the energy
+// from it.  FAR: x6 <= 1/2, where neither the flip nor the cap acts.
+__device__ __forceinline__ float pair_x6(float r2, float sij2)
 {
-    float s2 = sij2 * __builtin_amdgcn_rcpf(r2);
-    float x6 = s2 * s2 * s2;
-    float base = __builtin_fmaf(x6, x6, -x6);
-    bool flip = (eij4 > 0.0f) & (x6 > 0.5f);
-    float e = eij4 * (flip ? base + 0.5f : -base);
-    return fminf(e, 1e30f);
+    const float s2 = sij2 * __builtin_amdgcn_rcpf(r2);
+    return s2 * s2 * s2;
 }
 
-// pair_lj_dh of every pair, charged or not, with the Debye-Hueckel exponent
-// scale given (k_dh times the length unit of r2).
-__device__ __forceinline__ float pair_lj_dh_k(float r2, float eij4, float sij2, float qq, float kdh)
+__device__ __forceinline__ float pair_x6_root(float rinv, float sij2)
 {
-    float rinv = __builtin_amdgcn_rsqf(r2);
-    float s2 = sij2 * (rinv * rinv);
-    float x6 = s2 * s2 * s2;
-    float base = __builtin_fmaf(x6, x6, -x6);
-    bool flip = (eij4 > 0.0f) & (x6 > 0.5f);
-    float e = eij4 * (flip ? base + 0.5f : -base);
-    e = e + qq * __builtin_amdgcn_exp2f(r2 * rinv * kdh) * rinv;
-    return fminf(e, 1e30f);
+    const float s2 = sij2 * (rinv * rinv);
+    return s2 * s2 * s2;
+}
+
+// (Products and differences are rounded one by one, the fused operations are
+// written out: the terms are the same numbers on both branches.)
+template <bool FAR>
+__device__ __forceinline__ float pair_lj_x6(float x6, float eij4)
+{
+#pragma clang fp contract(off)
+    const float base = __builtin_fmaf(x6, x6, -x6);
+    if (FAR) return eij4 * -base;
+    const bool flip = (eij4 > 0.0f) & (x6 > 0.5f);
+    return fminf(eij4 * (flip ? base + 0.5f : -base), 1e30f);
+}
+
+template <bool FAR>
+__device__ __forceinline__ float pair_lj_dh_x6(float x6, float r2, float rinv, float eij4, float qq, float kdh)
+{
+#pragma clang fp contract(off)
+    const float base = __builtin_fmaf(x6, x6, -x6);
+    const bool flip = !FAR && (eij4 > 0.0f) & (x6 > 0.5f);
+    const float dh = qq * __builtin_amdgcn_exp2f(r2 * rinv * kdh) * rinv;
+    const float e = __builtin_fmaf(eij4, flip ? base + 0.5f : -base, dh);
+    return FAR ? e : fminf(e, 1e30f);
 }
 
 // pair_crowder with the squared cutoff and the constant given (in the length
@@ -1097,8 +1109,9 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
         pick_split_memo<BLOCK>(smemo, nmu, nj, lane, G, kper);
         const int g = div_floor_small(tid, G), l = tid - g * G;
         const int k0 = min(nm, g * kper), k1 = min(nm, k0 + kper);
-        // compensated (Kahan) FP32 sum of the differences en - eo per thread
-        float acc = 0.0f, comp = 0.0f;
+        // FP64 sum of the differences en - eo per thread (an FP64 add is issued at
+        // the rate of an FP32 one here: two instructions a pass, four compensated)
+        double acc = 0.0;
         // two partner beads in registers per pass (jj0 and jj0 + G): each moved
         // bead's staging is read once for both
         for (int jj0 = l; jj0 < nj; jj0 += 2 * G) {
@@ -1171,22 +1184,45 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                         }
                         const float ro0 = dist2_unit(xs[0], ys[0], zs[0], o), rn0 = dist2_unit(xs[0], ys[0], zs[0], n);
                         const float ro1 = dist2_unit(xs[1], ys[1], zs[1], o), rn1 = dist2_unit(xs[1], ys[1], zs[1], n);
+                        // none of the x6 is negative, so a sum of at most 1/2
+                        // bounds each (and is no NaN): the flips and the caps of
+                        // the four terms sit behind one test of the wave
                         float eo0, en0, eo1, en1;
                         if (__any(o.w != 0.0f)) {
                             const float qq0 = o.w * qj[0], qq1 = o.w * qj[1];
-                            eo0 = pair_lj_dh_k(ro0, e0.x, ss0, qq0, kdh);
-                            en0 = pair_lj_dh_k(rn0, e0.x, ss0, qq0, kdh);
-                            eo1 = pair_lj_dh_k(ro1, e1.x, ss1, qq1, kdh);
-                            en1 = pair_lj_dh_k(rn1, e1.x, ss1, qq1, kdh);
+                            const float io0 = __builtin_amdgcn_rsqf(ro0), in0 = __builtin_amdgcn_rsqf(rn0),
+                                        io1 = __builtin_amdgcn_rsqf(ro1), in1 = __builtin_amdgcn_rsqf(rn1);
+                            const float xo0 = pair_x6_root(io0, ss0), xn0 = pair_x6_root(in0, ss0),
+                                        xo1 = pair_x6_root(io1, ss1), xn1 = pair_x6_root(in1, ss1);
+                            if (__all((xo0 + xn0) + (xo1 + xn1) <= 0.5f)) {
+                                eo0 = pair_lj_dh_x6<true>(xo0, ro0, io0, e0.x, qq0, kdh);
+                                en0 = pair_lj_dh_x6<true>(xn0, rn0, in0, e0.x, qq0, kdh);
+                                eo1 = pair_lj_dh_x6<true>(xo1, ro1, io1, e1.x, qq1, kdh);
+                                en1 = pair_lj_dh_x6<true>(xn1, rn1, in1, e1.x, qq1, kdh);
+                            } else {
+                                eo0 = pair_lj_dh_x6<false>(xo0, ro0, io0, e0.x, qq0, kdh);
+                                en0 = pair_lj_dh_x6<false>(xn0, rn0, in0, e0.x, qq0, kdh);
+                                eo1 = pair_lj_dh_x6<false>(xo1, ro1, io1, e1.x, qq1, kdh);
+                                en1 = pair_lj_dh_x6<false>(xn1, rn1, in1, e1.x, qq1, kdh);
+                            }
                         } else {
-                            eo0 = pair_lj(ro0, e0.x, ss0);
-                            en0 = pair_lj(rn0, e0.x, ss0);
-                            eo1 = pair_lj(ro1, e1.x, ss1);
-                            en1 = pair_lj(rn1, e1.x, ss1);
+                            const float xo0 = pair_x6(ro0, ss0), xn0 = pair_x6(rn0, ss0), xo1 = pair_x6(ro1, ss1),
+                                        xn1 = pair_x6(rn1, ss1);
+                            if (__all((xo0 + xn0) + (xo1 + xn1) <= 0.5f)) {
+                                eo0 = pair_lj_x6<true>(xo0, e0.x);
+                                en0 = pair_lj_x6<true>(xn0, e0.x);
+                                eo1 = pair_lj_x6<true>(xo1, e1.x);
+                                en1 = pair_lj_x6<true>(xn1, e1.x);
+                            } else {
+                                eo0 = pair_lj_x6<false>(xo0, e0.x);
+                                en0 = pair_lj_x6<false>(xn0, e0.x);
+                                eo1 = pair_lj_x6<false>(xo1, e1.x);
+                                en1 = pair_lj_x6<false>(xn1, e1.x);
+                            }
                         }
                         // the two partners' differences are added (one rounding, as
-                        // each difference has), then to the compensated sum
-                        kahan_add(acc, comp, (en0 - eo0) + (on[1] ? en1 - eo1 : 0.0f));
+                        // each difference has), then in FP64
+                        acc += (double)((en0 - eo0) + (on[1] ? en1 - eo1 : 0.0f));
                     }
                 };
                 if (p.sigtab)
@@ -1215,7 +1251,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                     const float en0 = pair_crowder_u(dist2_unit(xs[0], ys[0], zs[0], n), cut2, ck);
                     const float eo1 = pair_crowder_u(dist2_unit(xs[1], ys[1], zs[1], o), cut2, ck);
                     const float en1 = pair_crowder_u(dist2_unit(xs[1], ys[1], zs[1], n), cut2, ck);
-                    kahan_add(acc, comp, (en0 - eo0) + (on[1] ? en1 - eo1 : 0.0f));
+                    acc += (double)((en0 - eo0) + (on[1] ? en1 - eo1 : 0.0f));
                 }
                 continue;
             }
@@ -1237,11 +1273,11 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                         eo = pair_lj_dh(dist2(xj[u], yj[u], zj[u], o, S), eij, sij2, qq, ff);
                         en = pair_lj_dh(dist2(xj[u], yj[u], zj[u], n, S), eij, sij2, qq, ff);
                     }
-                    kahan_add(acc, comp, en - eo);
+                    acc += (double)(en - eo);
                 }
             }
         }
-        const double v = wave_sum_dpp((double)acc - (double)comp);
+        const double v = wave_sum_dpp(acc);
         if (lane == 0) s_red[wave] = v;
         __syncthreads();
         double dE = 0.0;
