@@ -150,6 +150,7 @@ struct remc_ctx {
     unsigned long long *d_rec_start = nullptr;
     int rec_max = 0;
     unsigned long long *d_slots = nullptr;
+    int slot_row = 0; // entries of a row that d_slots has room for
     int *d_err = nullptr;
     uint32_t *h_pin = nullptr; // pinned host memory that read-backs go through (ReadBack)
     size_t pin_words = 0;
@@ -167,7 +168,16 @@ struct remc_ctx {
     int mc_block = 0;
     int mc_coop = 0;
     int coop_min_pairs = 8192; // moves below this many pair terms are evaluated whole by every member
-    int synced_copies = 1;   // state copies [0, synced_copies) hold the current conformation
+    // The workgroups of an MC launch (KParams::wg), made once and kept: as many
+    // for every replica (coop), or by the systems' cost at a workgroup size
+    // (coop = 0).
+    struct McPlan {
+        int coop, block, grid, row;
+        McWg *wg;
+    };
+    std::vector<McPlan> plans;
+    bool mc_balanced = false; // autotuned: the members follow the systems' cost (mc_coop is then 1)
+    const McWg *synced = nullptr; // the workgroups whose state copies hold the current conformation (null: none but the canonical)
     int n_cu = 0;
     int lds_per_block = 0, lds_per_cu = 0;
     bool lds_cache = true;   // partner-bead LDS cache of the MC kernel allowed
@@ -514,7 +524,9 @@ int finalize(remc_ctx *c)
     HIP_TRY(dalloc(&c->d_cy, cy.size() * REMC_MAX_COOP));
     HIP_TRY(dalloc(&c->d_cz, cz.size() * REMC_MAX_COOP));
     HIP_TRY(dalloc(&c->d_quat, quat.size() * REMC_MAX_COOP));
-    HIP_TRY(dalloc(&c->d_slots, (size_t)R * REMC_SLOTS_PER_REP));
+    // (every launch that uses the slots empties them first)
+    HIP_TRY(dalloc(&c->d_slots, (size_t)R * 2 * REMC_SLOT_K * REMC_MAX_COOP));
+    c->slot_row = REMC_MAX_COOP;
     HIP_TRY(dalloc(&c->d_err, (size_t)1));
     HIP_TRY(dalloc(&c->d_E, (size_t)R));
     HIP_TRY(dalloc(&c->d_T, (size_t)R));
@@ -566,8 +578,6 @@ int finalize(remc_ctx *c)
     HIP_TRY(upload(c->d_exswaps, zeros_s, s));
     HIP_TRY(upload(c->d_exoff, zeros_si, s));
     {
-        std::vector<unsigned long long> empty((size_t)R * REMC_SLOTS_PER_REP, ~0ull);
-        HIP_TRY(upload(c->d_slots, empty, s));
         int zero = 0;
         HIP_TRY(hipMemcpyAsync(c->d_err, &zero, sizeof(int), hipMemcpyHostToDevice, s));
     }
@@ -598,7 +608,7 @@ int finalize(remc_ctx *c)
                                                   adj_words <= PIN_ADJ_WORDS ? adj_words : 0}) + 8));
     if (prc != REMC_OK) return prc;
     HIP_TRY(hipStreamSynchronize(s));
-    c->synced_copies = 1;
+    c->synced = nullptr;
     c->finalized = true;
 
     // initial energies of every replica
@@ -625,20 +635,48 @@ int finalize(remc_ctx *c)
         if ((r) < 0 || (r) >= (int)(c)->reps.size()) return fail(REMC_ERR_ARG, "replica %d out of range", (r)); \
     } while (0)
 
-// Copies [synced_copies, coop) of the dynamic state are refreshed from copy 0.
-int sync_copies(remc_ctx *c, int coop)
+hipError_t upload_wg(const std::vector<McWg> &wg, McWg **out)
 {
-    if (c->synced_copies >= coop) return REMC_OK;
-    const size_t nb = (size_t)c->total_rep_beads, nm = (size_t)c->total_rep_bodies;
-    float *fb[6] = {c->d_px, c->d_py, c->d_pz, c->d_rx, c->d_ry, c->d_rz};
-    float *fm[3] = {c->d_cx, c->d_cy, c->d_cz};
-    for (int k = c->synced_copies; k < coop; ++k) {
-        for (float *a : fb) HIP_TRY(hipMemcpyAsync(a + k * nb, a, nb * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-        for (float *a : fm) HIP_TRY(hipMemcpyAsync(a + k * nm, a, nm * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-        HIP_TRY(hipMemcpyAsync(c->d_quat + 4 * k * nm, c->d_quat, 4 * nm * sizeof(double), hipMemcpyDeviceToDevice,
-                               c->stream));
+    hipError_t e = dalloc(out, wg.size());
+    if (e != hipSuccess) return e;
+    e = hipMemcpy(*out, wg.data(), wg.size() * sizeof(McWg), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipFree(*out);
+        *out = nullptr;
     }
-    c->synced_copies = coop;
+    return e;
+}
+
+// The plan with coop workgroups for every replica (copy k of the state is
+// [k * total, (k + 1) * total) of the dynamic arrays).
+int uniform_plan(remc_ctx *c, int coop, remc_ctx::McPlan *out)
+{
+    for (const auto &pl : c->plans)
+        if (pl.coop == coop) {
+            *out = pl;
+            return REMC_OK;
+        }
+    const int R = (int)c->reps.size();
+    std::vector<McWg> wg((size_t)R * coop);
+    for (int k = 0; k < coop; ++k)
+        for (int r = 0; r < R; ++r)
+            wg[(size_t)k * R + r] = {r, k, coop, 0, (long long)k * c->total_rep_beads + c->rep_bead_off[r],
+                                     (long long)k * c->total_rep_bodies + c->rep_body_off[r]};
+    remc_ctx::McPlan pl{coop, 0, R * coop, REMC_MAX_COOP, nullptr};
+    HIP_TRY(upload_wg(wg, &pl.wg));
+    c->plans.push_back(pl);
+    *out = pl;
+    return REMC_OK;
+}
+
+// The state copies of a plan's members are refreshed from the canonical state.
+int sync_members(remc_ctx *c, const remc_ctx::McPlan &pl)
+{
+    if (c->synced == pl.wg || pl.coop == 1) return REMC_OK;
+    KParams p = c->params();
+    p.wg = pl.wg;
+    HIP_TRY(launch_copy_state(p, pl.grid, c->stream));
+    c->synced = pl.wg;
     return REMC_OK;
 }
 
@@ -709,10 +747,12 @@ int energies_out(remc_ctx *c, int noncrowder_only, double *out)
 // always; the partner beads of the replica (or of the member's slice when
 // every move is split) and the body table when they fit the LDS share of one
 // workgroup at the occupancy the grid needs.
-void fill_mc_lds(remc_ctx *c, KParams &p, int coop, int block)
+void fill_mc_lds(remc_ctx *c, KParams &p, const remc_ctx::McPlan &pl, int block)
 {
-    const int R = (int)c->reps.size();
-    const long long wgs = (long long)R * coop;
+    const int coop = std::max(1, pl.coop);
+    const long long wgs = pl.grid;
+    p.wg = pl.wg;
+    p.slot_row = pl.row;
     const int per_cu = (int)std::max<long long>(1, (wgs + c->n_cu - 1) / c->n_cu);
     // etab, draws, window staging and reduction scratch, as the kernel declares them, and slack
     const int kernel_lds = mc_static_lds(block);
@@ -726,7 +766,8 @@ void fill_mc_lds(remc_ctx *c, KParams &p, int coop, int block)
     p.cache_bodies = 0;
     p.cache_rel = 0;
     p.cache_quat = 0;
-    p.spec = 0;
+    // speculative windows, with the partners from the cache or from HBM
+    p.spec = c->mc_window ? 1 : 0;
     p.draw2 = 0;
     if (!c->lds_cache || budget <= 0) return;
     const long long full = 24LL * c->max_beads;
@@ -743,8 +784,6 @@ void fill_mc_lds(remc_ctx *c, KParams &p, int coop, int block)
         } else {
             return;
         }
-        // speculative windows read the partner range (the replica, or the member's slice) from LDS
-        p.spec = c->mc_window ? 1 : 0;
         if (20LL * c->max_bodies <= budget) {
             p.lds_nbody = c->max_bodies;
             p.cache_bodies = 1;
@@ -770,30 +809,177 @@ void fill_mc_lds(remc_ctx *c, KParams &p, int coop, int block)
     }
 }
 
+// Workgroups of a plan that run at once at this workgroup size.
+int resident(remc_ctx *c, const remc_ctx::McPlan &pl, int block, long long *out)
+{
+    KParams p = c->params();
+    fill_mc_lds(c, p, pl, block);
+    int per_cu = 0;
+    HIP_TRY(mc_max_active_per_cu(p, block, &per_cu));
+    *out = (long long)per_cu * c->n_cu;
+    return REMC_OK;
+}
+
 // Largest workgroups-per-replica count whose grid is co-resident.
 int max_coop(remc_ctx *c, int block, int *out)
 {
     const int R = (int)c->reps.size();
     int m = REMC_MAX_COOP;
     for (; m > 1; m >>= 1) {
-        KParams p = c->params();
-        fill_mc_lds(c, p, m, block);
-        int per_cu = 0;
-        HIP_TRY(mc_max_active_per_cu(p, block, &per_cu));
-        if ((long long)m * R <= (long long)per_cu * c->n_cu) break;
+        long long fit = 0;
+        const int rc = resident(c, {m, 0, R * m, REMC_MAX_COOP, nullptr}, block, &fit);
+        if (rc != REMC_OK) return rc;
+        if ((long long)m * R <= fit) break;
     }
     *out = m;
     return REMC_OK;
 }
 
-int mc_launch(remc_ctx *c, const KParams &p0, int nsteps, int block, int coop)
+// A plan for unequal systems: members by cost.  The replicas of a launch run
+// side by side, so it ends with its slowest, and a step of a system of long
+// chains and few crowders (most of its moves are chains') costs a hundred times
+// the pair terms of a light one's: with as many workgroups for every replica a
+// few replicas held the launch while the rest of the device idled.  64 systems
+// of 500-4000 beads, 512 replicas, 500 steps: 27.8 ms with one workgroup each
+// (the most that fits), 6.9 ms with 1-16 members on 1024 workgroups.  The
+// estimate of a step is its moves' mean pair terms, those of windows and split
+// moves over the members, at MC_TERMS_US terms a microsecond and 256 threads,
+// and MC_EXCHANGE_US for each split move's exchange; the slowest system's
+// replicas take one member more while the grid stays co-resident and the copies
+// fit.  (0.5, 2 and 8 us an exchange: 6.9, 7.3 and 7.2 ms; doubling instead of
+// one more: 7.35 ms.)  Members of a replica are placed on one XCD (workgroup b
+// runs on XCD b mod 8), each XCD's in order of cost, so that the costly ones
+// start first and on different CUs.  No plan (grid 0) where that leaves one
+// workgroup per replica.
+constexpr double MC_TERMS_US = 1300.0; // a quarter of a CU
+constexpr double MC_EXCHANGE_US = 0.5;
+
+int balanced_plan(remc_ctx *c, int block, remc_ctx::McPlan *out)
 {
-    int rc = sync_copies(c, coop);
+    for (const auto &pl : c->plans)
+        if (pl.coop == 0 && pl.block == block) {
+            *out = pl;
+            return REMC_OK;
+        }
+    const int R = (int)c->reps.size(), n_sys = (int)c->systems.size(), xcds = 8;
+    remc_ctx::McPlan pl{0, block, R, REMC_MAX_MEMBERS, nullptr};
+    // with the caches that a filled device leaves room for (4 waves a SIMD)
+    long long fit = 0;
+    pl.grid = c->n_cu * (1024 / block);
+    int rc = resident(c, pl, block, &fit);
+    if (rc != REMC_OK) return rc;
+    const double rate = MC_TERMS_US * block / 256;
+    std::vector<double> whole(n_sys, 0.0), split(n_sys, 0.0), moves(n_sys, 0.0);
+    for (int s = 0; s < n_sys; ++s) {
+        const HostSys &hs = c->systems[s];
+        if (hs.replicas.empty()) continue; // no cost
+        for (int m = 0; m < hs.n_bodies; ++m) {
+            const double nm = hs.body_start[m + 1] - hs.body_start[m], pairs = nm * (hs.n_beads - nm);
+            const bool window = c->mc_window && nm <= SPEC_MAX; // split, many moves to an exchange
+            (window || pairs >= c->coop_min_pairs ? split : whole)[s] += 2.0 * pairs / hs.n_bodies / rate;
+            if (pairs >= c->coop_min_pairs && !window) moves[s] += 1.0 / hs.n_bodies;
+        }
+    }
+    std::vector<int> coop(n_sys, 1);
+    auto cost = [&](int s, int k) { return whole[s] + split[s] / k + (k > 1 ? MC_EXCHANGE_US * moves[s] : 0.0); };
+    // each XCD's replicas: the next costly one goes where the fewest workgroups are
+    std::vector<int> order;
+    for (int r = 0; r < R; ++r) order.push_back(r);
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int a, int b) { return cost(c->reps[a].sys, 1) > cost(c->reps[b].sys, 1); });
+    std::vector<std::vector<int>> queue;
+    auto place = [&] {
+        std::vector<long long> len(xcds, 0);
+        queue.assign(xcds, {});
+        for (int r : order) {
+            const int x = (int)(std::min_element(len.begin(), len.end()) - len.begin());
+            queue[x].push_back(r);
+            len[x] += coop[c->reps[r].sys];
+        }
+        return xcds * *std::max_element(len.begin(), len.end());
+    };
+    long long members = R, beads = c->total_rep_beads, bodies = c->total_rep_bodies;
+    for (;;) {
+        int s = 0;
+        for (int t = 1; t < n_sys; ++t)
+            if (cost(t, coop[t]) > cost(s, coop[s])) s = t;
+        const HostSys &hs = c->systems[s];
+        const long long more = (long long)hs.replicas.size();
+        if (coop[s] >= REMC_MAX_MEMBERS || cost(s, coop[s] + 1) >= cost(s, coop[s])) break;
+        if (beads + more * hs.n_beads > (long long)REMC_MAX_COOP * c->total_rep_beads ||
+            bodies + more * hs.n_bodies > (long long)REMC_MAX_COOP * c->total_rep_bodies)
+            break;
+        ++coop[s];
+        if (place() > fit) {
+            --coop[s];
+            break;
+        }
+        members += more;
+        beads += more * hs.n_beads;
+        bodies += more * hs.n_bodies;
+    }
+    pl.grid = 0;
+    std::vector<McWg> wg;
+    if (members > R) {
+        pl.grid = (int)place();
+        wg.assign(pl.grid, McWg{-1, 0, 0, 0, 0, 0});
+        long long bead = c->total_rep_beads, body = c->total_rep_bodies;
+        for (int x = 0; x < xcds; ++x) {
+            size_t at = x;
+            for (int r : queue[x]) {
+                const HostSys &hs = c->systems[c->reps[r].sys];
+                const int k = coop[c->reps[r].sys];
+                for (int m = 0; m < k; ++m, at += xcds) {
+                    wg[at] = {r, m, k, 0, m == 0 ? c->rep_bead_off[r] : bead, m == 0 ? c->rep_body_off[r] : body};
+                    if (m > 0) {
+                        bead += hs.n_beads;
+                        body += hs.n_bodies;
+                    }
+                }
+            }
+        }
+        // members wait for each other: all must run at once
+        rc = resident(c, pl, block, &fit);
+        if (rc != REMC_OK) return rc;
+        if (pl.grid > fit) pl.grid = 0;
+    }
+    if (pl.grid > 0) {
+        // without the memory for it there is no such plan
+        unsigned long long *slots = nullptr;
+        if (c->slot_row < REMC_MAX_MEMBERS && dalloc(&slots, (size_t)R * 2 * REMC_SLOT_K * REMC_MAX_MEMBERS) != hipSuccess)
+            pl.grid = 0;
+        else if (upload_wg(wg, &pl.wg) != hipSuccess)
+            pl.grid = 0;
+        if (pl.grid == 0) {
+            (void)hipGetLastError();
+            if (slots) (void)hipFree(slots);
+        } else if (slots) {
+            HIP_TRY(hipStreamSynchronize(c->stream));
+            HIP_TRY(hipFree(c->d_slots));
+            c->d_slots = slots;
+            c->slot_row = REMC_MAX_MEMBERS;
+        }
+    }
+    c->plans.push_back(pl);
+    *out = pl;
+    return REMC_OK;
+}
+
+// The plan of the context's MC configuration.
+int mc_plan(remc_ctx *c, remc_ctx::McPlan *out)
+{
+    return c->mc_balanced ? balanced_plan(c, c->mc_block, out) : uniform_plan(c, c->mc_coop, out);
+}
+
+int mc_launch(remc_ctx *c, const KParams &p0, int nsteps, int block, const remc_ctx::McPlan &pl)
+{
+    int rc = sync_members(c, pl);
     if (rc != REMC_OK) return rc;
     KParams p = p0;
-    fill_mc_lds(c, p, coop, block);
-    HIP_TRY(launch_mc(p, (int)c->reps.size(), nsteps, block, coop, c->stream));
-    c->synced_copies = coop;
+    p.slots = c->d_slots;
+    fill_mc_lds(c, p, pl, block);
+    HIP_TRY(launch_mc(p, pl.grid, pl.coop != 1, nsteps, block, c->stream));
+    if (c->synced != pl.wg) c->synced = nullptr; // the other members' copies are behind now
     return REMC_OK;
 }
 
@@ -824,8 +1010,6 @@ struct StateGuard {
     }
     int save()
     {
-        int rc = sync_copies(c, 1);
-        if (rc != REMC_OK) return rc;
         for (auto &b : bufs) {
             void *ptr = nullptr;
             HIP_TRY(hipMalloc(&ptr, b.bytes));
@@ -838,7 +1022,7 @@ struct StateGuard {
     {
         for (auto &b : bufs)
             if (b.save) HIP_TRY(hipMemcpyAsync(b.dev, b.save, b.bytes, hipMemcpyDeviceToDevice, c->stream));
-        c->synced_copies = 1;
+        c->synced = nullptr;
         return REMC_OK;
     }
     ~StateGuard()
@@ -863,44 +1047,67 @@ int autotune_mc(remc_ctx *c)
     const int blocks[3] = {256, 512, 1024};
     double best = 1e30;
     int best_block = 256, best_coop = 1;
+    bool best_balanced = false;
     const int trial_steps = 256;
+    // every trial starts from the same saved state, so each one makes the same moves;
+    // the best of two repeats discounts launch and clock noise
+    auto trial = [&](int blk, const remc_ctx::McPlan &pl, float *ms_best) -> int {
+        *ms_best = 1e30f;
+        for (int rep = 0; rep < 2; ++rep) {
+            c->synced = nullptr;
+            int rc = mc_launch(c, p, 4, blk, pl); // warm
+            if (rc != REMC_OK) return rc;
+            HIP_TRY(hipEventRecord(ev.a, c->stream));
+            rc = mc_launch(c, p, trial_steps, blk, pl);
+            if (rc != REMC_OK) return rc;
+            HIP_TRY(hipEventRecord(ev.b, c->stream));
+            HIP_TRY(hipEventSynchronize(ev.b));
+            rc = check_err(c);
+            if (rc != REMC_OK) return rc;
+            float ms = 0.f;
+            HIP_TRY(hipEventElapsedTime(&ms, ev.a, ev.b));
+            *ms_best = std::min(*ms_best, ms);
+            rc = st.restore();
+            if (rc != REMC_OK) return rc;
+        }
+        return REMC_OK;
+    };
     for (int bi = 0; bi < 3; ++bi) {
         const int blk = blocks[bi];
         if (c->mc_block && blk != c->mc_block) continue;
         int cmax = 1;
         rc = max_coop(c, blk, &cmax);
         if (rc != REMC_OK) return rc;
+        float ms = 0.f;
+        remc_ctx::McPlan pl;
         for (int coop = 1; coop <= cmax; coop *= 2) {
             if (c->mc_coop && coop != c->mc_coop) continue;
-            // every trial starts from the same saved state, so each one makes the same moves;
-            // the best of two repeats discounts launch and clock noise
-            float ms_best = 1e30f;
-            for (int rep = 0; rep < 2; ++rep) {
-                c->synced_copies = 1;
-                rc = mc_launch(c, p, 4, blk, coop); // warm
-                if (rc != REMC_OK) return rc;
-                HIP_TRY(hipEventRecord(ev.a, c->stream));
-                rc = mc_launch(c, p, trial_steps, blk, coop);
-                if (rc != REMC_OK) return rc;
-                HIP_TRY(hipEventRecord(ev.b, c->stream));
-                HIP_TRY(hipEventSynchronize(ev.b));
-                rc = check_err(c);
-                if (rc != REMC_OK) return rc;
-                float ms = 0.f;
-                HIP_TRY(hipEventElapsedTime(&ms, ev.a, ev.b));
-                ms_best = std::min(ms_best, ms);
-                rc = st.restore();
-                if (rc != REMC_OK) return rc;
-            }
-            if (ms_best < best) {
-                best = ms_best;
+            rc = uniform_plan(c, coop, &pl);
+            if (rc == REMC_OK) rc = trial(blk, pl, &ms);
+            if (rc != REMC_OK) return rc;
+            if (ms < best) {
+                best = ms;
                 best_block = blk;
                 best_coop = coop;
+                best_balanced = false;
             }
+        }
+        if (c->systems.size() < 2 || c->mc_coop) continue;
+        rc = balanced_plan(c, blk, &pl);
+        if (rc != REMC_OK) return rc;
+        if (pl.grid == 0) continue;
+        rc = trial(blk, pl, &ms);
+        if (rc != REMC_OK) return rc;
+        if (ms < best) {
+            best = ms;
+            best_block = blk;
+            best_coop = 1;
+            best_balanced = true;
         }
     }
     c->mc_block = best_block;
     c->mc_coop = best_coop;
+    c->mc_balanced = best_balanced;
     return REMC_OK;
 }
 
@@ -929,8 +1136,9 @@ int fb_prepare(remc_ctx *c, int block, KParams *out, int *coop_out)
     // as many as give every workgroup a CU of its own; never more than run
     // co-resident (the members of a replica wait for each other)
     const int R = (int)c->reps.size();
-    int coop = c->mc_coop > 0 ? c->mc_coop : REMC_MAX_COOP;
-    if (c->mc_coop <= 0)
+    const bool set = c->mc_coop > 0 && !c->mc_balanced;
+    int coop = set ? c->mc_coop : REMC_MAX_COOP;
+    if (!set)
         while (coop > 1 && (long long)R * coop > (long long)c->n_cu) coop >>= 1;
     if (coop > 1) {
         int per_cu = 0;
@@ -940,6 +1148,17 @@ int fb_prepare(remc_ctx *c, int block, KParams *out, int *coop_out)
     *out = p;
     *coop_out = coop;
     return REMC_OK;
+}
+
+// The force-biased kernel's members, like the MC kernel's with as many
+// workgroups for every replica, start from the same state.
+int fb_sync(remc_ctx *c, int coop)
+{
+    remc_ctx::McPlan pl;
+    int rc = uniform_plan(c, coop, &pl);
+    if (rc == REMC_OK) rc = sync_members(c, pl);
+    if (rc == REMC_OK && c->synced != pl.wg) c->synced = nullptr; // the launch leaves other members' copies behind
+    return rc;
 }
 
 // Workgroup size of the force-biased kernel: each of 256, 512 and 1024
@@ -965,7 +1184,7 @@ int autotune_fb(remc_ctx *c)
         p.rec = nullptr;
         float ms_best = 1e30f;
         for (int rep = 0; rep < 2; ++rep) {
-            rc = sync_copies(c, coop);
+            rc = fb_sync(c, coop);
             if (rc != REMC_OK) return rc;
             HIP_TRY(launch_mc_fb(p, R, 4, blocks[bi], coop, c->stream)); // warm
             HIP_TRY(hipEventRecord(ev.a, c->stream));
@@ -990,9 +1209,32 @@ int autotune_fb(remc_ctx *c)
     return REMC_OK;
 }
 
+// After a change of what the plans by cost are made from: they are made anew,
+// and a configuration that uses one is tuned again.
+void retune_balanced(remc_ctx *c)
+{
+    for (size_t k = 0; k < c->plans.size();) {
+        if (c->plans[k].coop != 0) {
+            ++k;
+            continue;
+        }
+        if (c->plans[k].wg) {
+            (void)hipStreamSynchronize(c->stream);
+            if (c->synced == c->plans[k].wg) c->synced = nullptr;
+            (void)hipFree(c->plans[k].wg);
+        }
+        c->plans.erase(c->plans.begin() + (long)k);
+    }
+    if (c->mc_balanced) {
+        c->mc_balanced = false;
+        c->mc_coop = 0;
+    }
+}
+
 int ensure_mc_config(remc_ctx *c)
 {
     if (c->mc_block == 0 || c->mc_coop == 0) return autotune_mc(c);
+    if (c->mc_balanced) return REMC_OK; // made to fit
     int cmax = 1;
     int rc = max_coop(c, c->mc_block, &cmax);
     if (rc != REMC_OK) return rc;
@@ -1165,6 +1407,8 @@ int remc_ctx_destroy(remc_ctx *c)
                     c->d_ana};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    for (const auto &pl : c->plans)
+        if (pl.wg) (void)hipFree(pl.wg);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
     for (auto e : c->free_events) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1390,11 +1634,13 @@ int remc_mc_steps(remc_ctx *c, int nsteps)
     if (nsteps == 0) return REMC_OK;
     int rc = ensure_mc_config(c);
     if (rc != REMC_OK) return rc;
-    rc = sync_copies(c, c->mc_coop);
+    remc_ctx::McPlan pl;
+    rc = mc_plan(c, &pl);
+    if (rc == REMC_OK) rc = sync_members(c, pl);
     if (rc != REMC_OK) return rc;
     {
         TimedLaunch t(c, 0);
-        rc = mc_launch(c, c->params(), nsteps, c->mc_block, c->mc_coop);
+        rc = mc_launch(c, c->params(), nsteps, c->mc_block, pl);
     }
     return rc;
 }
@@ -1419,14 +1665,12 @@ int remc_mc_steps_fb(remc_ctx *c, int nsteps, int block)
     int coop = 1;
     rc = fb_prepare(c, block, &p, &coop);
     if (rc != REMC_OK) return rc;
-    // every member starts from the same state
-    rc = sync_copies(c, coop);
+    rc = fb_sync(c, coop);
     if (rc != REMC_OK) return rc;
     {
         TimedLaunch t(c, 0);
         HIP_TRY(launch_mc_fb(p, (int)c->reps.size(), nsteps, block, coop, c->stream));
     }
-    c->synced_copies = coop;
     return REMC_OK;
 }
 
@@ -1528,7 +1772,7 @@ int remc_mc_steps_plain(remc_ctx *c, int replica, int nsteps, int block)
     HIP_TRY(hipMemcpyAsync(c->d_step + replica, &step, 8, hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync(c->d_cnt + 3 * replica, cnt, 24, hipMemcpyHostToDevice, st));
     HIP_TRY(hipStreamSynchronize(st));
-    c->synced_copies = 1;
+    c->synced = nullptr;
     return REMC_OK;
 }
 
@@ -1562,17 +1806,19 @@ int remc_run(remc_ctx *c, int rounds, int steps_per_round)
     if (rounds == 0) return REMC_OK;
     int rc = ensure_mc_config(c);
     if (rc != REMC_OK) return rc;
-    rc = sync_copies(c, c->mc_coop);
+    remc_ctx::McPlan pl;
+    rc = mc_plan(c, &pl);
+    if (rc == REMC_OK) rc = sync_members(c, pl);
     if (rc != REMC_OK) return rc;
     if (!c->graph || c->graph_steps != steps_per_round) {
         destroy_graph(c);
         KParams p = c->params();
-        fill_mc_lds(c, p, c->mc_coop, c->mc_block);
+        fill_mc_lds(c, p, pl, c->mc_block);
         int per_cu = 0; // also sets the kernel's dynamic-LDS attribute before capture
         HIP_TRY(mc_max_active_per_cu(p, c->mc_block, &per_cu));
         hipGraph_t g = nullptr;
         HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        hipError_t e1 = launch_mc(p, (int)c->reps.size(), steps_per_round, c->mc_block, c->mc_coop, c->stream);
+        hipError_t e1 = launch_mc(p, pl.grid, pl.coop != 1, steps_per_round, c->mc_block, c->stream);
         // with the refresh, the exchange reads full energies, as the reference's does
         if (e1 == hipSuccess && c->run_refresh)
             e1 = launch_energy_full(p, (int)c->reps.size(), c->max_beads, c->d_fix, c->d_full_partials, nullptr, 0, 1, c->stream);
@@ -1594,6 +1840,7 @@ int remc_run(remc_ctx *c, int rounds, int steps_per_round)
         TimedLaunch t(c, 0);
         HIP_TRY(hipGraphLaunch(c->graph, c->stream));
     }
+    if (c->synced != pl.wg) c->synced = nullptr; // the other members' copies are behind now
     return REMC_OK;
 }
 
@@ -1747,7 +1994,7 @@ int remc_set_state(remc_ctx *c, int replica, const float *x, const float *y, con
         if (src_m[i]) HIP_TRY(hipMemcpyAsync(dst_m[i] + mo, src_m[i], 4 * nm, hipMemcpyHostToDevice, st));
     if (quat) HIP_TRY(hipMemcpyAsync(c->d_quat + 4 * (size_t)mo, quat, 32 * nm, hipMemcpyHostToDevice, st));
     HIP_TRY(hipStreamSynchronize(st));
-    c->synced_copies = 1;
+    c->synced = nullptr;
     return REMC_OK;
 }
 
@@ -2045,6 +2292,7 @@ int remc_set_mc_block(remc_ctx *c, int block)
     if (block != 0 && block != 256 && block != 512 && block != 1024)
         return fail(REMC_ERR_ARG, "MC block must be 0, 256, 512 or 1024");
     c->mc_block = block;
+    retune_balanced(c);
     destroy_graph(c);
     return REMC_OK;
 }
@@ -2055,6 +2303,7 @@ int remc_set_mc_coop(remc_ctx *c, int coop)
     if (coop != 0 && coop != 1 && coop != 2 && coop != 4 && coop != 8)
         return fail(REMC_ERR_ARG, "workgroups per replica must be 0, 1, 2, 4 or 8");
     c->mc_coop = coop;
+    c->mc_balanced = false;
     destroy_graph(c);
     return REMC_OK;
 }
@@ -2073,6 +2322,7 @@ int remc_set_mc_tuning(remc_ctx *c, int lds_cache, int split_min_pairs)
     if (split_min_pairs < 0) return fail(REMC_ERR_ARG, "split threshold must be >= 0");
     c->lds_cache = lds_cache != 0;
     if (split_min_pairs > 0) c->coop_min_pairs = split_min_pairs;
+    retune_balanced(c);
     destroy_graph(c);
     return REMC_OK;
 }
@@ -2081,6 +2331,7 @@ int remc_set_mc_window(remc_ctx *c, int enable)
 {
     CHECK_CTX(c);
     c->mc_window = enable != 0;
+    retune_balanced(c);
     destroy_graph(c);
     return REMC_OK;
 }

@@ -53,6 +53,14 @@ struct DevFF {
     float crow_cut;  // crowder cutoff
 };
 
+// One workgroup of the MC kernel: member c of the coop workgroups of replica r
+// (r < 0: none), and where its copy of the replica's state begins in the dynamic
+// arrays (member 0's is the canonical one).
+struct McWg {
+    int r, c, coop, pad;
+    long long bead, body;
+};
+
 struct KParams {
     // static
     const int *tc;
@@ -87,7 +95,9 @@ struct KParams {
     int coop_min_pairs;     // moves with fewer pair terms are not split across members
     size_t copy_beads;      // stride between state copies (beads)
     size_t copy_bodies;     // stride between state copies (bodies)
-    unsigned long long *slots; // n_rep * REMC_SLOTS_PER_REP
+    unsigned long long *slots; // n_rep x 2 banks of REMC_SLOT_K x slot_row tagged partial sums
+    int slot_row;           // entries of a row: REMC_MAX_COOP, or REMC_MAX_MEMBERS where a replica has more members
+    const McWg *wg;         // the launch's workgroups
     int *err;               // set when a member waited too long
     // MC dynamic LDS: moved-body staging size and partner-bead/body caches
     int lds_mb;             // largest body (beads)
@@ -107,7 +117,10 @@ struct KParams {
 };
 
 // launchers (remc_kernels.hip)
-hipError_t launch_mc(const KParams &p, int n_rep, int nsteps, int block, int coop, hipStream_t s);
+// p.wg holds grid workgroups; shared: some replica has several members
+hipError_t launch_mc(const KParams &p, int grid, bool shared, int nsteps, int block, hipStream_t s);
+// copies every replica's canonical state to the copies of its other members
+hipError_t launch_copy_state(const KParams &p, int grid, hipStream_t s);
 size_t mc_dynamic_lds(const KParams &p);
 // static LDS of the MC kernel at this block size (its largest variant), or -1
 int mc_static_lds(int block);
@@ -173,10 +186,10 @@ constexpr int FULL_PER_MAX = 32;
 constexpr int FULL_WG = 2048;
 constexpr int SPEC_MAX = 16;     // largest body (beads) a speculative window slot takes
 static_assert(SPEC_MAX > 1, "a window slot's thread 1 forms its rotation");
-constexpr int REMC_MAX_COOP = 8; // workgroups per replica in the cooperative MC kernel
+constexpr int REMC_MAX_COOP = 8; // workgroups per replica where all replicas have as many
+constexpr int REMC_MAX_MEMBERS = 32; // workgroups of one replica where they follow its system's cost
 constexpr int REMC_SLOT_K = 64;  // partial sums per member and exchange (MC window slots, force-biased window values)
-// two banks of REMC_SLOT_K x REMC_MAX_COOP tagged partial sums per replica
-constexpr int REMC_SLOTS_PER_REP = 2 * REMC_SLOT_K * REMC_MAX_COOP;
+static_assert(REMC_MAX_MEMBERS <= 64 && REMC_MAX_MEMBERS % REMC_MAX_COOP == 0, "a lane per member, rows of whole polls");
 static_assert(REMC_SLOT_K >= 64, "every lane of a polling wave reads a slot row of its own");
 
 } // namespace remc

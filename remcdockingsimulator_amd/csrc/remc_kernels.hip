@@ -115,9 +115,10 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float v)
 // --------------------------------------------------------------------------
 // batched persistent MC
 //
-// Grid = coop * n_rep workgroups; workgroup b serves replica r = b % n_rep as
-// member c = b / n_rep of its cooperative group (so with n_rep a multiple of 8
-// the members of one replica share an XCD and its L2).  Member c keeps a
+// Workgroup b serves replica p.wg[b].r as member c of its coop members.  Where
+// all replicas have as many, b = c n_rep + r (so with n_rep a multiple of 8 the
+// members of one replica share an XCD and its L2); in a context of unequal
+// systems the members may follow the systems' cost (balanced_plan).  Member c keeps a
 // private copy c of the replica's dynamic state and evaluates dE over the
 // partner-bead slice [c*N/coop, (c+1)*N/coop).  Members publish their partial
 // dE per split step (per window: one per slot) in a 64-bit slot (value with
@@ -294,13 +295,12 @@ size_t mc_draw_batch_bytes() { return sizeof(StepDraw) * DRAW_BATCH; }
 // Decisions, energies and states are those of taking the steps one at a time,
 // up to the FP32 rounding of the reassociated pair sums.
 template <int BLOCK, bool CACHE, bool SPEC>
-__global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
+__global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
 {
     constexpr int NW = BLOCK / 64;
     constexpr int WK = SPEC ? 2 * NW : 1; // window slots: at most 32 (the slot masks are 32-bit)
     static_assert(WK <= 32 && WK <= REMC_SLOT_K, "window slots");
     constexpr int WS = SPEC ? WK * SPEC_MAX : 1;
-    __shared__ float s_etab[REMC_NTYPES * REMC_NTYPES];
     // (4 E_ij, and with p.sigtab the replica's system's sigma_ij^2 / box^2) per type pair
     __shared__ float2 s_et2[REMC_NTYPES * REMC_NTYPES];
     __shared__ double s_red[NW];
@@ -344,14 +344,14 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    const int r = blockIdx.x % p.n_rep;
-    const int c = blockIdx.x / p.n_rep;
+    const McWg W = p.wg[blockIdx.x];
+    if (W.r < 0) return; // the whole workgroup, before any barrier
+    const int r = W.r, c = W.c, coop = W.coop;
     const DevRep R = p.rep[r];
     const DevSys S = p.sys[R.sys];
     const DevFF ff = p.ff;
 
     for (int k = tid; k < REMC_NTYPES * REMC_NTYPES; k += BLOCK) {
-        s_etab[k] = p.etab[k];
         s_et2[k] = make_float2(p.etab[k], p.sigtab ? p.sstab[(size_t)2 * R.sys * (REMC_NTYPES * REMC_NTYPES) + k] : 0.0f);
     }
     if (tid == 0) s_abort = 0;
@@ -365,9 +365,8 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
     const double beta = remc_beta(p.T[r]);
     unsigned long long step = p.step[r];
 
-    // private copy c of this replica's dynamic state (always current in HBM)
-    const size_t cb = (size_t)c * p.copy_beads + R.bead_off;
-    const size_t cmo = (size_t)c * p.copy_bodies + R.body_off;
+    // member c's copy of this replica's dynamic state (always current in HBM)
+    const size_t cb = (size_t)W.bead, cmo = (size_t)W.body;
     float *gx = p.px + cb, *gy = p.py + cb, *gz = p.pz + cb;
     float *grx = p.rx + cb, *gry = p.ry + cb, *grz = p.rz + cb;
     float *gcx = p.cx + cmo, *gcy = p.cy + cmo, *gcz = p.cz + cmo;
@@ -376,7 +375,8 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
     const float *qs = p.q + S.bead_off, *sgs = p.sig + S.bead_off;
     const int N = S.n_beads;
     const int cjs = (int)(((long long)c * N) / coop), cje = (int)(((long long)(c + 1) * N) / coop);
-    unsigned long long *slots = p.slots + (size_t)r * REMC_SLOTS_PER_REP;
+    const int row = p.slot_row;
+    unsigned long long *slots = p.slots + (size_t)r * (2 * REMC_SLOT_K) * row;
     unsigned int n_x = 0; // partial-sum exchanges so far in this launch: selects the slot bank
 
     // cached partner beads: all of them, or only this member's slice when
@@ -706,7 +706,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
             // partner slice, the members' partials then exchanged once for the
             // whole window
             const unsigned long long wtag = step & 0x7FFFFull;
-            unsigned long long *bank = slots + (n_x & 1u) * (REMC_SLOT_K * REMC_MAX_COOP);
+            unsigned long long *bank = slots + (n_x & 1u) * (REMC_SLOT_K * row);
             const int wjs = coop > 1 ? cjs : 0, wje = coop > 1 ? cje : N;
             // Static slots: a one-bead body whose move leaves its position as it
             // is (the rotation of a sphere) has dE = 0 exactly, with no partner
@@ -730,8 +730,8 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                 const float lim2a = crowder_screen2(oa, na, S, ff), lim2b = crowder_screen2(ob, nb, S, ff);
                 float acc_a = 0.0f, comp_a = 0.0f, acc_b = 0.0f, comp_b = 0.0f;
                 for (int j = wjs + lane; j < wje; j += 64) {
-                    const int jc = j - clo;
-                    const float xj = s_jx[jc], yj = s_jy[jc], zj = s_jz[jc];
+                    const float xj = CACHE ? s_jx[j - clo] : gx[j], yj = CACHE ? s_jy[j - clo] : gy[j],
+                                zj = CACHE ? s_jz[j - clo] : gz[j];
                     // the terms at the new positions only where a partner of the
                     // wave is near enough to give any (crowders are sparse)
                     const float r2a = dist2(xj, yj, zj, oa, S), r2b = dist2(xj, yj, zj, ob, S);
@@ -751,9 +751,9 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                 const double vb = wave_sum_dpp((double)acc_b - (double)comp_b);
                 if (lane == 0) {
                     if (coop > 1) {
-                        __hip_atomic_store(bank + ka * REMC_MAX_COOP + c, slot_pack(va, wtag), __ATOMIC_RELAXED,
+                        __hip_atomic_store(bank + ka * row + c, slot_pack(va, wtag), __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
-                        __hip_atomic_store(bank + kb * REMC_MAX_COOP + c, slot_pack(vb, wtag), __ATOMIC_RELAXED,
+                        __hip_atomic_store(bank + kb * row + c, slot_pack(vb, wtag), __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
                     } else {
                         s_wbase[ka] = va;
@@ -773,8 +773,8 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                     const float4 o = s_wold[k * SPEC_MAX], n = s_wnew[k * SPEC_MAX];
                     const float lim2 = crowder_screen2(o, n, S, ff);
                     for (int j = wjs + lane; j < wje; j += 64) {
-                        const int jc = j - clo;
-                        const float xj = s_jx[jc], yj = s_jy[jc], zj = s_jz[jc];
+                        const float xj = CACHE ? s_jx[j - clo] : gx[j], yj = CACHE ? s_jy[j - clo] : gy[j],
+                                    zj = CACHE ? s_jz[j - clo] : gz[j];
                         const float r2o = dist2(xj, yj, zj, o, S);
                         if (!__any(j != m0k && r2o < lim2)) continue;
                         if (j != m0k) {
@@ -786,21 +786,21 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                 }
                 for (int i = 0; i < (nmk == 1 && crow_m ? 0 : nmk); ++i) {
                     const float4 o = s_wold[k * SPEC_MAX + i], n = s_wnew[k * SPEC_MAX + i];
-                    const float *erow = s_etab + (s_wtc[k * SPEC_MAX + i] & 0xff) * REMC_NTYPES;
+                    const float2 *erow = s_et2 + (s_wtc[k * SPEC_MAX + i] & 0xff) * REMC_NTYPES;
                     for (int j = wjs + lane; j < wje; j += 64) {
                         if (j >= m0k && j < m1k) continue;
-                        const int jc = j - clo; // the partner range lies in the cache
-                        const float xj = s_jx[jc], yj = s_jy[jc], zj = s_jz[jc];
-                        const int tcj = s_jtc[jc];
+                        const int jc = j - clo; // with the cache the partner range lies in it
+                        const float xj = CACHE ? s_jx[jc] : gx[j], yj = CACHE ? s_jy[jc] : gy[j], zj = CACHE ? s_jz[jc] : gz[j];
+                        const int tcj = CACHE ? s_jtc[jc] : tcs[j];
                         float eo, en;
                         if (crow_m || (tcj >> 8) != 0) {
                             eo = pair_crowder(dist2(xj, yj, zj, o, S), ff);
                             en = pair_crowder(dist2(xj, yj, zj, n, S), ff);
                         } else {
-                            const float eij = erow[tcj & 0xff];
-                            const float sij = 0.5f * (n.w + s_js[jc]);
+                            const float eij = erow[tcj & 0xff].x;
+                            const float sij = 0.5f * (n.w + (CACHE ? s_js[jc] : sgs[j]));
                             const float sij2 = sij * sij;
-                            const float qq = o.w * s_jq[jc];
+                            const float qq = o.w * (CACHE ? s_jq[jc] : qs[j]);
                             eo = pair_lj_dh(dist2(xj, yj, zj, o, S), eij, sij2, qq, ff);
                             en = pair_lj_dh(dist2(xj, yj, zj, n, S), eij, sij2, qq, ff);
                         }
@@ -810,7 +810,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                 const double v = wave_sum_dpp((double)acc - (double)comp);
                 if (lane == 0) {
                     if (coop > 1)
-                        __hip_atomic_store(bank + k * REMC_MAX_COOP + c, slot_pack(v, wtag), __ATOMIC_RELAXED,
+                        __hip_atomic_store(bank + k * row + c, slot_pack(v, wtag), __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
                     else
                         s_wbase[k] = v;
@@ -843,7 +843,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                                     e_oo = pair_crowder(dist2(O.x, O.y, O.z, o, S), ff);
                                 } else {
                                     const int sl = jj * SPEC_MAX + l;
-                                    const float eij = s_etab[ti * REMC_NTYPES + (s_wtc[sl] & 0xff)];
+                                    const float eij = s_et2[ti * REMC_NTYPES + (s_wtc[sl] & 0xff)].x;
                                     const float sij = 0.5f * (n.w + Nn.w);
                                     const float sij2 = sij * sij;
                                     const float qq = o.w * s_wrel[sl].w;
@@ -910,32 +910,37 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                 if (coop > 1) {
                     // lane k gathers slot k's coop partials (bank[k][m]) and adds
                     // them in member order: the same total in every member
-                    // Every lane reads all REMC_MAX_COOP entries of its slot row
-                    // (the row exists for every lane: REMC_SLOT_K >= 64) with no
-                    // branch between the loads, so a poll costs one memory round
-                    // trip, not one per member.
-                    unsigned long long v[REMC_MAX_COOP];
-                    int spins = 0;
+                    // Every lane reads REMC_MAX_COOP entries of its slot row at a
+                    // time (the row exists for every lane: REMC_SLOT_K >= 64) with
+                    // no branch between the loads, so a poll costs one memory
+                    // round trip, not one per member.
                     bool failed = false;
-                    for (;;) {
+                    for (int m0 = 0; m0 < coop && !failed; m0 += REMC_MAX_COOP) {
+                        unsigned long long v[REMC_MAX_COOP];
+                        int spins = 0;
+                        for (;;) {
+#pragma unroll
+                            for (int m = 0; m < REMC_MAX_COOP; ++m)
+                                v[m] = __hip_atomic_load(bank + lane * row + m0 + m, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT);
+                            bool mine = true;
+#pragma unroll
+                            for (int m = 0; m < REMC_MAX_COOP; ++m)
+                                mine = mine && (m0 + m >= coop || (v[m] & SLOT_TAG_MASK) == wtag);
+                            if (__all(mine || lane >= w || st_l)) break;
+                            if (++spins >= SLOT_SPIN_LIMIT) {
+                                failed = true;
+                                break;
+                            }
+                            if ((spins & 255) == 0 && __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                                failed = true;
+                                break;
+                            }
+                            __builtin_amdgcn_s_sleep(1);
+                        }
 #pragma unroll
                         for (int m = 0; m < REMC_MAX_COOP; ++m)
-                            v[m] = __hip_atomic_load(bank + lane * REMC_MAX_COOP + m, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
-                        bool mine = true;
-#pragma unroll
-                        for (int m = 0; m < REMC_MAX_COOP; ++m)
-                            mine = mine && (m >= coop || (v[m] & SLOT_TAG_MASK) == wtag);
-                        if (__all(mine || lane >= w || st_l)) break;
-                        if (++spins >= SLOT_SPIN_LIMIT) {
-                            failed = true;
-                            break;
-                        }
-                        if ((spins & 255) == 0 && __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                            failed = true;
-                            break;
-                        }
-                        __builtin_amdgcn_s_sleep(1);
+                            if (m0 + m < coop) dEl += slot_value(v[m]);
                     }
                     if (failed) {
                         if (lane == 0) {
@@ -943,9 +948,6 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                             s_abort = 1;
                         }
                     }
-#pragma unroll
-                    for (int m = 0; m < REMC_MAX_COOP; ++m)
-                        if (m < coop) dEl += slot_value(v[m]);
                     if (lane >= w || st_l) dEl = 0.0;
                 } else {
                     dEl = lane < w && !st_l ? s_wbase[lane] : 0.0;
@@ -1266,7 +1268,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                         eo = pair_crowder(dist2(xj[u], yj[u], zj[u], o, S), ff);
                         en = pair_crowder(dist2(xj[u], yj[u], zj[u], n, S), ff);
                     } else {
-                        const float eij = s_etab[ti * REMC_NTYPES + (tcj[u] & 0xff)];
+                        const float eij = s_et2[ti * REMC_NTYPES + (tcj[u] & 0xff)].x;
                         const float sij = 0.5f * (n.w + sj[u]);
                         const float sij2 = sij * sij;
                         const float qq = o.w * qj[u];
@@ -1322,7 +1324,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps, int coop)
                 // slot only after every member has read it (they all wrote
                 // their partial of the split step in between)
                 const unsigned long long tag = step & 0x7FFFFull;
-                unsigned long long *slot = slots + (n_x & 1u) * (REMC_SLOT_K * REMC_MAX_COOP);
+                unsigned long long *slot = slots + (n_x & 1u) * (REMC_SLOT_K * row);
                 if (lane == 0) __hip_atomic_store(slot + c, slot_pack(part, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 unsigned long long wv = 0ull;
                 bool ok = lane >= coop;
@@ -1458,14 +1460,45 @@ __global__ void k_reset_slots(unsigned long long *slots, int n)
     if (i < n) slots[i] = ~0ull;
 }
 
+// The canonical state of each replica to the copies of its other members.
+__global__ __launch_bounds__(256) void k_copy_state(KParams p)
+{
+    const McWg W = p.wg[blockIdx.x];
+    if (W.r < 0 || W.c == 0) return;
+    const DevRep R = p.rep[W.r];
+    const DevSys S = p.sys[R.sys];
+    for (int b = threadIdx.x; b < S.n_beads; b += 256) {
+        const long long i = R.bead_off + b, o = W.bead + b;
+        p.px[o] = p.px[i];
+        p.py[o] = p.py[i];
+        p.pz[o] = p.pz[i];
+        p.rx[o] = p.rx[i];
+        p.ry[o] = p.ry[i];
+        p.rz[o] = p.rz[i];
+    }
+    for (int m = threadIdx.x; m < S.n_bodies; m += 256) {
+        const long long i = R.body_off + m, o = W.body + m;
+        p.cx[o] = p.cx[i];
+        p.cy[o] = p.cy[i];
+        p.cz[o] = p.cz[i];
+    }
+    for (int m = threadIdx.x; m < 4 * S.n_bodies; m += 256) p.quat[4 * W.body + m] = p.quat[4 * (long long)R.body_off + m];
+}
+
+hipError_t launch_copy_state(const KParams &p, int grid, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_copy_state, dim3(grid), dim3(256), 0, s, p);
+    return hipGetLastError();
+}
+
 template <int BLOCK, bool CACHE, bool SPEC>
-static hipError_t launch_mc_t(const KParams &p, int grid, int nsteps, int coop, hipStream_t s)
+static hipError_t launch_mc_t(const KParams &p, int grid, int nsteps, hipStream_t s)
 {
     const size_t lds = mc_dynamic_lds(p);
     hipError_t e = hipFuncSetAttribute((const void *)k_mc<BLOCK, CACHE, SPEC>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_mc<BLOCK, CACHE, SPEC>), dim3(grid), dim3(BLOCK), lds, s, p, nsteps, coop);
+    hipLaunchKernelGGL((k_mc<BLOCK, CACHE, SPEC>), dim3(grid), dim3(BLOCK), lds, s, p, nsteps);
     return hipGetLastError();
 }
 
@@ -1590,7 +1623,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc_fb(KParams p, int nsteps, int coop
     const float *qs = p.q + S.bead_off, *sgs = p.sig + S.bead_off;
     const int N = S.n_beads;
     const int cjs = (int)(((long long)c * N) / coop), cje = (int)(((long long)(c + 1) * N) / coop);
-    unsigned long long *slots = p.slots + (size_t)r * REMC_SLOTS_PER_REP;
+    unsigned long long *slots = p.slots + (size_t)r * (2 * REMC_SLOT_K * REMC_MAX_COOP);
     unsigned int n_x = 0; // exchanges so far in this launch: selects the slot bank
     if (cached)
         for (int b = tid; b < N; b += BLOCK) {
@@ -2402,7 +2435,7 @@ hipError_t launch_mc_fb(const KParams &p, int n_rep, int nsteps, int block, int 
     if (n_rep <= 0 || nsteps <= 0) return hipSuccess;
     if (coop < 1 || coop > REMC_MAX_COOP) return hipErrorInvalidValue;
     if (coop > 1) {
-        const int n = n_rep * REMC_SLOTS_PER_REP;
+        const int n = n_rep * (2 * REMC_SLOT_K * REMC_MAX_COOP);
         hipLaunchKernelGGL(k_reset_slots, dim3((n + 255) / 256), dim3(256), 0, s, p.slots, n);
     }
     switch (block) {
@@ -2413,35 +2446,31 @@ hipError_t launch_mc_fb(const KParams &p, int n_rep, int nsteps, int block, int 
     }
 }
 
-// kernel variant: 0 = no partner cache, 1 = partner cache, 2 = speculative windows
-static int mc_variant(const KParams &p) { return p.lds_cl <= 0 ? 0 : p.spec ? 2 : 1; }
+// kernel variant: partner cache (bit 0), speculative windows (bit 1)
+static int mc_variant(const KParams &p) { return (p.lds_cl > 0 ? 1 : 0) | (p.spec ? 2 : 0); }
 
 template <int BLOCK>
-static hipError_t launch_mc_b(const KParams &p, int grid, int nsteps, int coop, hipStream_t s)
+static hipError_t launch_mc_b(const KParams &p, int grid, int nsteps, hipStream_t s)
 {
     switch (mc_variant(p)) {
-    case 0: return launch_mc_t<BLOCK, false, false>(p, grid, nsteps, coop, s);
-    case 1: return launch_mc_t<BLOCK, true, false>(p, grid, nsteps, coop, s);
-    default: return launch_mc_t<BLOCK, true, true>(p, grid, nsteps, coop, s);
+    case 0: return launch_mc_t<BLOCK, false, false>(p, grid, nsteps, s);
+    case 1: return launch_mc_t<BLOCK, true, false>(p, grid, nsteps, s);
+    case 2: return launch_mc_t<BLOCK, false, true>(p, grid, nsteps, s);
+    default: return launch_mc_t<BLOCK, true, true>(p, grid, nsteps, s);
     }
 }
 
-hipError_t launch_mc(const KParams &p, int n_rep, int nsteps, int block, int coop, hipStream_t s)
+hipError_t launch_mc(const KParams &p, int grid, bool shared, int nsteps, int block, hipStream_t s)
 {
-    if (n_rep <= 0 || nsteps <= 0) return hipSuccess;
-    if (coop < 1 || coop > REMC_MAX_COOP) return hipErrorInvalidValue;
-    // the speculative kernel reads its partner range from the cache (the whole replica, or with
-    // every member on its own slice the member's slice)
-    if (p.spec && p.lds_cl <= 0) return hipErrorInvalidValue;
-    if (coop > 1) {
-        const int n = n_rep * REMC_SLOTS_PER_REP;
+    if (grid <= 0 || nsteps <= 0) return hipSuccess;
+    if (shared) {
+        const int n = p.n_rep * (2 * REMC_SLOT_K) * p.slot_row;
         hipLaunchKernelGGL(k_reset_slots, dim3((n + 255) / 256), dim3(256), 0, s, p.slots, n);
     }
-    const int grid = n_rep * coop;
     switch (block) {
-    case 256: return launch_mc_b<256>(p, grid, nsteps, coop, s);
-    case 512: return launch_mc_b<512>(p, grid, nsteps, coop, s);
-    case 1024: return launch_mc_b<1024>(p, grid, nsteps, coop, s);
+    case 256: return launch_mc_b<256>(p, grid, nsteps, s);
+    case 512: return launch_mc_b<512>(p, grid, nsteps, s);
+    case 1024: return launch_mc_b<1024>(p, grid, nsteps, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -2462,6 +2491,7 @@ static hipError_t occupancy_b(const KParams &p, int *out)
     switch (mc_variant(p)) {
     case 0: return occupancy_t<BLOCK, false, false>(p, out);
     case 1: return occupancy_t<BLOCK, true, false>(p, out);
+    case 2: return occupancy_t<BLOCK, false, true>(p, out);
     default: return occupancy_t<BLOCK, true, true>(p, out);
     }
 }
