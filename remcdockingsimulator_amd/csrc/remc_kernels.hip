@@ -531,11 +531,61 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
         // Staging of a large move (draws Dm) into s_old / s_new, their
         // box-scaled copies and s_tc, by threads t0, t0 + stride, ... over its
         // beads.  It reads only the moved body.
-        auto stage_move = [&](const int t0, const int stride, const StepDraw &Dm) {
-            // the bead range comes with the draw: the centre and the beads'
-            // reads wait on the draw only
-            const int bd = Dm.body, mb0 = Dm.m0, mb1 = Dm.m0 + Dm.nm;
-            float bcx, bcy, bcz;
+        auto stage_move = [&](const int t0, const int stride, const StepDraw &Dm, const float bcx, const float bcy,
+                              const float bcz, const float nbx, const float nby, const float nbz) {
+            const int mb0 = Dm.m0, mb1 = Dm.m0 + Dm.nm;
+            for (int k = t0; k < mb1 - mb0; k += stride) {
+                const int b = mb0 + k;
+                float rx, ry, rz, ox, oy, oz, ob, sb;
+                int tb;
+                if (cache_rel) { // then every bead is cached: the reads go out together
+                    rx = lds_ld(s_rx + b);
+                    ry = lds_ld(s_ry + b);
+                    rz = lds_ld(s_rz + b);
+                    ox = lds_ld(s_jx + b);
+                    oy = lds_ld(s_jy + b);
+                    oz = lds_ld(s_jz + b);
+                    ob = lds_ld(s_jq + b);
+                    sb = lds_ld(s_js + b);
+                    tb = lds_ld(s_jtc + b);
+                } else {
+                    rx = grx[b];
+                    ry = gry[b];
+                    rz = grz[b];
+                    if (CACHE && b >= clo && b < chi) {
+                        const int kb = b - clo;
+                        ox = lds_ld(s_jx + kb);
+                        oy = lds_ld(s_jy + kb);
+                        oz = lds_ld(s_jz + kb);
+                        ob = lds_ld(s_jq + kb);
+                        sb = lds_ld(s_js + kb);
+                        tb = lds_ld(s_jtc + kb);
+                    } else {
+                        ox = gx[b];
+                        oy = gy[b];
+                        oz = gz[b];
+                        ob = qs[b];
+                        sb = sgs[b];
+                        tb = tcs[b];
+                    }
+                }
+                float nrx = rx, nry = ry, nrz = rz;
+                if (Dm.rotate) remc_qrotate(Dm.coef, rx, ry, rz, &nrx, &nry, &nrz);
+                const float4 ov = make_float4(ox, oy, oz, ob * ff.c_dh);
+                const float4 nv = make_float4(nrx + nbx, nry + nby, nrz + nbz, sb);
+                s_old[k] = ov;
+                s_new[k] = nv;
+                // box-scaled about the body's old centre: the beads near it, which
+                // give the steep contact terms, keep every bit of their offsets
+                const float ib = S.inv_box;
+                s_olds[k] = make_float4((ov.x - bcx) * ib, (ov.y - bcy) * ib, (ov.z - bcz) * ib, ov.w * ib);
+                s_news[k] = make_float4((nv.x - bcx) * ib, (nv.y - bcy) * ib, (nv.z - bcz) * ib, 0.5f * nv.w);
+                s_tc[k] = tb;
+            }
+        };
+        // A body's centre and, for a translation, its new one.
+        auto centres = [&](const StepDraw &Dm, float &bcx, float &bcy, float &bcz, float &nbx, float &nby, float &nbz) {
+            const int bd = Dm.body;
             if (cache_bodies) {
                 bcx = lds_ld(s_cx + bd);
                 bcy = lds_ld(s_cy + bd);
@@ -545,41 +595,10 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                 bcy = gcy[bd];
                 bcz = gcz[bd];
             }
-            float nbx = bcx, nby = bcy, nbz = bcz;
+            nbx = bcx;
+            nby = bcy;
+            nbz = bcz;
             if (!Dm.rotate) remc_wrap_centre(bcx, bcy, bcz, Dm.t[0], Dm.t[1], Dm.t[2], S.box, &nbx, &nby, &nbz);
-            for (int k = t0; k < mb1 - mb0; k += stride) {
-                const int b = mb0 + k;
-                const bool inc = CACHE && b >= clo && b < chi;
-                float rx, ry, rz;
-                if (cache_rel) {
-                    rx = lds_ld(s_rx + b);
-                    ry = lds_ld(s_ry + b);
-                    rz = lds_ld(s_rz + b);
-                } else {
-                    rx = grx[b];
-                    ry = gry[b];
-                    rz = grz[b];
-                }
-                float nrx = rx, nry = ry, nrz = rz;
-                if (Dm.rotate) remc_qrotate(Dm.coef, rx, ry, rz, &nrx, &nry, &nrz);
-                float4 ov, nv;
-                if (inc) {
-                    const int kb = b - clo;
-                    ov = make_float4(lds_ld(s_jx + kb), lds_ld(s_jy + kb), lds_ld(s_jz + kb), lds_ld(s_jq + kb) * ff.c_dh);
-                    nv = make_float4(nrx + nbx, nry + nby, nrz + nbz, lds_ld(s_js + kb));
-                } else {
-                    ov = make_float4(gx[b], gy[b], gz[b], qs[b] * ff.c_dh);
-                    nv = make_float4(nrx + nbx, nry + nby, nrz + nbz, sgs[b]);
-                }
-                s_old[k] = ov;
-                s_new[k] = nv;
-                // box-scaled about the body's old centre: the beads near it, which
-                // give the steep contact terms, keep every bit of their offsets
-                const float ib = S.inv_box;
-                s_olds[k] = make_float4((ov.x - bcx) * ib, (ov.y - bcy) * ib, (ov.z - bcz) * ib, ov.w * ib);
-                s_news[k] = make_float4((nv.x - bcx) * ib, (nv.y - bcy) * ib, (nv.z - bcz) * ib, 0.5f * nv.w);
-                s_tc[k] = inc ? lds_ld(s_jtc + (b - clo)) : tcs[b];
-            }
         };
         // Staging of a speculative window's slots [0, wn) from step off_ of
         // the draw batch sd, one thread st per slot bead (slot st / SPEC_MAX,
@@ -869,7 +888,11 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
             // the window moves, so the staging holds whatever the decisions.
             const int nxo = off + w;
             const bool nx_big = w < WK && nxo < have && it + w < nsteps && ((elig >> nxo) & 1ull) == 0ull;
-            if (wave != 0 && nx_big) stage_move(tid - 64, BLOCK - 64, s_draw[nxo]);
+            if (wave != 0 && nx_big) {
+                float bx, by, bz, nx, ny, nz;
+                centres(s_draw[nxo], bx, by, bz, nx, ny, nz);
+                stage_move(tid - 64, BLOCK - 64, s_draw[nxo], bx, by, bz, nx, ny, nz);
+            }
             if (nx_big) pre_it = it + w;
 
             // The commit's data (everything but the decisions) is read into
@@ -1072,22 +1095,12 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
         const int body = D.body;
         const bool rotate = D.rotate != 0;
         const int m0 = D.m0, m1 = D.m0 + D.nm; // the bead range formed with the draw
-        float cx, cy, cz;
-        if (cache_bodies) {
-            cx = lds_ld(s_cx + body);
-            cy = lds_ld(s_cy + body);
-            cz = lds_ld(s_cz + body);
-        } else {
-            cx = gcx[body];
-            cy = gcy[body];
-            cz = gcz[body];
-        }
+        float cx, cy, cz, ncx, ncy, ncz;
+        centres(D, cx, cy, cz, ncx, ncy, ncz);
         const int nm = m1 - m0;
         const bool crow_m = (CACHE && m0 >= clo && m0 < chi) ? (s_jtc[m0 - clo] >> 8) != 0
                                                              : p.bcrow[S.body_off + body] != 0;
-        float ncx = cx, ncy = cy, ncz = cz;
-        if (!rotate) remc_wrap_centre(cx, cy, cz, D.t[0], D.t[1], D.t[2], S.box, &ncx, &ncy, &ncz);
-        if (!pre_mv) stage_move(tid, BLOCK, D);
+        if (!pre_mv) stage_move(tid, BLOCK, D, cx, cy, cz, ncx, ncy, ncz);
         __syncthreads();
 
         // Moves with few pair terms are evaluated whole by every member (no
@@ -1400,7 +1413,9 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                     }
                 }
             }
-            if (tid == 0) {
+            // (a wave of its own for the body's rotation or centre, and one for the
+            // tallies below: a body of up to 128 beads leaves these idle here)
+            if (tid == 192) {
                 if (rotate) {
                     double qo[4], qn[4];
                     if (cache_quat)
@@ -1424,7 +1439,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                 }
             }
         }
-        if (tid == 0) {
+        if (tid == 128) {
             if (decision) s_E += dE;
             ++s_cnt[decision == 1 ? 0 : decision == 2 ? 1 : 2];
         }
