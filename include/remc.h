@@ -211,6 +211,9 @@ REMC_API int remc_get_ladder(remc_ctx *ctx, int sys_id, int *slot_replica);
  * its body count, quat 4 per body.  Any pointer may be NULL on get. */
 REMC_API int remc_get_state(remc_ctx *ctx, int replica, float *x, float *y, float *z,
                    float *rx, float *ry, float *rz, float *cx, float *cy, float *cz, double *quat);
+/* The same conformation as rows of three: pos and rel n_beads x 3, centre
+ * n_bodies x 3, quat n_bodies x 4; no pointer may be NULL. */
+REMC_API int remc_get_state_rows(remc_ctx *ctx, int replica, float *pos, float *rel, float *centre, double *quat);
 REMC_API int remc_set_state(remc_ctx *ctx, int replica, const float *x, const float *y, const float *z,
                    const float *rx, const float *ry, const float *rz,
                    const float *cx, const float *cy, const float *cz, const double *quat);

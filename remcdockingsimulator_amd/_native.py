@@ -75,6 +75,7 @@ SIGNATURES = {
     "remc_get_temperatures": (ctypes.c_int, [_vp, _dp]),
     "remc_get_counters": (ctypes.c_int, [_vp, ctypes.POINTER(remc_counters)]),
     "remc_get_ladder": (ctypes.c_int, [_vp, ctypes.c_int, _ip]),
+    "remc_get_state_rows": (ctypes.c_int, [_vp, ctypes.c_int] + [_vp] * 4),  # float* x 3, double*
     "remc_get_state": (ctypes.c_int, [_vp, ctypes.c_int] + [_vp] * 10),  # float* x 9, double*
     "remc_set_state": (ctypes.c_int, [_vp, ctypes.c_int] + [_fp] * 9 + [_dp]),
     "remc_set_energies": (ctypes.c_int, [_vp, _dp]),

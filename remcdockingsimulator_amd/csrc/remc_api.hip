@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -154,6 +156,8 @@ struct remc_ctx {
     int *d_err = nullptr;
     uint32_t *h_pin = nullptr; // pinned host memory that read-backs go through (ReadBack)
     size_t pin_words = 0;
+    uint32_t *h_flag = nullptr, *d_count = nullptr; // Signal of the read-backs, and their number
+    uint32_t ticket = 0;
     double *d_adj = nullptr; // adjoint scratch: bead gradients, tile partials, body forces, parameter gradients
     size_t adj_cap = 0;      // doubles held by d_adj
     int adj_target = 0;      // all-replica adjoint's workgroup target (0: tune on first use)
@@ -528,6 +532,9 @@ int finalize(remc_ctx *c)
     HIP_TRY(dalloc(&c->d_slots, (size_t)R * 2 * REMC_SLOT_K * REMC_MAX_COOP));
     c->slot_row = REMC_MAX_COOP;
     HIP_TRY(dalloc(&c->d_err, (size_t)1));
+    HIP_TRY(dalloc(&c->d_count, (size_t)1));
+    HIP_TRY(hipHostMalloc((void **)&c->h_flag, sizeof(uint32_t), hipHostMallocDefault));
+    *c->h_flag = 0;
     HIP_TRY(dalloc(&c->d_E, (size_t)R));
     HIP_TRY(dalloc(&c->d_T, (size_t)R));
     HIP_TRY(dalloc(&c->d_step, (size_t)R));
@@ -580,6 +587,7 @@ int finalize(remc_ctx *c)
     {
         int zero = 0;
         HIP_TRY(hipMemcpyAsync(c->d_err, &zero, sizeof(int), hipMemcpyHostToDevice, s));
+        HIP_TRY(hipMemcpyAsync(c->d_count, &zero, sizeof(int), hipMemcpyHostToDevice, s));
     }
     hipDeviceProp_t prop;
     HIP_TRY(hipGetDeviceProperties(&prop, c->device));
@@ -680,6 +688,28 @@ int sync_members(remc_ctx *c, const remc_ctx::McPlan &pl)
     return REMC_OK;
 }
 
+Signal next_signal(remc_ctx *c) { return Signal{c->d_count, c->h_flag, ++c->ticket}; }
+
+// Waits for the read-back launched last, and with it for the stream: for its
+// flag while the wait is as long as a read-back alone (the stream's own end
+// comes several us after the kernel's last store), then for the stream.
+int wait_signal(remc_ctx *c)
+{
+    const auto t0 = std::chrono::steady_clock::now();
+    const volatile uint32_t *flag = c->h_flag;
+    do {
+        for (int k = 0; k < 64; ++k) {
+            if (*flag == c->ticket) {
+                std::atomic_thread_fence(std::memory_order_acquire);
+                return REMC_OK;
+            }
+            __builtin_ia32_pause();
+        }
+    } while (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(100));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return REMC_OK;
+}
+
 // Device arrays read back together: add() each (a null destination is left
 // out), then run() packs them into the context's pinned memory by one launch,
 // waits once and copies them out.
@@ -700,8 +730,13 @@ struct ReadBack {
     int run()
     {
         if (g.at[g.n] > c->pin_words) return fail(REMC_ERR_STATE, "read-back of %u words exceeds its buffer", g.at[g.n]);
-        HIP_TRY(launch_gather(g, c->h_pin, c->stream));
-        HIP_TRY(hipStreamSynchronize(c->stream));
+        if (g.at[g.n] == 0) { // nothing asked for: the wait alone
+            HIP_TRY(hipStreamSynchronize(c->stream));
+            return REMC_OK;
+        }
+        HIP_TRY(launch_gather(g, c->h_pin, next_signal(c), c->stream));
+        const int rc = wait_signal(c);
+        if (rc != REMC_OK) return rc;
         for (int k = 0; k < g.n; ++k) std::memcpy(out[k], c->h_pin + g.at[k], 4 * (size_t)(g.at[k + 1] - g.at[k]));
         return REMC_OK;
     }
@@ -1403,13 +1438,14 @@ int remc_ctx_destroy(remc_ctx *c)
                     c->d_sys, c->d_rep, c->d_px, c->d_py, c->d_pz, c->d_rx, c->d_ry, c->d_rz,
                     c->d_cx, c->d_cy, c->d_cz, c->d_quat, c->d_E, c->d_T, c->d_step, c->d_cnt,
                     c->d_slot, c->d_exoff, c->d_ladder, c->d_exround, c->d_exswaps, c->d_full_partials,
-                    c->d_fix, c->d_grp, c->d_border, c->d_plain_partials, c->d_rec, c->d_rec_start, c->d_slots, c->d_err, c->d_adj,
+                    c->d_fix, c->d_grp, c->d_border, c->d_plain_partials, c->d_rec, c->d_rec_start, c->d_slots, c->d_err, c->d_count, c->d_adj,
                     c->d_ana};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (const auto &pl : c->plans)
         if (pl.wg) (void)hipFree(pl.wg);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
+    if (c->h_flag) (void)hipHostFree(c->h_flag);
     for (auto e : c->free_events) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1959,6 +1995,32 @@ int remc_get_state(remc_ctx *c, int replica, float *x, float *y, float *z, float
     for (int i = 0; i < 3; ++i) rb.add(dst_m[i], src_m[i] + mo, nm);
     rb.add(quat, c->d_quat + 4 * (size_t)mo, 8 * nm);
     return rb.run();
+}
+
+int remc_get_state_rows(remc_ctx *c, int replica, float *pos, float *rel, float *centre, double *quat)
+{
+    CHECK_CTX(c);
+    FINALIZE(c);
+    CHECK_REP(c, replica);
+    if (!pos || !rel || !centre || !quat) return fail(REMC_ERR_ARG, "null output");
+    const HostSys &s = c->systems[c->reps[replica].sys];
+    const size_t nb = s.n_beads, nm = s.n_bodies;
+    const int bo = c->rep_bead_off[replica], mo = c->rep_body_off[replica];
+    if (6 * nb + 11 * nm > c->pin_words) return fail(REMC_ERR_STATE, "read-back of a replica exceeds its buffer");
+    const StateRows g{{c->d_px + bo, c->d_py + bo, c->d_pz + bo, c->d_rx + bo, c->d_ry + bo, c->d_rz + bo},
+                      {c->d_cx + mo, c->d_cy + mo, c->d_cz + mo},
+                      (const uint32_t *)(c->d_quat + 4 * (size_t)mo),
+                      (int)nb,
+                      (int)nm};
+    HIP_TRY(launch_state_rows(g, c->h_pin, next_signal(c), c->stream));
+    const int rc = wait_signal(c);
+    if (rc != REMC_OK) return rc;
+    const uint32_t *h = c->h_pin;
+    std::memcpy(quat, h, 32 * nm);
+    std::memcpy(pos, h + 8 * nm, 12 * nb);
+    std::memcpy(rel, h + 8 * nm + 3 * nb, 12 * nb);
+    std::memcpy(centre, h + 8 * nm + 6 * nb, 12 * nm);
+    return REMC_OK;
 }
 
 int remc_set_state(remc_ctx *c, int replica, const float *x, const float *y, const float *z, const float *rx,

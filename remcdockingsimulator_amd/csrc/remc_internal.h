@@ -175,7 +175,21 @@ struct Gather {
     uint32_t at[GATHER_MAX + 1];
     int n;
 };
-hipError_t launch_gather(const Gather &g, uint32_t *dst, hipStream_t s);
+// How the host learns that a gather's words are there: the last workgroup
+// (counted in *count, which is left at 0) writes ticket to *flag.
+struct Signal {
+    uint32_t *count, *flag;
+    uint32_t ticket;
+};
+hipError_t launch_gather(const Gather &g, uint32_t *dst, const Signal &sig, hipStream_t s);
+// One replica's state as rows: double quat[n_bodies][4], then float pos[n_beads][3],
+// rel[n_beads][3], centre[n_bodies][3], from the arrays at bead / body
+struct StateRows {
+    const float *p[6], *c[3];
+    const uint32_t *quat;
+    int n_beads, n_bodies;
+};
+hipError_t launch_state_rows(const StateRows &g, uint32_t *dst, const Signal &sig, hipStream_t s);
 size_t adjoint_ff_size();
 void adjoint_ff_fill(void *dst, const float *table, double lambda, double e0, double xi, double c_lj, double c_dh);
 

@@ -2661,24 +2661,77 @@ hipError_t launch_exchange(const KParams &p, int n_sys, hipStream_t s)
 // One thread per 32-bit word; consecutive words of an array go out as whole
 // cache lines over the host link.  Latency bound: the launch and the host's
 // wait are paid once for all arrays, where a copy per array into the caller's
-// pageable memory paid a staged copy and its wait for each of ten.  Reading
-// one 1300-bead replica (45 KB): 195 -> 29 us with the caller's part.
+// pageable memory paid a staged copy and its wait for each of ten (195 us for
+// the state of one 1300-bead replica, 45 KB, 29 us so).  The end is signalled by
+// the last workgroup's store to pinned memory, which the host sees several us
+// before the stream's end, and a state comes as the rows that its reader keeps,
+// transposed here for nothing instead of on the host: 18 us; 55 instead of 170
+// us at 11000 beads.
 // --------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_gather(Gather g, uint32_t *dst)
+
+// Called by every thread of every workgroup after its stores to the host.
+__device__ __forceinline__ void signal_done(const Signal &sig)
 {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= g.at[g.n]) return;
-    int k = 0;
-#pragma unroll
-    for (int q = 1; q < GATHER_MAX; ++q) k += q < g.n && i >= g.at[q] ? 1 : 0;
-    dst[i] = g.src[k][i - g.at[k]];
+    __threadfence_system(); // each wave waits for its own stores
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        // wraps to 0 with the last workgroup
+        const uint32_t before = atomicInc(sig.count, gridDim.x - 1);
+        if (before == gridDim.x - 1) {
+            __threadfence_system();
+            __hip_atomic_store(sig.flag, sig.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
 }
 
-hipError_t launch_gather(const Gather &g, uint32_t *dst, hipStream_t s)
+__global__ __launch_bounds__(256) void k_gather(Gather g, uint32_t *dst, Signal sig)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < g.at[g.n]) {
+        int k = 0;
+#pragma unroll
+        for (int q = 1; q < GATHER_MAX; ++q) k += q < g.n && i >= g.at[q] ? 1 : 0;
+        dst[i] = g.src[k][i - g.at[k]];
+    }
+    signal_done(sig);
+}
+
+hipError_t launch_gather(const Gather &g, uint32_t *dst, const Signal &sig, hipStream_t s)
 {
     const uint32_t words = g.at[g.n];
-    if (words == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_gather, dim3((words + 255) / 256), dim3(256), 0, s, g, dst);
+    hipLaunchKernelGGL(k_gather, dim3((words + 255) / 256), dim3(256), 0, s, g, dst, sig);
+    return hipGetLastError();
+}
+
+// One thread per word of the output, so that the host link sees whole lines;
+// the three axes' reads of a wave share their cache lines.
+__global__ __launch_bounds__(256) void k_state_rows(StateRows g, uint32_t *dst, Signal sig)
+{
+    uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t nq = 8u * g.n_bodies, nb = 3u * g.n_beads, nc = 3u * g.n_bodies;
+    if (i < nq + 2 * nb + nc) {
+        uint32_t w;
+        if (i < nq) {
+            w = g.quat[i];
+        } else {
+            const uint32_t j = i - nq;
+            const bool rel = j >= nb, cen = j >= 2 * nb;
+            const uint32_t k = cen ? j - 2 * nb : rel ? j - nb : j;
+            const uint32_t row = k / 3u, axis = k - 3u * row;
+            const float *x = cen ? g.c[0] : rel ? g.p[3] : g.p[0];
+            const float *y = cen ? g.c[1] : rel ? g.p[4] : g.p[1];
+            const float *z = cen ? g.c[2] : rel ? g.p[5] : g.p[2];
+            w = __float_as_uint((axis == 0 ? x : axis == 1 ? y : z)[row]);
+        }
+        dst[i] = w;
+    }
+    signal_done(sig);
+}
+
+hipError_t launch_state_rows(const StateRows &g, uint32_t *dst, const Signal &sig, hipStream_t s)
+{
+    const uint32_t words = 11u * g.n_bodies + 6u * g.n_beads;
+    hipLaunchKernelGGL(k_state_rows, dim3((words + 255) / 256), dim3(256), 0, s, g, dst, sig);
     return hipGetLastError();
 }
 

@@ -234,14 +234,11 @@ class Engine:
     def state(self, replica):
         sa = self.systems[self.replica_sys[replica]]
         n, m = sa.n_beads, sa.n_bodies
-        b = np.empty((6, n), dtype=np.float32)
-        c = np.empty((3, m), dtype=np.float32)
-        q = np.empty((m, 4), dtype=np.float64)
-        pb, pc = b.ctypes.data, c.ctypes.data
-        self._chk(self.lib.remc_get_state(self.ctx, replica, *[pb + 4 * n * k for k in range(6)],
-                                          *[pc + 4 * m * k for k in range(3)], q.ctypes.data), "remc_get_state")
-        return dict(pos=np.ascontiguousarray(b[:3].T), rel=np.ascontiguousarray(b[3:].T),
-                    center=np.ascontiguousarray(c.T), quat=q)
+        pos, rel = np.empty((n, 3), dtype=np.float32), np.empty((n, 3), dtype=np.float32)
+        center, quat = np.empty((m, 3), dtype=np.float32), np.empty((m, 4), dtype=np.float64)
+        self._chk(self.lib.remc_get_state_rows(self.ctx, replica, pos.ctypes.data, rel.ctypes.data, center.ctypes.data,
+                                               quat.ctypes.data), "remc_get_state_rows")
+        return dict(pos=pos, rel=rel, center=center, quat=quat)
 
     def set_state(self, replica, pos=None, rel=None, center=None, quat=None):
         def cols(a, k):
