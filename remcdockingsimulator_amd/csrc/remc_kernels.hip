@@ -625,36 +625,49 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                     // the moved beads come from the partner cache when it holds
                     // them (a member's slice may not), else from HBM
                     const int b = m0k + i;
-                    const bool inc = b >= clo && b < chi;
-                    // typed loads: LDS reads where the data is cached (a
-                    // select between the two pointers would be a flat load)
-                    float rx, ry, rz, cx, cy, cz, ox, oy, oz;
-                    if (cache_rel) {
+                    float rx, ry, rz, cx, cy, cz, ox, oy, oz, qb, sb;
+                    int tb;
+                    if (cache_rel) { // then every bead and body is cached: the reads go out together
                         rx = lds_ld(s_rx + b);
                         ry = lds_ld(s_ry + b);
                         rz = lds_ld(s_rz + b);
+                        cx = lds_ld(s_cx + bk);
+                        cy = lds_ld(s_cy + bk);
+                        cz = lds_ld(s_cz + bk);
+                        ox = lds_ld(s_jx + b);
+                        oy = lds_ld(s_jy + b);
+                        oz = lds_ld(s_jz + b);
+                        qb = lds_ld(s_jq + b);
+                        sb = lds_ld(s_js + b);
+                        tb = lds_ld(s_jtc + b);
                     } else {
                         rx = grx[b];
                         ry = gry[b];
                         rz = grz[b];
-                    }
-                    if (cache_bodies) {
-                        cx = lds_ld(s_cx + bk);
-                        cy = lds_ld(s_cy + bk);
-                        cz = lds_ld(s_cz + bk);
-                    } else {
-                        cx = gcx[bk];
-                        cy = gcy[bk];
-                        cz = gcz[bk];
-                    }
-                    if (inc) {
-                        ox = lds_ld(s_jx + (b - clo));
-                        oy = lds_ld(s_jy + (b - clo));
-                        oz = lds_ld(s_jz + (b - clo));
-                    } else {
-                        ox = gx[b];
-                        oy = gy[b];
-                        oz = gz[b];
+                        if (cache_bodies) {
+                            cx = lds_ld(s_cx + bk);
+                            cy = lds_ld(s_cy + bk);
+                            cz = lds_ld(s_cz + bk);
+                        } else {
+                            cx = gcx[bk];
+                            cy = gcy[bk];
+                            cz = gcz[bk];
+                        }
+                        if (b >= clo && b < chi) {
+                            ox = lds_ld(s_jx + (b - clo));
+                            oy = lds_ld(s_jy + (b - clo));
+                            oz = lds_ld(s_jz + (b - clo));
+                            qb = lds_ld(s_jq + (b - clo));
+                            sb = lds_ld(s_js + (b - clo));
+                            tb = lds_ld(s_jtc + (b - clo));
+                        } else {
+                            ox = gx[b];
+                            oy = gy[b];
+                            oz = gz[b];
+                            qb = qs[b];
+                            sb = sgs[b];
+                            tb = tcs[b];
+                        }
                     }
                     if (chained) {
                         // slot j's proposal, formed as slot j's own staging forms it
@@ -668,15 +681,13 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                     float nrx = rx, nry = ry, nrz = rz, ncx = cx, ncy = cy, ncz = cz;
                     if (Dk.rotate) remc_qrotate(Dk.coef, rx, ry, rz, &nrx, &nry, &nrz);
                     else remc_wrap_centre(cx, cy, cz, Dk.t[0], Dk.t[1], Dk.t[2], S.box, &ncx, &ncy, &ncz);
-                    const float qb = inc ? lds_ld(s_jq + (b - clo)) : qs[b];
-                    const float sb = inc ? lds_ld(s_js + (b - clo)) : sgs[b];
                     s_wold[st] = make_float4(ox, oy, oz, qb * ff.c_dh);
                     s_wnew[st] = make_float4(nrx + ncx, nry + ncy, nrz + ncz, sb);
                     // a static slot: one bead whose move leaves it where it is
                     if (i == 0)
                         s_wstat[k] = nmk == 1 && ox == nrx + ncx && oy == nry + ncy && oz == nrz + ncz ? 1 : 0;
                     s_wrel[st] = make_float4(nrx, nry, nrz, qb);
-                    s_wtc[st] = inc ? lds_ld(s_jtc + (b - clo)) : tcs[b];
+                    s_wtc[st] = tb;
                     if (i == 0 && !Dk.rotate) s_wcen[k] = make_float4(ncx, ncy, ncz, 0.0f);
                 }
                 // a rotated slot's new rotation, formed by the slot's thread 1
@@ -840,14 +851,26 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
             if (tid < WK * WK) {
                 const int jj = tid / WK, kk = tid % WK;
                 if (jj < kk && kk < w) {
+                    // (read ahead of the tests, in one round of LDS reads)
                     const int bj = s_draw[off + jj].body, bk = s_draw[off + kk].body;
+                    const int nmj = s_draw[off + jj].nm, nmk = s_draw[off + kk].nm;
+                    const bool crow = ((s_wtc[jj * SPEC_MAX] | s_wtc[kk * SPEC_MAX]) >> 8) != 0;
+                    const unsigned int chain = s_wchain[kk];
+                    const float4 o0 = s_wold[kk * SPEC_MAX], n0 = s_wnew[kk * SPEC_MAX];
+                    const float4 O0 = s_wold[jj * SPEC_MAX], N0 = s_wnew[jj * SPEC_MAX];
                     float cv = 0.0f;
                     // the same body: slot kk's proposal depends on slot jj's
                     // move, unless kk is chained to jj (the decision handles it)
-                    bool touches = bj == bk && s_wchain[kk] == 0u;
-                    if (bj != bk && ((statm >> jj) & 1ull) == 0ull && ((statm >> kk) & 1ull) == 0ull) {
-                        const int nmj = s_draw[off + jj].nm, nmk = s_draw[off + kk].nm;
-                        const bool crow = ((s_wtc[jj * SPEC_MAX] | s_wtc[kk * SPEC_MAX]) >> 8) != 0;
+                    bool touches = bj == bk && chain == 0u;
+                    const bool apart = bj != bk && ((statm >> jj) & 1ull) == 0ull && ((statm >> kk) & 1ull) == 0ull;
+                    if (apart && crow && nmj == 1 && nmk == 1) {
+                        // one-bead bodies, the common case: four crowder terms
+                        const float e_nn = pair_crowder(dist2(N0.x, N0.y, N0.z, n0, S), ff);
+                        const float e_on = pair_crowder(dist2(N0.x, N0.y, N0.z, o0, S), ff);
+                        const float e_no = pair_crowder(dist2(O0.x, O0.y, O0.z, n0, S), ff);
+                        const float e_oo = pair_crowder(dist2(O0.x, O0.y, O0.z, o0, S), ff);
+                        touches = (e_nn - e_on) - (e_no - e_oo) != 0.0f;
+                    } else if (apart) {
                         float acc = 0.0f, comp = 0.0f;
                         for (int i = 0; i < nmk; ++i) {
                             const float4 o = s_wold[kk * SPEC_MAX + i], n = s_wnew[kk * SPEC_MAX + i];
@@ -924,6 +947,9 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
             }
 
             // decisions in step order (wave 0); lane l carries slot l's dE
+            double w_dE = 0.0;
+            unsigned long long w_acc = 0ull, w_nz = 0ull;
+            int w_nbz = 0;
             if (wave == 0) {
                 // the slot's uniform and masks, read before the wait for the partials
                 const double nll = lane < w ? s_draw[off + lane].nlu : 0.0;
@@ -993,20 +1019,11 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                 }
                 const unsigned long long accm = weff < 64 ? acc0 & ((1ull << weff) - 1ull) : acc0;
                 const unsigned long long boltzm = __ballot(dl == 2) & accm;
-                if (lane == 0) {
-                    // the tracked energy gains the accepted dE in step order, as one step at a time does
-                    double Ew = s_E;
-                    for (unsigned long long m = accm; m; m &= m - 1ull) {
-                        const int k = (int)__builtin_ctzll(m);
-                        Ew += __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(dEl), k),
-                                               __builtin_amdgcn_readlane(__double2loint(dEl), k));
-                    }
-                    s_E = Ew;
-                    const int nacc = __popcll(accm), nbz = __popcll(boltzm);
-                    s_cnt[0] += (unsigned long long)(nacc - nbz);
-                    s_cnt[1] += (unsigned long long)nbz;
-                    s_cnt[2] += (unsigned long long)(weff - nacc);
-                }
+                // kept for the tallies below
+                w_dE = dEl;
+                w_acc = accm;
+                w_nz = accm & __ballot(dEl != 0.0);
+                w_nbz = __popcll(boltzm);
                 // an accepted chained slot supersedes its (accepted) predecessor's
                 // proposal in what the two moves both change
                 if (lane < weff && dl != 0 && chl != 0u) s_wnext[__builtin_ctz(chl)] = lane;
@@ -1016,6 +1033,25 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
             if (s_abort) break;
             if (coop > 1) ++n_x;
             const int weff = s_weff;
+
+            if (wave == 0) {
+                // The tracked energy gains the accepted dE in step order, as one
+                // step at a time does (a slot whose dE is zero adds nothing): a
+                // serial chain, run while the upper half commits.
+                double Ew = s_E;
+                for (unsigned long long m = w_nz; m; m &= m - 1ull) {
+                    const int k = (int)__builtin_ctzll(m);
+                    Ew += __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(w_dE), k),
+                                           __builtin_amdgcn_readlane(__double2loint(w_dE), k));
+                }
+                if (lane == 0) {
+                    s_E = Ew;
+                    const int nacc = __popcll(w_acc);
+                    s_cnt[0] += (unsigned long long)(nacc - w_nbz);
+                    s_cnt[1] += (unsigned long long)w_nbz;
+                    s_cnt[2] += (unsigned long long)(weff - nacc);
+                }
+            }
 
             // commit the accepted moves: copies of what staging formed.  Bodies
             // are distinct except for a chained pair, where the later slot writes
