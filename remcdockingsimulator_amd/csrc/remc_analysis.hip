@@ -119,13 +119,15 @@ __global__ __launch_bounds__(64 * DRMS_WAVES) void k_drms(KParams p, int sys_id,
 }
 
 // one wave per replica: lane l adds units l, l + 64, ..., then a fixed butterfly
-__global__ __launch_bounds__(64) void k_drms_sum(const double *partials, int units, double inv_pairs, double *out)
+__global__ __launch_bounds__(64) void k_drms_sum(const double *partials, int units, double inv_pairs, double *out,
+                                                 Signal sig)
 {
     const int k = blockIdx.x, lane = threadIdx.x;
     double t = 0.0;
     for (int i = lane; i < units; i += 64) t += partials[(size_t)k * units + i];
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-    if (lane == 0) out[k] = t * inv_pairs;
+    if (lane == 0) host_store(out + k, t * inv_pairs);
+    signal_done(sig);
 }
 
 // Columns per unit: 64 until the launch holds enough units for every SIMD to
@@ -143,14 +145,14 @@ size_t drms_units(int n_beads, int n_rep)
 }
 
 hipError_t launch_drms(const KParams &p, int sys_id, int n_beads, int n_rep, const float *rx, const float *ry,
-                       const float *rz, double *partials, double inv_pairs, double *out, hipStream_t s)
+                       const float *rz, double *partials, double inv_pairs, double *out, const Signal &sig, hipStream_t s)
 {
     if (n_rep <= 0 || n_beads <= 0) return hipSuccess;
     const int cols = drms_cols(n_beads, n_rep), nct = (n_beads + cols - 1) / cols;
     const int units = (int)drms_units(n_beads, n_rep);
     hipLaunchKernelGGL(k_drms, dim3(units, (n_rep + DRMS_REPS - 1) / DRMS_REPS), dim3(64 * DRMS_WAVES), 0, s, p, sys_id,
                        rx, ry, rz, partials, n_rep, cols, nct);
-    hipLaunchKernelGGL(k_drms_sum, dim3(n_rep), dim3(64), 0, s, partials, units, inv_pairs, out);
+    hipLaunchKernelGGL(k_drms_sum, dim3(n_rep), dim3(64), 0, s, partials, units, inv_pairs, out, sig);
     return hipGetLastError();
 }
 
@@ -276,7 +278,7 @@ constexpr int HOUT_BINS = 16, HOUT_GROUPS = 64;
 __global__ __launch_bounds__(HOUT_BINS * HOUT_GROUPS) void k_hist_out(const unsigned int *part, int n_part,
                                                                       const int *type_count, int n_types, int nbin,
                                                                       double lo, double dr, double frames_over_volume,
-                                                                      unsigned long long *counts, double *gr)
+                                                                      unsigned long long *counts, double *gr, Signal sig)
 {
     __shared__ unsigned long long s_sum[HOUT_GROUPS][HOUT_BINS];
     const int nh = n_types * n_types * nbin;
@@ -288,21 +290,21 @@ __global__ __launch_bounds__(HOUT_BINS * HOUT_GROUPS) void k_hist_out(const unsi
         for (int g = group; g < n_part; g += HOUT_GROUPS) c += part[(size_t)g * nh + t];
     s_sum[group][bin] = c;
     __syncthreads();
-    if (group != 0 || t >= nh) return;
-    for (int w = 1; w < HOUT_GROUPS; ++w) c += s_sum[w][bin];
-    if (!gr) {
-        counts[t] = c;
-        return;
+    if (group == 0 && t < nh) {
+        for (int w = 1; w < HOUT_GROUPS; ++w) c += s_sum[w][bin];
+        const int b = t % nbin, pair = t / nbin, ti = pair / n_types, tj = pair % n_types;
+        if (!gr) {
+            host_store(counts + t, c);
+        } else if (ti > tj) {
+            host_store(gr + t, 0.0);
+        } else {
+            const double r = lo + (0.5 + (double)b) * dr;
+            const double four_pi = 12.566370614359172953850573533118;
+            const double norm = frames_over_volume * four_pi * r * r * dr * (double)type_count[ti] * (double)type_count[tj];
+            host_store(gr + t, norm > 0.0 ? (double)c / norm : 0.0);
+        }
     }
-    const int b = t % nbin, pair = t / nbin, ti = pair / n_types, tj = pair % n_types;
-    if (ti > tj) {
-        gr[t] = 0.0;
-        return;
-    }
-    const double r = lo + (0.5 + (double)b) * dr;
-    const double four_pi = 12.566370614359172953850573533118;
-    const double norm = frames_over_volume * four_pi * r * r * dr * (double)type_count[ti] * (double)type_count[tj];
-    gr[t] = norm > 0.0 ? (double)c / norm : 0.0;
+    signal_done(sig);
 }
 
 // Workgroups of the histogram: one a unit up to four a CU; fewer where their
@@ -317,14 +319,14 @@ int hist_workgroups(int n_bodies, int n_rep, int nh)
 
 hipError_t launch_centre_hist(const KParams &p, int sys_id, int n_bodies, int n_rep, const int *btype, const int *site,
                               int n_types, int nbin, double lo, double dr, unsigned int *part, const int *type_count,
-                              double frames_over_volume, unsigned long long *counts, double *gr, hipStream_t s)
+                              double frames_over_volume, unsigned long long *counts, double *gr, const Signal &sig, hipStream_t s)
 {
     if (n_rep <= 0 || n_bodies <= 0) return hipSuccess;
     const int nh = n_types * n_types * nbin, n_part = hist_workgroups(n_bodies, n_rep, nh);
     hipLaunchKernelGGL(k_centre_hist, dim3(n_part), dim3(64 * HIST_WAVES), sizeof(unsigned int) * (size_t)nh, s, p, sys_id,
                        n_rep, btype, site, n_types, nbin, lo, dr, part);
     hipLaunchKernelGGL(k_hist_out, dim3((nh + HOUT_BINS - 1) / HOUT_BINS), dim3(HOUT_BINS * HOUT_GROUPS), 0, s, part, n_part,
-                       type_count, n_types, nbin, lo, dr, frames_over_volume, counts, gr);
+                       type_count, n_types, nbin, lo, dr, frames_over_volume, counts, gr, sig);
     return hipGetLastError();
 }
 

@@ -771,9 +771,10 @@ int energies_out(remc_ctx *c, int noncrowder_only, double *out)
     {
         TimedLaunch t(c, 1);
         HIP_TRY(launch_energy_full(c->params(), R, c->max_beads, c->d_fix, c->d_full_partials, (double *)c->h_pin, noncrowder_only,
-                                   0, c->stream));
+                                   0, c->stream, next_signal(c)));
     }
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    const int rc = wait_signal(c);
+    if (rc != REMC_OK) return rc;
     std::memcpy(out, c->h_pin, sizeof(double) * R);
     return REMC_OK;
 }
@@ -2203,8 +2204,9 @@ int remc_drms(remc_ctx *c, int sys_id, const float *ref_x, const float *ref_y, c
     std::memcpy(hx + N, ref_y, sizeof(float) * N);
     std::memcpy(hx + 2 * (size_t)N, ref_z, sizeof(float) * N);
     HIP_TRY(hipMemcpyAsync(rx, hx, 3 * sizeof(float) * N, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(launch_drms(c->params(), sys_id, N, R, rx, ry, rz, part, 1.0 / pairs, hout, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(launch_drms(c->params(), sys_id, N, R, rx, ry, rz, part, 1.0 / pairs, hout, next_signal(c), c->stream));
+    rc = wait_signal(c);
+    if (rc != REMC_OK) return rc;
     std::memcpy(out, hout, sizeof(double) * R);
     return REMC_OK;
 }
@@ -2240,8 +2242,9 @@ static int centre_hist(remc_ctx *c, int sys_id, const int *body_type, const int 
     char *hout = (char *)c->h_pin + ib;
     HIP_TRY(launch_centre_hist(c->params(), sys_id, M, R, d, dsite, n_types, nbin, lo, (hi - lo) / nbin,
                                (unsigned int *)((char *)c->d_ana + ib), dcount, frames_over_volume,
-                               (unsigned long long *)hout, gr ? (double *)hout : nullptr, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+                               (unsigned long long *)hout, gr ? (double *)hout : nullptr, next_signal(c), c->stream));
+    rc = wait_signal(c);
+    if (rc != REMC_OK) return rc;
     std::memcpy(gr ? (void *)gr : (void *)counts, hout, 8 * nh);
     return REMC_OK;
 }

@@ -488,16 +488,18 @@ __global__ __launch_bounds__(COLS) void k_energy_full(KParams p, const int *fix,
 
 // one wave per replica: lane l adds workgroups l, l+64, ... in order, then a
 // fixed-order wave sum (the same total on every call)
-__global__ __launch_bounds__(64) void k_sum_partials(KParams p, int units, const double *partials, double *out, int write_E)
+__global__ __launch_bounds__(64) void k_sum_partials(KParams p, int units, const double *partials, double *out, int write_E,
+                                                     Signal sig)
 {
     const int r = blockIdx.x, lane = threadIdx.x;
     double t = 0.0;
     for (int x = lane; x < units; x += 64) t += partials[(size_t)r * units + x];
     t = wave_sum_dpp(t);
     if (lane == 0) {
-        if (out) out[r] = t;
+        if (out) host_store(out + r, t);
         if (write_E) p.E[r] = t;
     }
+    signal_done(sig);
 }
 
 int full_units(int n_rep, int max_beads)
@@ -510,13 +512,13 @@ int full_units(int n_rep, int max_beads)
 }
 
 hipError_t launch_energy_full(const KParams &p, int n_rep, int max_beads, int *fix, double *partials, double *out,
-                              int noncrowder_only, int write_E, hipStream_t s)
+                              int noncrowder_only, int write_E, hipStream_t s, const Signal &sig)
 {
     if (n_rep <= 0) return hipSuccess;
     launch_fix(p, 0, n_rep, max_beads, fix, s);
     const int units = full_units(n_rep, max_beads);
     hipLaunchKernelGGL(k_energy_full, dim3(units, n_rep), dim3(COLS), 0, s, p, fix, partials, noncrowder_only);
-    hipLaunchKernelGGL(k_sum_partials, dim3(n_rep), dim3(64), 0, s, p, units, partials, out, write_E);
+    hipLaunchKernelGGL(k_sum_partials, dim3(n_rep), dim3(64), 0, s, p, units, partials, out, write_E, sig);
     return hipGetLastError();
 }
 

@@ -131,8 +131,38 @@ size_t mc_fb_dynamic_lds(const KParams &p);
 hipError_t mc_max_active_per_cu(const KParams &p, int block, int *out);
 // full energies of n_rep replicas of at most max_beads beads: fix holds
 // fix_ints(...) ints (scratch), partials n_rep x full_units(...) doubles
+// How the host learns that a kernel's results are in pinned memory: the last workgroup
+// (counted in *count, which is left at 0) writes ticket to *flag.
+struct Signal {
+    uint32_t *count, *flag;
+    uint32_t ticket;
+};
+// A result's store to pinned memory: written through to the host, so that its
+// completion (counted by the wave) is its visibility, with no cache to flush.
+template <typename T>
+__device__ __forceinline__ void host_store(T *ptr, T v)
+{
+    __hip_atomic_store(ptr, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Called by every thread of every workgroup after its host_store's (no flag:
+// nobody waits for it).  Every wave waits for its own stores, so the last
+// workgroup to count itself stores the ticket after all of them.  (A system
+// fence here writes back the L2 for every wave: 25 us in a gather of 476 KB.)
+__device__ __forceinline__ void signal_done(const Signal &sig)
+{
+    if (!sig.flag) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        // wraps to 0 with the last workgroup
+        const uint32_t before = atomicInc(sig.count, gridDim.x - 1);
+        if (before == gridDim.x - 1) host_store(sig.flag, sig.ticket);
+    }
+}
+
 hipError_t launch_energy_full(const KParams &p, int n_rep, int max_beads, int *fix, double *partials, double *out,
-                              int noncrowder_only, int write_E, hipStream_t s);
+                              int noncrowder_only, int write_E, hipStream_t s, const Signal &sig = Signal{});
 int full_units(int n_rep, int max_beads);
 constexpr int GROUP = 16;                          // beads of a column group of the all-pairs kernels
 constexpr int GROUP_CHAIN = 1, GROUP_CROWDER = 2; // kinds of beads present (KParams::grp)
@@ -158,14 +188,14 @@ hipError_t launch_adjoint(const KParams &p, const void *adj_ff, const AdjPlan &a
                           int max_beads, int body_waves, int bead_base, size_t bead_stride, int body_base, int *fix,
                           double *scratch, double *force_torque, double *dparams, hipStream_t s);
 hipError_t launch_drms(const KParams &p, int sys_id, int n_beads, int n_rep, const float *rx, const float *ry,
-                       const float *rz, double *partials, double inv_pairs, double *out, hipStream_t s);
+                       const float *rz, double *partials, double inv_pairs, double *out, const Signal &sig, hipStream_t s);
 size_t drms_units(int n_beads, int n_rep); // partials of launch_drms per replica
 // part: hist_workgroups(...) x nh 32-bit counts; the result goes to gr when it
 // is given, else to counts
 int hist_workgroups(int n_bodies, int n_rep, int nh);
 hipError_t launch_centre_hist(const KParams &p, int sys_id, int n_bodies, int n_rep, const int *btype, const int *site,
                               int n_types, int nbin, double lo, double dr, unsigned int *part, const int *type_count,
-                              double frames_over_volume, unsigned long long *counts, double *gr, hipStream_t s);
+                              double frames_over_volume, unsigned long long *counts, double *gr, const Signal &sig, hipStream_t s);
 // Up to GATHER_MAX device arrays read back by one launch: array k's words go to
 // dst[at[k]] .. dst[at[k + 1]) (32-bit words, packed without gaps), dst being
 // pinned host memory.
@@ -174,12 +204,6 @@ struct Gather {
     const uint32_t *src[GATHER_MAX];
     uint32_t at[GATHER_MAX + 1];
     int n;
-};
-// How the host learns that a gather's words are there: the last workgroup
-// (counted in *count, which is left at 0) writes ticket to *flag.
-struct Signal {
-    uint32_t *count, *flag;
-    uint32_t ticket;
 };
 hipError_t launch_gather(const Gather &g, uint32_t *dst, const Signal &sig, hipStream_t s);
 // One replica's state as rows: double quat[n_bodies][4], then float pos[n_beads][3],

@@ -2701,24 +2701,9 @@ hipError_t launch_exchange(const KParams &p, int n_sys, hipStream_t s)
 // the state of one 1300-bead replica, 45 KB, 29 us so).  The end is signalled by
 // the last workgroup's store to pinned memory, which the host sees several us
 // before the stream's end, and a state comes as the rows that its reader keeps,
-// transposed here for nothing instead of on the host: 18 us; 55 instead of 170
+// transposed here for nothing instead of on the host: 14 us; 29 instead of 170
 // us at 11000 beads.
 // --------------------------------------------------------------------------
-
-// Called by every thread of every workgroup after its stores to the host.
-__device__ __forceinline__ void signal_done(const Signal &sig)
-{
-    __threadfence_system(); // each wave waits for its own stores
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        // wraps to 0 with the last workgroup
-        const uint32_t before = atomicInc(sig.count, gridDim.x - 1);
-        if (before == gridDim.x - 1) {
-            __threadfence_system();
-            __hip_atomic_store(sig.flag, sig.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
-    }
-}
 
 __global__ __launch_bounds__(256) void k_gather(Gather g, uint32_t *dst, Signal sig)
 {
@@ -2727,7 +2712,7 @@ __global__ __launch_bounds__(256) void k_gather(Gather g, uint32_t *dst, Signal 
         int k = 0;
 #pragma unroll
         for (int q = 1; q < GATHER_MAX; ++q) k += q < g.n && i >= g.at[q] ? 1 : 0;
-        dst[i] = g.src[k][i - g.at[k]];
+        host_store(dst + i, g.src[k][i - g.at[k]]);
     }
     signal_done(sig);
 }
@@ -2759,7 +2744,7 @@ __global__ __launch_bounds__(256) void k_state_rows(StateRows g, uint32_t *dst, 
             const float *z = cen ? g.c[2] : rel ? g.p[5] : g.p[2];
             w = __float_as_uint((axis == 0 ? x : axis == 1 ? y : z)[row]);
         }
-        dst[i] = w;
+        host_store(dst + i, w);
     }
     signal_done(sig);
 }
