@@ -510,7 +510,7 @@ def main(argv=None):
                 "pair_terms_per_s": terms / (ek / 1e3),
                 "roofline_frac": terms / (ek / 1e3) * FLOPS_PER_PAIR / 1e12 / PEAK_FP32_TFLOPS,
                 "calls_per_s_wall": args.energy_calls / (t9 - t8),
-                "kernel": "k_energy_full + k_sum_partials (full FP32-Kahan energy of every replica, FP64 totals)",
+                "kernel": "k_energy_full + k_sum_partials (full energy of every replica, FP32 terms, FP64 sums)",
                 "work_per_call": "%d inter-body pair terms over all replicas" % terms}
         log("full energy: %.3f ms per refresh of all replicas (kernels)" % ek)
 
@@ -559,7 +559,7 @@ def main(argv=None):
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32",
-        "precision": "f32 pair terms, Kahan per thread, f64 totals/Metropolis/exchange",
+        "precision": "f32 pair terms, f64 sums (Kahan f32 in windows)/Metropolis/exchange",
         "data": "synthetic (seeded self-avoiding chains, uniform residue types, seeded [-0.6,0] kT contact table)",
         "config": {"workload": workload_label(cid, wl), "replicas": R, "steps_per_exchange": spl,
                    "timed_mc_steps_per_replica": pl["timed_mc_steps_per_replica"],

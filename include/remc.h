@@ -125,8 +125,8 @@ REMC_API int remc_get_sizes(remc_ctx *ctx, int *n_systems, int *n_replicas, int 
  * (Replica.cpp:1601-1616).  block = 0 picks the reference's rule (32 if
  * N < 1024 else 64, main.cpp:1746-1747). */
 REMC_API int remc_energy_plain(remc_ctx *ctx, int replica, int block, double *out);
-/* Batched full energy of every replica in one launch: FP32 pair terms with
- * Kahan sums per thread, FP64 across threads and tiles.  out[n_replicas].
+/* Batched full energy of every replica in one launch: FP32 pair terms, FP64
+ * sums.  out[n_replicas].
  * Same quantity as Replica::E() (Replica.cpp:603-745). */
 REMC_API int remc_energy_all(remc_ctx *ctx, double *out);
 /* remc_energy_all without any allocation, for callers that cannot allocate
@@ -290,6 +290,8 @@ REMC_API int remc_get_mc_block(remc_ctx *ctx, int *block);
  * has been called with block 0). */
 REMC_API int remc_get_fb_block(remc_ctx *ctx, int *block);
 /* Workgroups per replica of the MC kernel (0 = autotune; else 1, 2, 4 or 8).
+ * The autotuner may give the replicas of unequal systems 1 to 32 each, by the
+ * systems' cost; remc_get_mc_coop is then 1.
  * With more than one, each workgroup keeps a private copy of its replica's
  * state, evaluates dE over a slice of the partner beads, and the members add
  * their partials through device memory (once per split step, once per
@@ -309,8 +311,7 @@ REMC_API int remc_set_mc_tuning(remc_ctx *ctx, int lds_cache, int split_min_pair
  * window interacts with (exact pair corrections between the moved bodies) or
  * whose body it moved.  A step whose body exactly one earlier step of the
  * window moved is proposed from that step's proposal instead, and ends the
- * window only if that step is rejected.  Used when a partner cache fits in
- * LDS (the replica, or each member's slice).  Decisions and states equal those
+ * window only if that step is rejected.  Decisions and states equal those
  * of one step at a time up to FP32 rounding.  The force-biased kernel's windows
  * of one-bead crowder moves follow the same switch.  0 turns the windows off.
  * No counterpart in the reference. */

@@ -1,6 +1,6 @@
 // remc_kernels.hip -- gfx950 kernels of the REMC hot path.
 //
-//   k_mc<BLOCK,CACHE,SPEC>  batched persistent MC: 1-8 workgroups per replica
+//   k_mc<BLOCK,CACHE,SPEC>  batched persistent MC: 1-32 workgroups per replica
 //                      run nsteps steps (proposal, dE of the moved body against
 //                      all other beads, FP64 Metropolis, commit) without
 //                      leaving the GPU, small moves in speculative windows.
@@ -118,12 +118,11 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float v)
 // Workgroup b serves replica p.wg[b].r as member c of its coop members.  Where
 // all replicas have as many, b = c n_rep + r (so with n_rep a multiple of 8 the
 // members of one replica share an XCD and its L2); in a context of unequal
-// systems the members may follow the systems' cost (balanced_plan).  Member c keeps a
-// private copy c of the replica's dynamic state and evaluates dE over the
+// systems the members may follow the systems' cost (balanced_plan).  Member c
+// keeps a private copy of the replica's dynamic state and evaluates dE over the
 // partner-bead slice [c*N/coop, (c+1)*N/coop).  Members publish their partial
-// dE per split step (per window: one per slot) in a 64-bit slot (value with
-// its low 20 bits replaced by the step
-// tag, written with one atomic store) and every member adds the coop partials
+// dE per split step (per window: one per slot) in a 64-bit slot (value with its
+// low 20 bits replaced by the step tag, written with one atomic store) and every member adds the coop partials
 // in member order, so all members take the identical decision and update
 // their copies identically.  With coop = 1 no slot is used.  A member that
 // waits longer than a bounded number of polls sets the error flag; every
