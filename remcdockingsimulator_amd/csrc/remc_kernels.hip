@@ -2132,15 +2132,21 @@ __global__ __launch_bounds__(BLOCK) void k_mc_fb(KParams p, int nsteps, int coop
                     p.rec[(size_t)r * p.rec_max + idx] = rr;
                 }
             }
-            // the tracked energy and the counters, in step order, in every thread
-            for (int k = 0; k < weff; ++k) {
-                const int dk = s_wdec[k];
-                if (dk) {
-                    E += s_wdE[k];
-                    if (dk == 1) ++n_acc; else ++n_accb;
-                } else {
-                    ++n_rej;
+            // the tracked energy, in step order, and the counters, in every
+            // thread: each lane reads one slot (a read of each slot in turn
+            // waited twice for LDS 16 times over), and a dE of zero adds nothing
+            {
+                const int dl = lane < weff ? s_wdec[lane] : 0;
+                const double el = lane < weff ? s_wdE[lane] : 0.0;
+                const unsigned long long acc = __ballot(dl != 0), down = __ballot(dl == 1);
+                for (unsigned long long m = acc & __ballot(el != 0.0); m; m &= m - 1ull) {
+                    const int k = (int)__builtin_ctzll(m);
+                    E += __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(el), k),
+                                          __builtin_amdgcn_readlane(__double2loint(el), k));
                 }
+                n_acc += __popcll(down);
+                n_accb += __popcll(acc & ~down);
+                n_rej += weff - __popcll(acc);
             }
             __syncthreads();
             it += weff - 1;
