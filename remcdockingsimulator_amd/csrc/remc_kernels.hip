@@ -749,6 +749,29 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
             const int wv = __builtin_amdgcn_readfirstlane(wave);
             const unsigned long long ma = __ballot(wk_l && rank_l == wv), mb = __ballot(wk_l && rank_l == wv + NW);
             int ka = ma ? (int)__builtin_ctzll(ma) : WK, kb = mb ? (int)__builtin_ctzll(mb) : WK;
+            // The crowder terms of a one-bead move from o to n.  Without the
+            // cache they are the single steps' own (box units about o): such
+            // contexts took single steps where windows needed the cache, and a
+            // distance that rounds to the other side of the cutoff changes an
+            // energy by the whole step there.
+            const float w_ib = S.inv_box, w_ib2 = w_ib * w_ib;
+            const float w_cut2 = ff.crow_cut2 * w_ib2, w_ck = ff.crow_k * (w_ib2 * w_ib2 * w_ib2);
+            const bool w_A = CACHE || !(w_ib > 0.0f); // in Angstrom
+            auto crow_limit = [&](float4 o, float4 n) {
+                const float lim2 = crowder_screen2(o, n, S, ff);
+                return w_A ? lim2 : lim2 * w_ib2;
+            };
+            // (products rounded before they are subtracted, as the staged ones are)
+            auto crow_unit = [&](float px, float py, float pz, float4 o) {
+#pragma clang fp contract(off)
+                return make_float4((px - o.x) * w_ib, (py - o.y) * w_ib, (pz - o.z) * w_ib, 0.0f);
+            };
+            auto crow_r2 = [&](float px, float py, float pz, float4 o, float4 at) {
+                if (w_A) return dist2(px, py, pz, at, S);
+                const float4 u = crow_unit(px, py, pz, o);
+                return dist2_unit(u.x, u.y, u.z, crow_unit(at.x, at.y, at.z, o));
+            };
+            auto crow_term = [&](float r2) { return w_A ? pair_crowder(r2, ff) : pair_crowder_u(r2, w_cut2, w_ck); };
             if (kb < w && s_draw[off + ka].nm == 1 && s_draw[off + kb].nm == 1 &&
                 ((s_wtc[ka * SPEC_MAX] & s_wtc[kb * SPEC_MAX]) >> 8) != 0) {
                 // both slots of the wave move one crowder bead: one pass over the
@@ -756,23 +779,23 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                 const float4 oa = s_wold[ka * SPEC_MAX], na = s_wnew[ka * SPEC_MAX];
                 const float4 ob = s_wold[kb * SPEC_MAX], nb = s_wnew[kb * SPEC_MAX];
                 const int ba = s_draw[off + ka].m0, bb = s_draw[off + kb].m0;
-                const float lim2a = crowder_screen2(oa, na, S, ff), lim2b = crowder_screen2(ob, nb, S, ff);
+                const float lim2a = crow_limit(oa, na), lim2b = crow_limit(ob, nb);
                 float acc_a = 0.0f, comp_a = 0.0f, acc_b = 0.0f, comp_b = 0.0f;
                 for (int j = wjs + lane; j < wje; j += 64) {
                     const float xj = CACHE ? s_jx[j - clo] : gx[j], yj = CACHE ? s_jy[j - clo] : gy[j],
                                 zj = CACHE ? s_jz[j - clo] : gz[j];
                     // the terms at the new positions only where a partner of the
                     // wave is near enough to give any (crowders are sparse)
-                    const float r2a = dist2(xj, yj, zj, oa, S), r2b = dist2(xj, yj, zj, ob, S);
+                    const float r2a = crow_r2(xj, yj, zj, oa, oa), r2b = crow_r2(xj, yj, zj, ob, ob);
                     if (!__any((j != ba && r2a < lim2a) || (j != bb && r2b < lim2b))) continue;
                     if (j != ba) {
-                        const float eo = pair_crowder(r2a, ff);
-                        const float en = pair_crowder(dist2(xj, yj, zj, na, S), ff);
+                        const float eo = crow_term(r2a);
+                        const float en = crow_term(crow_r2(xj, yj, zj, oa, na));
                         kahan_add(acc_a, comp_a, en - eo);
                     }
                     if (j != bb) {
-                        const float eo = pair_crowder(r2b, ff);
-                        const float en = pair_crowder(dist2(xj, yj, zj, nb, S), ff);
+                        const float eo = crow_term(r2b);
+                        const float en = crow_term(crow_r2(xj, yj, zj, ob, nb));
                         kahan_add(acc_b, comp_b, en - eo);
                     }
                 }
@@ -800,15 +823,15 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                 if (nmk == 1 && crow_m) {
                     // one crowder bead: partners screened as in the two-slot pass
                     const float4 o = s_wold[k * SPEC_MAX], n = s_wnew[k * SPEC_MAX];
-                    const float lim2 = crowder_screen2(o, n, S, ff);
+                    const float lim2 = crow_limit(o, n);
                     for (int j = wjs + lane; j < wje; j += 64) {
                         const float xj = CACHE ? s_jx[j - clo] : gx[j], yj = CACHE ? s_jy[j - clo] : gy[j],
                                     zj = CACHE ? s_jz[j - clo] : gz[j];
-                        const float r2o = dist2(xj, yj, zj, o, S);
+                        const float r2o = crow_r2(xj, yj, zj, o, o);
                         if (!__any(j != m0k && r2o < lim2)) continue;
                         if (j != m0k) {
-                            const float eo = pair_crowder(r2o, ff);
-                            const float en = pair_crowder(dist2(xj, yj, zj, n, S), ff);
+                            const float eo = crow_term(r2o);
+                            const float en = crow_term(crow_r2(xj, yj, zj, o, n));
                             kahan_add(acc, comp, en - eo);
                         }
                     }
