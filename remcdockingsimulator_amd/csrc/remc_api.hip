@@ -2191,6 +2191,7 @@ int remc_drms(remc_ctx *c, int sys_id, const float *ref_x, const float *ref_y, c
         beads_before += nm;
     }
     if (pairs <= 0.0) return fail(REMC_ERR_ARG, "system %d has fewer than two non-crowder bodies", sys_id);
+    if (R == 0) return REMC_OK; // no replica, no value
     // scratch: the reference, then the partials; the reference goes up in one
     // copy from pinned memory, the results come back into it
     const size_t fbytes = ((3 * (size_t)N * sizeof(float) + 255) / 256) * 256;
@@ -2220,6 +2221,10 @@ static int centre_hist(remc_ctx *c, int sys_id, const int *body_type, const int 
     const HostSys &s = c->systems[sys_id];
     const int M = s.n_bodies, R = (int)s.replicas.size();
     const size_t nh = (size_t)n_types * n_types * nbin;
+    if (R == 0) { // no conformation to count: nothing is launched, so nothing would be read back
+        std::memset(gr ? (void *)gr : (void *)counts, 0, 8 * nh);
+        return REMC_OK;
+    }
     const size_t ints = (site_bead ? 2 : 1) * (size_t)M + (type_count ? n_types : 0);
     const size_t ib = (ints * sizeof(int) + 255) / 256 * 256;
     int rc = ana_reserve(c, ib + sizeof(unsigned int) * nh * (size_t)hist_workgroups(M, R, (int)nh));
