@@ -356,7 +356,7 @@ int finalize(remc_ctx *c)
         d.grp_off = (int)(grp.size() / 4);
         d.box = s.box > 0.f ? s.box : 0.f;
         d.inv_box = s.box > 0.f ? 1.0f / s.box : 0.f;
-        d.unit = s.box > 0.f ? 4294967296.0 / (double)s.box : 1.0;
+        d.unit = box_in_fractions(s.box) ? 4294967296.0 / (double)s.box : 1.0;
         dsys.push_back(d);
         for (int m = 0; m < s.n_bodies; ++m) {
             bstart.push_back(s.body_start[m]);

@@ -16,15 +16,13 @@
 // LDS returns 64 lanes' worth of data a column), and the work per pair is cut
 // to what the class needs:
 //   - the minimum image.  d - L rint(d/L) costs four instructions an axis in
-//     floating point.  k_fix writes every coordinate as a 32-bit fraction of
-//     the box: the difference of two wraps to the nearest image by itself, in
-//     one subtraction and one conversion, and is as exact as the difference of
-//     the two floats (a unit is 2^-32 of the box, far below their spacing; the
-//     conversion rounds to 24 bits as the subtraction of floats does).
+//     floating point.  In boxes of up to FIX_BOX_MAX k_fix writes every
+//     coordinate as a 32-bit fraction of the box: the difference of two wraps to
+//     the nearest image by itself, in one subtraction and one conversion.
 //     Contact distances are in that unit, with the constants scaled to it
 //     (sigma_ij^2 as a sum of two floats: rounded to one, its error would be the
-//     same in every pair and add up); a system without a box takes float
-//     differences in Angstrom.  Crowder pairs
+//     same in every pair and add up).  Larger boxes and systems without one take
+//     float differences in Angstrom (CoordForm).  Crowder pairs
 //     keep the float form, which decides what lies inside their cutoff.
 //   - crowder pairs end at 15 A.  The crowder columns of a chain's rows are
 //     screened by their distance from the rows' groups against the groups'
@@ -48,6 +46,23 @@ constexpr int ROWS = 64;                // row beads of a workgroup (a tile)
 constexpr int WAVES = 4;                // waves of a workgroup
 constexpr int COLS = 64 * WAVES;        // threads of a workgroup
 constexpr int TSTRIDE = REMC_NTYPES + 1; // row stride of the type tables in LDS: 21 entries keep rows on different banks
+
+// How a system's contact distances are formed.  A fraction of a box L is rounded
+// to L 2^-32, so a difference of two is off by up to that much, where the
+// difference of two near floats is exact: at 1024 A it is 2^-22 A, what a
+// difference of 4-8 A (a contact's) may be off by when rounded to 24 bits, and it
+// grows with the box.  Mean square error of (sigma/r)^6, pairs 4.5-8 A apart
+// anywhere in the box (emulated, reciprocals off by half a unit): 2.2e-7 at
+// 150 A, 2.3e-7 at 600, 2.5e-7 at 1000, 5.1e-7 at 5000, 9.5e-5 at 1e6 A; float
+// differences 1.8e-7 in any box, and 3.0e-7 with a squared reciprocal root, as
+// the moves' terms have.
+enum CoordForm {
+    FRACTION, // fractions of the box
+    IMAGE,    // float differences, nearest image
+    FLAT      // float differences, no box
+};
+template <CoordForm F>
+using Form = std::integral_constant<CoordForm, F>;
 
 // A replica's beads and groups for reads at wave-uniform indices: through the
 // constant address space they become scalar loads.  Nothing writes these arrays
@@ -87,6 +102,7 @@ struct Row {
     bool on, crow;
     int kinds, b0, b1; // kinds and body range of the rows (uniform)
     int g0, gn;        // their first group and its number of groups (uniform)
+    float size;        // their largest |x| + |y| + |z| (uniform, screen_limit)
 };
 
 __device__ __forceinline__ Row load_row(int tile, int N, const float *gx, const float *gy, const float *gz, const int *tcs,
@@ -110,11 +126,14 @@ __device__ __forceinline__ Row load_row(int tile, int N, const float *gx, const 
     r.b1 = __builtin_amdgcn_readlane(r.body, 63);
     r.g0 = tile * (ROWS / GROUP);
     r.gn = min(ROWS / GROUP, full_groups(N) - r.g0);
+    const int s = __float_as_int(row16<true>(fabsf(r.x) + fabsf(r.y) + fabsf(r.z)));
+    const float s0 = __int_as_float(__builtin_amdgcn_readlane(s, 0)), s1 = __int_as_float(__builtin_amdgcn_readlane(s, 16)),
+                s2 = __int_as_float(__builtin_amdgcn_readlane(s, 32)), s3 = __int_as_float(__builtin_amdgcn_readlane(s, 48));
+    r.size = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(fmaxf(fmaxf(s0, s1), fmaxf(s2, s3)))));
     return r;
 }
 
-// The lane's row and the unit of contact distances: fractions of the box
-// (PBC), or Angstrom.
+// The lane's row as fractions of the box (FRACTION).
 struct RowFix {
     int x, y, z;
 };
@@ -125,19 +144,19 @@ __device__ __forceinline__ RowFix load_row_fix(const Row &r, const int *fx, cons
 }
 
 // A column's bead as the contact pairs read it (uniform): coordinates as
-// fractions of the box (PBC) or in Angstrom.
+// fractions of the box (FRACTION) or in Angstrom.
 struct Column {
     int fx, fy, fz, tc;
     float x, y, z, q, s;
 };
-template <bool TAB, bool PBC, int N>
+template <bool TAB, CoordForm FORM, int N>
 __device__ __forceinline__ void load_columns(const Beads &B, int j, Column *c)
 {
     const auto fx = B.fx + j, fy = B.fy + j, fz = B.fz + j, tc = B.tc + j;
     const auto x = B.x + j, y = B.y + j, z = B.z + j, q = B.q + j, s = B.s + j;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-        if (PBC) {
+        if (FORM == FRACTION) {
             c[k].fx = fx[k];
             c[k].fy = fy[k];
             c[k].fz = fz[k];
@@ -153,10 +172,11 @@ __device__ __forceinline__ void load_columns(const Beads &B, int j, Column *c)
 }
 
 // Column minus the lane's row, nearest image.
-template <bool PBC>
-__device__ __forceinline__ void separation(const Column &c, const Row &r, const RowFix &f, float &dx, float &dy, float &dz)
+template <CoordForm FORM>
+__device__ __forceinline__ void separation(const Column &c, const Row &r, const RowFix &f, const DevSys &S, float &dx,
+                                           float &dy, float &dz)
 {
-    if (PBC) {
+    if (FORM == FRACTION) {
         dx = (float)(int)((unsigned)c.fx - (unsigned)f.x);
         dy = (float)(int)((unsigned)c.fy - (unsigned)f.y);
         dz = (float)(int)((unsigned)c.fz - (unsigned)f.z);
@@ -164,17 +184,34 @@ __device__ __forceinline__ void separation(const Column &c, const Row &r, const 
         dx = c.x - r.x;
         dy = c.y - r.y;
         dz = c.z - r.z;
+        if (FORM == IMAGE) {
+            dx = min_image(dx, S.box, S.inv_box);
+            dy = min_image(dy, S.box, S.inv_box);
+            dz = min_image(dz, S.box, S.inv_box);
+        }
     }
 }
 
 // (sigma_ij / r)^2 from 1/r^2: sigma_ij^2 from the table entry (TAB) or the two
 // beads' sigma.
-template <bool TAB, bool PBC>
+template <bool TAB, CoordForm FORM>
 __device__ __forceinline__ float sigma2_over_r2(const float4 &et, float inv2, float si, float sj, float u2, float u2l)
 {
-    if (TAB) return PBC ? __builtin_fmaf(inv2, et.y, inv2 * et.z) : inv2 * et.y;
+    if (TAB) return FORM == FRACTION ? __builtin_fmaf(inv2, et.y, inv2 * et.z) : inv2 * et.y;
     const float sij = 0.5f * (si + sj), t = sij * sij * inv2;
-    return PBC ? __builtin_fmaf(t, u2, t * u2l) : t;
+    return FORM == FRACTION ? __builtin_fmaf(t, u2, t * u2l) : t;
+}
+
+// How far from the middle of a group of extent w (k_fix) a bead of |x| + |y| +
+// |z| = size may lie to reach one of the group's beads within the crowder cutoff
+// as float distances have it.  0.1 A covers the distances' own rounding; each
+// difference of two coordinates is rounded by up to 2^-24 of their sizes (they
+// may lie boxes away, or in a box of 1e6 A), in the pair's distance and in the
+// screen's: 2^-22 of the bead's size here, of the group's in w.
+constexpr float SCREEN_ROUND = 2.384185791015625e-7f; // 2^-22
+__device__ __forceinline__ float screen_limit(float w, const DevFF &ff, float size)
+{
+    return __builtin_fmaf(size, SCREEN_ROUND, w + ff.crow_cut + 0.1f);
 }
 
 // Walks the columns of group g against the wave's rows.  op is called as
@@ -202,13 +239,14 @@ __device__ __forceinline__ void walk_group(OP &op, const Beads &B, int g, const 
     if (((kinds | r.kinds) & GROUP_CROWDER) == 0 || !op.crowders()) return;
     if (kinds & GROUP_CROWDER) {
         // crowder columns that may reach a row: lane 16 q + k looks at column k
-        // and row group q (0.1 A covers the rounding)
+        // and row group q
         const int lane = threadIdx.x & 63, k = lane & 15, q = lane >> 4;
         bool near = false;
         if (k < cnt && q < r.gn && (op.tcs[j + k] >> 8) != 0) {
             const float4 c = op.gc[r.g0 + q];
-            const float lim = c.w + ff.crow_cut + 0.1f;
-            near = !(dist2(op.gx[j + k], op.gy[j + k], op.gz[j + k], c, S) > lim * lim);
+            const float x = op.gx[j + k], y = op.gy[j + k], z = op.gz[j + k];
+            const float lim = screen_limit(c.w, ff, fabsf(x) + fabsf(y) + fabsf(z));
+            near = !(dist2(x, y, z, c, S) > lim * lim);
         }
         const unsigned long long m4 = __ballot(near);
         for (unsigned int m = (unsigned int)(m4 | m4 >> 16 | m4 >> 32 | m4 >> 48) & 0xFFFFu; m; m &= m - 1u)
@@ -216,7 +254,7 @@ __device__ __forceinline__ void walk_group(OP &op, const Beads &B, int g, const 
     }
     if ((kinds & GROUP_CHAIN) && (r.kinds & GROUP_CROWDER)) {
         // the group's extent against the crowder rows
-        const float lim = B.c[4 * g + 3] + ff.crow_cut + 0.1f;
+        const float lim = screen_limit(B.c[4 * g + 3], ff, r.size);
         const float d2 = dist2(B.c[4 * g], B.c[4 * g + 1], B.c[4 * g + 2], make_float4(r.x, r.y, r.z, 0.f), S);
         if (__any(r.crow && !(d2 > lim * lim)))
             for (int k = 0; k < cnt; ++k)
@@ -226,10 +264,10 @@ __device__ __forceinline__ void walk_group(OP &op, const Beads &B, int g, const 
 
 // What the kernels below read of the conformation, made once a call:
 //   fix[k * p.copy_beads + b], k = 0..2: coordinate k of replica bead b as a
-//     fraction of its box;
+//     fraction of its box (boxes of up to FIX_BOX_MAX);
 //   then per replica and group of 16 beads (R.grp_off groups before the
 //   replica's) the middle of the range of their coordinates and half its
-//   diagonal, 4 floats.
+//   diagonal (with what rounding may add, screen_limit), 4 floats.
 __global__ __launch_bounds__(256) void k_fix(KParams p, int rep_first, int *fix)
 {
     const DevRep R = p.rep[rep_first + blockIdx.y];
@@ -239,7 +277,7 @@ __global__ __launch_bounds__(256) void k_fix(KParams p, int rep_first, int *fix)
     const bool on = b < S.n_beads;
     const size_t i = (size_t)R.bead_off + min(b, S.n_beads - 1);
     const float x = p.px[i], y = p.py[i], z = p.pz[i];
-    if (on && S.box > 0.f) {
+    if (on && box_in_fractions(S.box)) {
         fix[i] = fix_coord(x, S.unit);
         fix[p.copy_beads + i] = fix_coord(y, S.unit);
         fix[2 * p.copy_beads + i] = fix_coord(z, S.unit);
@@ -249,8 +287,10 @@ __global__ __launch_bounds__(256) void k_fix(KParams p, int rep_first, int *fix)
     const float hx = row16<true>(x), hy = row16<true>(y), hz = row16<true>(z);
     if ((threadIdx.x & 15) == 0) {
         const float ex = hx - lx, ey = hy - ly, ez = hz - lz;
+        const float mx = fmaxf(-lx, hx), my = fmaxf(-ly, hy), mz = fmaxf(-lz, hz); // the largest sizes
         ((float4 *)(fix + fix_centres(p.copy_beads)))[(size_t)R.grp_off + b / GROUP] =
-            make_float4(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz), 0.5f * sqrtf(ex * ex + ey * ey + ez * ez));
+            make_float4(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz),
+                        0.5f * sqrtf(ex * ex + ey * ey + ez * ez) + SCREEN_ROUND * (mx + my + mz));
     }
 }
 
@@ -277,7 +317,7 @@ static void launch_fix(const KParams &p, int rep_first, int n_rep, int max_beads
 // and 15.7 in the other, of 250 beads 17.4 and 17.7.
 constexpr int FULL_SMALL = 256;
 
-template <bool TAB, bool PBC, bool SMALL>
+template <bool TAB, CoordForm FORM, bool SMALL>
 struct EnergyOp {
     const Beads &B;
     const float *gx, *gy, *gz; // positions, types and groups, for reads by lane
@@ -306,9 +346,9 @@ struct EnergyOp {
         Term t;
         const float4 et = erow[c.tc];
         float dx, dy, dz;
-        separation<PBC>(c, r, f, dx, dy, dz);
+        separation<FORM>(c, r, f, S, dx, dy, dz);
         t.r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-        const float s2 = sigma2_over_r2<TAB, PBC>(et, __builtin_amdgcn_rcpf(t.r2), s, c.s, u2, u2l);
+        const float s2 = sigma2_over_r2<TAB, FORM>(et, __builtin_amdgcn_rcpf(t.r2), s, c.s, u2, u2l);
         t.x6 = s2 * s2 * s2;
         t.e4 = et.x;
         t.e = et.x * __builtin_fmaf(-t.x6, t.x6, t.x6);
@@ -355,13 +395,13 @@ struct EnergyOp {
         int k = 0;
         for (; k + 3 < n; k += 4) {
             Column c[4];
-            load_columns<TAB, PBC, 4>(B, j + k, c);
+            load_columns<TAB, FORM, 4>(B, j + k, c);
             step<2>(c, chm >> k);
             step<2>(c + 2, chm >> (k + 2));
         }
         for (; k < n; ++k) {
             Column c;
-            load_columns<TAB, PBC, 1>(B, j + k, &c);
+            load_columns<TAB, FORM, 1>(B, j + k, &c);
             step<1>(&c, chm >> k);
         }
     }
@@ -369,7 +409,7 @@ struct EnergyOp {
     {
         for (int k = 0; k < n; ++k) {
             Column c;
-            load_columns<TAB, PBC, 1>(B, j + k, &c);
+            load_columns<TAB, FORM, 1>(B, j + k, &c);
             if ((c.tc >> 8) != 0) continue; // uniform
             const bool on = B.body[j + k] != r.body && !r.crow && (!diag || j + k > r.i);
             float e;
@@ -447,7 +487,7 @@ __global__ __launch_bounds__(COLS) void k_energy_full(KParams p, const int *fix,
     // this workgroup's column tiles, of all row tiles' in order
     const long long all = (long long)T * (h + 1);
     const int u0 = (int)(all * blockIdx.x / gridDim.x), u1 = (int)(all * (blockIdx.x + 1) / gridDim.x);
-    auto walk = [&](auto tab, auto pbc, auto small) {
+    auto walk = [&](auto tab, auto form, auto small) __attribute__((always_inline)) {
         double sum = 0.0;
         for (int u = u0; u < u1;) {
             const int a = u / (h + 1), bo0 = u % (h + 1), end = min(h + 1, bo0 + (u1 - u));
@@ -458,7 +498,7 @@ __global__ __launch_bounds__(COLS) void k_energy_full(KParams p, const int *fix,
             const int i = row.on ? row.i : N - 1;
             const RowFix rf = load_row_fix(row, fix + R.bead_off, fix + p.copy_beads + R.bead_off,
                                            fix + 2 * p.copy_beads + R.bead_off, N);
-            EnergyOp<decltype(tab)::value, decltype(pbc)::value, decltype(small)::value> op{
+            EnergyOp<decltype(tab)::value, decltype(form)::value, decltype(small)::value> op{
                 B, gx, gy, gz, tcs, gc, row, rf, S, ff, s_et + row.type * TSTRIDE, p.sig[S.bead_off + i],
                 (float)((double)(p.q[S.bead_off + i] * ff.c_dh) * unit), (float)((double)ff.k_dh / unit), u2h, u2l,
                 p.q[S.bead_off + i] * ff.c_dh, noncrowder_only != 0, 0.0};
@@ -474,9 +514,13 @@ __global__ __launch_bounds__(COLS) void k_energy_full(KParams p, const int *fix,
     };
     using T1 = std::true_type;
     using T0 = std::false_type;
-    const double v = wave_sum_dpp(N <= FULL_SMALL ? walk(T0{}, T0{}, T1{})
-                                  : S.box > 0.f   ? (p.sigtab ? walk(T1{}, T1{}, T0{}) : walk(T0{}, T1{}, T0{}))
-                                                  : (p.sigtab ? walk(T1{}, T0{}, T0{}) : walk(T0{}, T0{}, T0{})));
+    auto by_table = [&](auto form) __attribute__((always_inline)) {
+        return p.sigtab ? walk(T1{}, form, T0{}) : walk(T0{}, form, T0{});
+    };
+    const double v = wave_sum_dpp(N <= FULL_SMALL           ? walk(T0{}, Form<FLAT>{}, T1{})
+                                  : box_in_fractions(S.box) ? by_table(Form<FRACTION>{})
+                                  : S.box > 0.f             ? by_table(Form<IMAGE>{})
+                                                            : by_table(Form<FLAT>{}));
     if (lane == 0) s_red[wave] = v;
     __syncthreads();
     if (tid == 0) {
@@ -550,7 +594,7 @@ struct AdjFF {
 
 constexpr int ADJ_TARGET_WG = 2048; // workgroups a launch aims at
 
-template <bool TAB, bool PBC>
+template <bool TAB, CoordForm FORM>
 struct AdjointOp {
     const Beads &B;
     const float *gx, *gy, *gz; // positions, types and groups, for reads by lane
@@ -560,7 +604,7 @@ struct AdjointOp {
     const RowFix &f;
     const DevSys &S;
     const DevFF &ff;
-    const AdjFF &af;
+    float lambda;
     const float4 *erow; // of the row's type: 24 c_lj E_ij, sigma_ij^2 as above, T_ij - e0
     float s;            // the row's sigma
     float qu, kdh, ixu; // the row's charge times the Debye-Hueckel coefficient, the exponent scale and 1/xi in the
@@ -583,10 +627,10 @@ struct AdjointOp {
     {
         Term o;
         const float4 et = erow[c.tc];
-        separation<PBC>(c, r, f, o.dx, o.dy, o.dz);
+        separation<FORM>(c, r, f, S, o.dx, o.dy, o.dz);
         o.r2 = fmaxf(__builtin_fmaf(o.dx, o.dx, __builtin_fmaf(o.dy, o.dy, o.dz * o.dz)), 1e-36f);
         o.inv2 = __builtin_amdgcn_rcpf(o.r2);
-        const float s2 = sigma2_over_r2<TAB, PBC>(et, o.inv2, s, c.s, u2, u2l);
+        const float s2 = sigma2_over_r2<TAB, FORM>(et, o.inv2, s, c.s, u2, u2l);
         o.x6 = s2 * s2 * s2;
         o.kf = et.x * o.x6 * __builtin_fmaf(2.0f, o.x6, -1.0f) * o.inv2;
         if (PAR) {
@@ -599,7 +643,7 @@ struct AdjointOp {
     template <bool PAR>
     __device__ __forceinline__ void flip(Term &o, const Column &c)
     {
-        const bool f = o.x6 > 0.5f && af.lambda * erow[c.tc].w > 0.0f;
+        const bool f = o.x6 > 0.5f && lambda * erow[c.tc].w > 0.0f;
         o.kf = f ? -o.kf : o.kf;
         if (PAR) o.u = f ? 0.5f - o.u : o.u;
     }
@@ -639,13 +683,13 @@ struct AdjointOp {
         int k = 0;
         for (; k + 3 < n; k += 4) {
             Column c[4];
-            load_columns<TAB, PBC, 4>(B, j + k, c);
+            load_columns<TAB, FORM, 4>(B, j + k, c);
             two<PAR>(c, chm >> k);
             two<PAR>(c + 2, chm >> (k + 2));
         }
         for (; k < n; ++k) {
             Column c;
-            load_columns<TAB, PBC, 1>(B, j + k, &c);
+            load_columns<TAB, FORM, 1>(B, j + k, &c);
             Term a = term<PAR>(c);
             if (__any(a.x6 > 0.5f)) flip<PAR>(a, c);
             if ((chm >> k) & 1) charged<PAR>(a, c.q);
@@ -670,7 +714,7 @@ struct AdjointOp {
     {
         for (int k = 0; k < n; ++k) {
             Column c;
-            load_columns<TAB, PBC, 1>(B, j + k, &c);
+            load_columns<TAB, FORM, 1>(B, j + k, &c);
             if ((c.tc >> 8) != 0) continue; // uniform
             const int body = B.body[j + k];
             Term a = term<true>(c);
@@ -705,9 +749,10 @@ struct AdjointOp {
     }
 };
 
-__global__ __launch_bounds__(COLS) void k_adjoint_rows(KParams p, AdjFF af, int rep_first, int tiles, int split, int sub_len,
-                                                       int bead_base, size_t bead_stride, const int *fix,
-                                                       double *part_grad, double *param_part)
+// (6 waves a SIMD: 80 registers)
+__global__ __launch_bounds__(COLS, 6) void k_adjoint_rows(KParams p, AdjFF af, int rep_first, int tiles, int split,
+                                                          int sub_len, int bead_base, size_t bead_stride, const int *fix,
+                                                          double *part_grad, double *param_part)
 {
     __shared__ float4 s_et[REMC_NTYPES * TSTRIDE];
     __shared__ double s_g[WAVES - 1][3][ROWS];
@@ -734,28 +779,32 @@ __global__ __launch_bounds__(COLS) void k_adjoint_rows(KParams p, AdjFF af, int 
                                    fix + 2 * p.copy_beads + R.bead_off, N);
     __syncthreads();
     double g[3], v[3];
-    auto walk = [&](auto tab, auto pbc) {
-        AdjointOp<decltype(tab)::value, decltype(pbc)::value> op{
-            B, gx, gy, gz, p.tc + S.bead_off, gc, row, rf, S, ff, af, s_et + row.type * TSTRIDE, p.sig[S.bead_off + i],
-            (float)((double)(p.q[S.bead_off + i] * af.c_dh) * unit), (float)((double)ff.k_dh / unit),
-            (float)(1.0 / ((double)af.xi * unit)), u2h, u2l, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    const float lambda = af.lambda, xi = af.xi, c_lj = af.c_lj, c_dh = af.c_dh;
+    auto walk = [&](auto tab, auto form) __attribute__((always_inline)) {
+        AdjointOp<decltype(tab)::value, decltype(form)::value> op{
+            B, gx, gy, gz, p.tc + S.bead_off, gc, row, rf, S, ff, lambda, s_et + row.type * TSTRIDE, p.sig[S.bead_off + i],
+            (float)((double)(p.q[S.bead_off + i] * c_dh) * unit), (float)((double)ff.k_dh / unit),
+            (float)(1.0 / ((double)xi * unit)), u2h, u2l, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         for (int k = j0 / GROUP + wave; k < (j1 + GROUP - 1) / GROUP; k += WAVES) walk_group(op, B, k, row, false, S, ff);
         // column minus row: dE/dx_i is minus the sum; (dE/dr)/r times a
         // difference, both in units, is dE/dr per unit
         g[0] = -(op.ux * unit + op.ax);
         g[1] = -(op.uy * unit + op.ay);
         g[2] = -(op.uz * unit + op.az);
-        const double scale = 4.0 * (double)af.c_lj;
+        const double scale = 4.0 * (double)c_lj;
         v[0] = wave_sum_dpp(row.on ? scale * op.pl : 0.0);
-        v[1] = wave_sum_dpp(row.on ? -scale * (double)af.lambda * op.pe : 0.0);
-        v[2] = wave_sum_dpp(row.on ? op.px / (unit * (double)af.xi * (double)af.xi) : 0.0);
+        v[1] = wave_sum_dpp(row.on ? -scale * (double)lambda * op.pe : 0.0);
+        v[2] = wave_sum_dpp(row.on ? op.px / (unit * (double)xi * (double)xi) : 0.0);
     };
-    using T1 = std::true_type;
-    using T0 = std::false_type;
-    if (S.box > 0.f)
-        p.sigtab ? walk(T1{}, T1{}) : walk(T0{}, T1{});
+    auto by_table = [&](auto form) __attribute__((always_inline)) {
+        p.sigtab ? walk(std::true_type{}, form) : walk(std::false_type{}, form);
+    };
+    if (box_in_fractions(S.box))
+        by_table(Form<FRACTION>{});
+    else if (S.box > 0.f)
+        by_table(Form<IMAGE>{});
     else
-        p.sigtab ? walk(T1{}, T0{}) : walk(T0{}, T0{});
+        by_table(Form<FLAT>{});
     if (wave > 0) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) s_g[wave - 1][k][lane] = g[k];

@@ -29,8 +29,12 @@ struct DevSys {
     float box, inv_box;
     int grp_off; // groups of 16 beads of the systems before it
     int n_multi; // bodies of several beads
-    double unit; // 2^32 / box (1 without a box): units of fixed-point distances per Angstrom
+    double unit; // units of contact distances per Angstrom: 2^32 / box where they are fractions of it, else 1
 };
+
+// Boxes whose coordinates the all-pairs kernels take as 32-bit fractions
+constexpr float FIX_BOX_MAX = 1024.0f;
+__host__ __device__ inline bool box_in_fractions(float box) { return box > 0.0f && box <= FIX_BOX_MAX; }
 
 struct DevRep {
     int sys, bead_off, body_off;
