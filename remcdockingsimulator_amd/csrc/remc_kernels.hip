@@ -30,6 +30,7 @@
 #include "remc_internal.h"
 #include "remc_math.h"
 #include "remc_pair.h"
+#include "remc_slots.h"
 
 namespace remc {
 
@@ -1053,7 +1054,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
             }
             __syncthreads();
             if (s_abort) break;
-            if (coop > 1) ++n_x;
+            if (coop > 1) n_x = remc_exchanges_after_window(n_x, w, __popcll(statm));
             const int weff = s_weff;
 
             if (wave == 0) {
@@ -1391,9 +1392,9 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                 double part = 0.0;
 #pragma unroll
                 for (int w2 = 0; w2 < NW; ++w2) part += s_red[w2];
-                // slots alternate with the split-step count: a member reuses a
+                // slots alternate with the count of exchanges: a member reuses a
                 // slot only after every member has read it (they all wrote
-                // their partial of the split step in between)
+                // their partial of the exchange in between, remc_slots.h)
                 const unsigned long long tag = step & 0x7FFFFull;
                 unsigned long long *slot = slots + (n_x & 1u) * (REMC_SLOT_K * row);
                 if (lane == 0) __hip_atomic_store(slot + c, slot_pack(part, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
