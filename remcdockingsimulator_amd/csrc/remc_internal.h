@@ -35,6 +35,9 @@ struct DevSys {
 // Boxes whose coordinates the all-pairs kernels take as 32-bit fractions
 constexpr float FIX_BOX_MAX = 1024.0f;
 __host__ __device__ inline bool box_in_fractions(float box) { return box > 0.0f && box <= FIX_BOX_MAX; }
+// Whether there is a box, in whose units the MC kernel forms the distances of
+// its large moves
+__host__ __device__ inline bool box_is_unit(float inv_box) { return inv_box > 0.0f; }
 
 struct DevRep {
     int sys, bead_off, body_off;

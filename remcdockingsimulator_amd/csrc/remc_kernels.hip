@@ -757,7 +757,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
             // energy by the whole step there.
             const float w_ib = S.inv_box, w_ib2 = w_ib * w_ib;
             const float w_cut2 = ff.crow_cut2 * w_ib2, w_ck = ff.crow_k * (w_ib2 * w_ib2 * w_ib2);
-            const bool w_A = CACHE || !(w_ib > 0.0f); // in Angstrom
+            const bool w_A = CACHE || !box_is_unit(w_ib); // in Angstrom
             auto crow_limit = [&](float4 o, float4 n) {
                 const float lim2 = crowder_screen2(o, n, S, ff);
                 return w_A ? lim2 : lim2 * w_ib2;
@@ -1216,7 +1216,10 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                 }
             }
             const bool cr0 = crow_m || (tcj[0] >> 8) != 0, cr1 = crow_m || (tcj[1] >> 8) != 0;
-            if (__all(!cr0 && !(on[1] && cr1))) {
+            // (without a box the passes in box units have no unit: the last form below;
+            // part of the votes, since a branch of its own costs registers)
+            const bool in_units = box_is_unit(S.inv_box);
+            if (__all(in_units && !cr0 && !(on[1] && cr1))) {
                 // Every active lane's partners are non-crowder beads (a partner
                 // that is off repeats partner 0 and is masked out), the common
                 // case: the four terms of a moved bead (old and new position
@@ -1305,7 +1308,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                     fast_pass(std::false_type{});
                 continue;
             }
-            if (__all(cr0 && (!on[1] || cr1))) {
+            if (__all(in_units && cr0 && (!on[1] || cr1))) {
                 // every active lane's pairs are crowder pairs (the moved body or
                 // both partners are crowders): the same four-chain form with
                 // the crowder term only, in box units (cutoff^2 / box^2,
