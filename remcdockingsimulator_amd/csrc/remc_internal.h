@@ -35,9 +35,12 @@ struct DevSys {
 // Boxes whose coordinates the all-pairs kernels take as 32-bit fractions
 constexpr float FIX_BOX_MAX = 1024.0f;
 __host__ __device__ inline bool box_in_fractions(float box) { return box > 0.0f && box <= FIX_BOX_MAX; }
-// Whether there is a box, in whose units the MC kernel forms the distances of
-// its large moves
-__host__ __device__ inline bool box_is_unit(float inv_box) { return inv_box > 0.0f; }
+// Boxes in whose units the MC kernel forms the distances of its large moves:
+// there must be one, and the crowder term's sixth powers must be normal numbers
+// (in a box of 1e6 A the constant is above 1e-33 and the power below 1e38 beyond
+// 0.4 A; at 1e7 A both leave single precision).
+constexpr float UNIT_BOX_MAX = 1.0e6f;
+__host__ __device__ inline bool box_is_unit(float inv_box) { return inv_box >= 1.0f / UNIT_BOX_MAX; }
 
 struct DevRep {
     int sys, bead_off, body_off;

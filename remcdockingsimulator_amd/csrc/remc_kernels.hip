@@ -1216,8 +1216,8 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                 }
             }
             const bool cr0 = crow_m || (tcj[0] >> 8) != 0, cr1 = crow_m || (tcj[1] >> 8) != 0;
-            // (without a box the passes in box units have no unit: the last form below;
-            // part of the votes, since a branch of its own costs registers)
+            // (without a box that can be the unit, the last form below; part of the
+            // votes, since a branch of its own costs registers)
             const bool in_units = box_is_unit(S.inv_box);
             if (__all(in_units && !cr0 && !(on[1] && cr1))) {
                 // Every active lane's partners are non-crowder beads (a partner
