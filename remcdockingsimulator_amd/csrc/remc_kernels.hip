@@ -750,11 +750,13 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
             const int wv = __builtin_amdgcn_readfirstlane(wave);
             const unsigned long long ma = __ballot(wk_l && rank_l == wv), mb = __ballot(wk_l && rank_l == wv + NW);
             int ka = ma ? (int)__builtin_ctzll(ma) : WK, kb = mb ? (int)__builtin_ctzll(mb) : WK;
-            // The crowder terms of a one-bead move from o to n.  Without the
-            // cache they are the single steps' own (box units about o): such
+            // The crowder terms of a one-bead crowder's move from o to n.  Without
+            // the cache they are the single steps' own (box units about o): such
             // contexts took single steps where windows needed the cache, and a
             // distance that rounds to the other side of the cutoff changes an
-            // energy by the whole step there.
+            // energy by the whole step there.  The corrections of such a slot
+            // take the same form, so that they see every change of its dE0.
+            // (Bodies of 2 to SPEC_MAX beads are in Angstrom with and without.)
             const float w_ib = S.inv_box, w_ib2 = w_ib * w_ib;
             const float w_cut2 = ff.crow_cut2 * w_ib2, w_ck = ff.crow_k * (w_ib2 * w_ib2 * w_ib2);
             const bool w_A = CACHE || !box_is_unit(w_ib); // in Angstrom
@@ -773,6 +775,11 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                 return dist2_unit(u.x, u.y, u.z, crow_unit(at.x, at.y, at.z, o));
             };
             auto crow_term = [&](float r2) { return w_A ? pair_crowder(r2, ff) : pair_crowder_u(r2, w_cut2, w_ck); };
+            // crowder term of a slot's bead, moved from o, at `at` with a bead at b;
+            // lone: the slot moves a one-bead crowder
+            auto crow_pair = [&](float4 b, float4 o, float4 at, bool lone) {
+                return !w_A && lone ? crow_term(crow_r2(b.x, b.y, b.z, o, at)) : pair_crowder(dist2(b.x, b.y, b.z, at, S), ff);
+            };
             if (kb < w && s_draw[off + ka].nm == 1 && s_draw[off + kb].nm == 1 &&
                 ((s_wtc[ka * SPEC_MAX] & s_wtc[kb * SPEC_MAX]) >> 8) != 0) {
                 // both slots of the wave move one crowder bead: one pass over the
@@ -877,7 +884,8 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                     // (read ahead of the tests, in one round of LDS reads)
                     const int bj = s_draw[off + jj].body, bk = s_draw[off + kk].body;
                     const int nmj = s_draw[off + jj].nm, nmk = s_draw[off + kk].nm;
-                    const bool crow = ((s_wtc[jj * SPEC_MAX] | s_wtc[kk * SPEC_MAX]) >> 8) != 0;
+                    const int tcj = s_wtc[jj * SPEC_MAX], tck = s_wtc[kk * SPEC_MAX];
+                    const bool crow = ((tcj | tck) >> 8) != 0, lone = nmk == 1 && (tck >> 8) != 0;
                     const unsigned int chain = s_wchain[kk];
                     const float4 o0 = s_wold[kk * SPEC_MAX], n0 = s_wnew[kk * SPEC_MAX];
                     const float4 O0 = s_wold[jj * SPEC_MAX], N0 = s_wnew[jj * SPEC_MAX];
@@ -888,10 +896,8 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                     const bool apart = bj != bk && ((statm >> jj) & 1ull) == 0ull && ((statm >> kk) & 1ull) == 0ull;
                     if (apart && crow && nmj == 1 && nmk == 1) {
                         // one-bead bodies, the common case: four crowder terms
-                        const float e_nn = pair_crowder(dist2(N0.x, N0.y, N0.z, n0, S), ff);
-                        const float e_on = pair_crowder(dist2(N0.x, N0.y, N0.z, o0, S), ff);
-                        const float e_no = pair_crowder(dist2(O0.x, O0.y, O0.z, n0, S), ff);
-                        const float e_oo = pair_crowder(dist2(O0.x, O0.y, O0.z, o0, S), ff);
+                        const float e_nn = crow_pair(N0, o0, n0, lone), e_on = crow_pair(N0, o0, o0, lone);
+                        const float e_no = crow_pair(O0, o0, n0, lone), e_oo = crow_pair(O0, o0, o0, lone);
                         touches = (e_nn - e_on) - (e_no - e_oo) != 0.0f;
                     } else if (apart) {
                         float acc = 0.0f, comp = 0.0f;
@@ -902,10 +908,10 @@ __global__ __launch_bounds__(BLOCK) void k_mc(KParams p, int nsteps)
                                 const float4 O = s_wold[jj * SPEC_MAX + l], Nn = s_wnew[jj * SPEC_MAX + l];
                                 float e_nn, e_on, e_no, e_oo;
                                 if (crow) {
-                                    e_nn = pair_crowder(dist2(Nn.x, Nn.y, Nn.z, n, S), ff);
-                                    e_on = pair_crowder(dist2(Nn.x, Nn.y, Nn.z, o, S), ff);
-                                    e_no = pair_crowder(dist2(O.x, O.y, O.z, n, S), ff);
-                                    e_oo = pair_crowder(dist2(O.x, O.y, O.z, o, S), ff);
+                                    e_nn = crow_pair(Nn, o, n, lone);
+                                    e_on = crow_pair(Nn, o, o, lone);
+                                    e_no = crow_pair(O, o, n, lone);
+                                    e_oo = crow_pair(O, o, o, lone);
                                 } else {
                                     const int sl = jj * SPEC_MAX + l;
                                     const float eij = s_et2[ti * REMC_NTYPES + (s_wtc[sl] & 0xff)].x;
