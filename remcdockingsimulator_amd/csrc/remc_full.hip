@@ -574,9 +574,7 @@ hipError_t launch_energy_full(const KParams &p, int n_rep, int max_beads, int *f
 // term), dE/dx_i of their row bead and, over the unordered pairs (those whose
 // column belongs to a later body), the parameter derivatives
 // dE/dlambda = sum dE/dE_ij (T_ij - e0), dE/de0 = -lambda sum dE/dE_ij and
-// dE/dxi = sum DH r / xi^2.  Two columns' products meet in one FMA (two
-// roundings, as the two products have) before they are added in FP64.  The
-// waves' row gradients are added through LDS in wave order and written once per
+// dE/dxi = sum DH r / xi^2.  The waves' row gradients are added through LDS in wave order and written once per
 // (sub-range, bead), their parameter sums once per workgroup.
 // k_adjoint_bodies: one wave per (replica, body) adds each bead's sub-range
 // partials in sub-range order, forms F = -sum dE/dx_i and the torque
@@ -618,7 +616,7 @@ struct AdjointOp {
     __device__ __forceinline__ bool crowders() const { return true; }
     __device__ __forceinline__ bool general() const { return false; }
     struct Term {
-        float dx, dy, dz, r2, inv2, x6, kf, u, t0, dhr;
+        float dx, dy, dz, r2, inv2, x6, kf, u, t0;
     };
     // One contact pair without its charges: (dE/dr)/r in units^-2, and with PAR
     // the parameter terms.
@@ -637,7 +635,6 @@ struct AdjointOp {
             o.t0 = et.w;
             o.u = -(o.x6 * (o.x6 - 1.0f));
         }
-        o.dhr = 0.0f;
         return o;
     }
     template <bool PAR>
@@ -647,17 +644,37 @@ struct AdjointOp {
         o.kf = f ? -o.kf : o.kf;
         if (PAR) o.u = f ? 0.5f - o.u : o.u;
     }
-    template <bool PAR>
-    __device__ __forceinline__ void charged(Term &o, float qc)
+    // adds the Debye-Hueckel derivative; the term itself times r
+    __device__ __forceinline__ float charged(Term &o, float qc)
     {
         asm volatile("" : "+v"(o.r2)); // keeps the term behind its branch
         const float rinv = __builtin_amdgcn_rsqf(o.r2);
         const float rr = o.r2 * rinv;
         const float dh = qu * qc * __builtin_amdgcn_exp2f(rr * kdh) * rinv;
         o.kf = __builtin_fmaf(-dh * (ixu + rinv), rinv, o.kf);
-        if (PAR) o.dhr = dh * rr;
+        return dh * rr;
     }
-    // two columns: their products meet in one FMA before the FP64 sum
+    // A pair's products are formed and added in FP64 (an FMA each: seven
+    // instructions for the force, against nine for FP32 products added in FP64).
+    __device__ __forceinline__ void add_force(const Term &t)
+    {
+        const double k = (double)t.kf;
+        ux = __builtin_fma(k, (double)t.dx, ux);
+        uy = __builtin_fma(k, (double)t.dy, uy);
+        uz = __builtin_fma(k, (double)t.dz, uz);
+    }
+    __device__ __forceinline__ void add_params(const Term &t)
+    {
+        const double u = (double)t.u;
+        pl = __builtin_fma(u, (double)t.t0, pl);
+        pe += u;
+    }
+    template <bool PAR>
+    __device__ __forceinline__ void add_charge(float dhr)
+    {
+        if (PAR) px += (double)dhr;
+    }
+    // two columns: independent chains, one test of the near terms
     template <bool PAR>
     __device__ __forceinline__ void two(const Column *c, int ch)
     {
@@ -666,15 +683,13 @@ struct AdjointOp {
             flip<PAR>(a, c[0]);
             flip<PAR>(b, c[1]);
         }
-        if (ch & 1) charged<PAR>(a, c[0].q);
-        if (ch & 2) charged<PAR>(b, c[1].q);
-        ux += (double)__builtin_fmaf(b.kf, b.dx, a.kf * a.dx);
-        uy += (double)__builtin_fmaf(b.kf, b.dy, a.kf * a.dy);
-        uz += (double)__builtin_fmaf(b.kf, b.dz, a.kf * a.dz);
+        if (ch & 1) add_charge<PAR>(charged(a, c[0].q));
+        if (ch & 2) add_charge<PAR>(charged(b, c[1].q));
+        add_force(a);
+        add_force(b);
         if (PAR) {
-            pl += (double)__builtin_fmaf(b.u, b.t0, a.u * a.t0);
-            pe += (double)a.u + (double)b.u;
-            if (ch & 3) px += (double)(a.dhr + b.dhr);
+            add_params(a);
+            add_params(b);
         }
     }
     template <bool PAR>
@@ -692,15 +707,9 @@ struct AdjointOp {
             load_columns<TAB, FORM, 1>(B, j + k, &c);
             Term a = term<PAR>(c);
             if (__any(a.x6 > 0.5f)) flip<PAR>(a, c);
-            if ((chm >> k) & 1) charged<PAR>(a, c.q);
-            ux += (double)(a.kf * a.dx);
-            uy += (double)(a.kf * a.dy);
-            uz += (double)(a.kf * a.dz);
-            if (PAR) {
-                pl += (double)(a.u * a.t0);
-                pe += (double)a.u;
-                px += (double)a.dhr;
-            }
+            if ((chm >> k) & 1) add_charge<PAR>(charged(a, c.q));
+            add_force(a);
+            if (PAR) add_params(a);
         }
     }
     __device__ __forceinline__ void contact(int j, int n, int chm, bool later)
@@ -719,15 +728,12 @@ struct AdjointOp {
             const int body = B.body[j + k];
             Term a = term<true>(c);
             flip<true>(a, c);
-            if ((chm >> k) & 1) charged<true>(a, c.q);
+            const float dhr = (chm >> k) & 1 ? charged(a, c.q) : 0.0f;
             if (body != r.body && !r.crow) {
-                ux += (double)(a.kf * a.dx);
-                uy += (double)(a.kf * a.dy);
-                uz += (double)(a.kf * a.dz);
+                add_force(a);
                 if (body > r.body) { // each unordered pair once for the parameter sums
-                    pl += (double)(a.u * a.t0);
-                    pe += (double)a.u;
-                    px += (double)a.dhr;
+                    add_params(a);
+                    add_charge<true>(dhr);
                 }
             }
         }
