@@ -246,6 +246,8 @@ def config1_full(threads):
     synth.load_engine(e2, wl, seed=SEED)
     e2.set_mc_block(e.mc_block())
     e2.set_mc_coop(e.mc_coop())
+    if e.mc_by_cost()[0]:
+        e2.set_mc_by_cost()
     e.close()
     e2.synchronize()
     t0 = time.perf_counter()
@@ -380,8 +382,8 @@ def main(argv=None):
     e.run(warm, spl)
     e.synchronize()
     first_timed = rec_n + warm * spl
-    mc_block, mc_coop = e.mc_block(), e.mc_coop()
-    log("mc block:", mc_block, "workgroups per replica:", mc_coop)
+    mc_block, mc_coop, (mc_by_cost, mc_most) = e.mc_block(), e.mc_coop(), e.mc_by_cost()
+    log("mc block:", mc_block, "workgroups per replica:", "by cost, up to %d" % mc_most if mc_by_cost else mc_coop)
 
     # ---------------------------------------------------------- timed ----
     e.timing_enable(True)
@@ -563,7 +565,8 @@ def main(argv=None):
         "data": "synthetic (seeded self-avoiding chains, uniform residue types, seeded [-0.6,0] kT contact table)",
         "config": {"workload": workload_label(cid, wl), "replicas": R, "steps_per_exchange": spl,
                    "timed_mc_steps_per_replica": pl["timed_mc_steps_per_replica"],
-                   "mc_block": mc_block, "mc_workgroups_per_replica": mc_coop, "form": "batched persistent dE kernel, hipGraph rounds"},
+                   "mc_block": mc_block, "mc_workgroups_per_replica": mc_coop,
+                   "mc_most_workgroups_per_replica": mc_most, "form": "batched persistent dE kernel, hipGraph rounds"},
         "mc_steps_per_s": steps_total / wall,
         "pair_interactions_per_s": value,
         "kernel_pair_interactions_per_s": kernel_pairs_per_s,

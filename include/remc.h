@@ -291,7 +291,7 @@ REMC_API int remc_get_mc_block(remc_ctx *ctx, int *block);
 REMC_API int remc_get_fb_block(remc_ctx *ctx, int *block);
 /* Workgroups per replica of the MC kernel (0 = autotune; else 1, 2, 4 or 8).
  * The autotuner may give the replicas of unequal systems 1 to 32 each, by the
- * systems' cost; remc_get_mc_coop is then 1.
+ * systems' cost (remc_get_mc_by_cost); remc_get_mc_coop is then 1.
  * With more than one, each workgroup keeps a private copy of its replica's
  * state, evaluates dE over a slice of the partner beads, and the members add
  * their partials through device memory (once per split step, once per
@@ -299,6 +299,17 @@ REMC_API int remc_get_fb_block(remc_ctx *ctx, int *block);
  * (checked). */
 REMC_API int remc_set_mc_coop(remc_ctx *ctx, int coop);
 REMC_API int remc_get_mc_coop(remc_ctx *ctx, int *coop);
+/* Whether the MC kernel's workgroups follow the systems' cost, the third part of
+ * its configuration beside the workgroup size and the number per replica.
+ * remc_set_mc_by_cost(1) asks for it: at the workgroup size set (or the fastest,
+ * with size 0), for a context of several systems; where none can be made the
+ * configuration is tuned as with remc_set_mc_coop(0).  0 asks for the autotuned
+ * one again, and so does remc_set_mc_coop afterwards for its own.  The getter
+ * says what is in force (0 before the first MC call) and, if most is not NULL,
+ * the largest number of workgroups of a replica.  A configuration is carried to
+ * another context by setting the size, then the number, then this if it was 1. */
+REMC_API int remc_set_mc_by_cost(remc_ctx *ctx, int enable);
+REMC_API int remc_get_mc_by_cost(remc_ctx *ctx, int *by_cost, int *most);
 /* MC kernel tuning: lds_cache = 0 keeps partner beads in HBM instead of the
  * LDS cache; split_min_pairs (> 0) is the pair-term count from which a move is
  * split across cooperating workgroups (default 8192; 0 keeps the current). */

@@ -99,6 +99,8 @@ SIGNATURES = {
     "remc_get_mc_block": (ctypes.c_int, [_vp, _ip]),
     "remc_set_mc_coop": (ctypes.c_int, [_vp, ctypes.c_int]),
     "remc_get_mc_coop": (ctypes.c_int, [_vp, _ip]),
+    "remc_set_mc_by_cost": (ctypes.c_int, [_vp, ctypes.c_int]),
+    "remc_get_mc_by_cost": (ctypes.c_int, [_vp, _ip, _ip]),
     "remc_set_mc_tuning": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int]),
     "remc_set_mc_window": (ctypes.c_int, [_vp, ctypes.c_int]),
 }

@@ -178,9 +178,11 @@ struct remc_ctx {
     struct McPlan {
         int coop, block, grid, row;
         McWg *wg;
+        int most = 0; // largest number of workgroups of a replica (coop = 0)
     };
     std::vector<McPlan> plans;
-    bool mc_balanced = false; // autotuned: the members follow the systems' cost (mc_coop is then 1)
+    bool mc_balanced = false; // in force: the members follow the systems' cost (mc_coop is then 1)
+    bool mc_by_cost = false;  // asked for (remc_set_mc_by_cost)
     const McWg *synced = nullptr; // the workgroups whose state copies hold the current conformation (null: none but the canonical)
     int n_cu = 0;
     int lds_per_block = 0, lds_per_cu = 0;
@@ -956,6 +958,7 @@ int balanced_plan(remc_ctx *c, int block, remc_ctx::McPlan *out)
     }
     pl.grid = 0;
     std::vector<McWg> wg;
+    pl.most = *std::max_element(coop.begin(), coop.end());
     if (members > R) {
         pl.grid = (int)place();
         wg.assign(pl.grid, McWg{-1, 0, 0, 0, 0, 0});
@@ -1072,6 +1075,18 @@ struct StateGuard {
 
 int autotune_mc(remc_ctx *c)
 {
+    const bool several = c->systems.size() > 1;
+    const bool by_cost = c->mc_by_cost && several;
+    if (by_cost && c->mc_block) { // nothing to choose if there is such a plan
+        remc_ctx::McPlan pl;
+        const int rc = balanced_plan(c, c->mc_block, &pl);
+        if (rc != REMC_OK) return rc;
+        if (pl.grid > 0) {
+            c->mc_coop = 1;
+            c->mc_balanced = true;
+            return REMC_OK;
+        }
+    }
     // time each (workgroup size, workgroups per replica) on the live state, then restore it exactly
     StateGuard st(c);
     int rc = st.save();
@@ -1108,39 +1123,41 @@ int autotune_mc(remc_ctx *c)
         }
         return REMC_OK;
     };
-    for (int bi = 0; bi < 3; ++bi) {
-        const int blk = blocks[bi];
-        if (c->mc_block && blk != c->mc_block) continue;
-        int cmax = 1;
-        rc = max_coop(c, blk, &cmax);
-        if (rc != REMC_OK) return rc;
-        float ms = 0.f;
-        remc_ctx::McPlan pl;
-        for (int coop = 1; coop <= cmax; coop *= 2) {
-            if (c->mc_coop && coop != c->mc_coop) continue;
-            rc = uniform_plan(c, coop, &pl);
-            if (rc == REMC_OK) rc = trial(blk, pl, &ms);
+    // plans by cost alone where they are asked for and there is one, else all
+    for (int pass = by_cost ? 0 : 1; pass < 2 && best == 1e30; ++pass)
+        for (int bi = 0; bi < 3; ++bi) {
+            const int blk = blocks[bi];
+            if (c->mc_block && blk != c->mc_block) continue;
+            int cmax = 1;
+            rc = max_coop(c, blk, &cmax);
+            if (rc != REMC_OK) return rc;
+            float ms = 0.f;
+            remc_ctx::McPlan pl;
+            for (int coop = 1; pass == 1 && coop <= cmax; coop *= 2) {
+                if (c->mc_coop && coop != c->mc_coop) continue;
+                rc = uniform_plan(c, coop, &pl);
+                if (rc == REMC_OK) rc = trial(blk, pl, &ms);
+                if (rc != REMC_OK) return rc;
+                if (ms < best) {
+                    best = ms;
+                    best_block = blk;
+                    best_coop = coop;
+                    best_balanced = false;
+                }
+            }
+            if (!several || c->mc_coop) continue;
+            rc = balanced_plan(c, blk, &pl);
+            if (rc != REMC_OK) return rc;
+            if (pl.grid == 0) continue;
+            rc = trial(blk, pl, &ms);
             if (rc != REMC_OK) return rc;
             if (ms < best) {
                 best = ms;
                 best_block = blk;
-                best_coop = coop;
-                best_balanced = false;
+                best_coop = 1;
+                best_balanced = true;
             }
         }
-        if (c->systems.size() < 2 || c->mc_coop) continue;
-        rc = balanced_plan(c, blk, &pl);
-        if (rc != REMC_OK) return rc;
-        if (pl.grid == 0) continue;
-        rc = trial(blk, pl, &ms);
-        if (rc != REMC_OK) return rc;
-        if (ms < best) {
-            best = ms;
-            best_block = blk;
-            best_coop = 1;
-            best_balanced = true;
-        }
-    }
     c->mc_block = best_block;
     c->mc_coop = best_coop;
     c->mc_balanced = best_balanced;
@@ -2374,7 +2391,31 @@ int remc_set_mc_coop(remc_ctx *c, int coop)
         return fail(REMC_ERR_ARG, "workgroups per replica must be 0, 1, 2, 4 or 8");
     c->mc_coop = coop;
     c->mc_balanced = false;
+    c->mc_by_cost = false;
     destroy_graph(c);
+    return REMC_OK;
+}
+
+int remc_set_mc_by_cost(remc_ctx *c, int enable)
+{
+    CHECK_CTX(c);
+    c->mc_by_cost = enable != 0;
+    c->mc_coop = 0;
+    c->mc_balanced = false;
+    destroy_graph(c);
+    return REMC_OK;
+}
+
+int remc_get_mc_by_cost(remc_ctx *c, int *by_cost, int *most)
+{
+    CHECK_CTX(c);
+    if (!by_cost) return fail(REMC_ERR_ARG, "null output");
+    *by_cost = c->mc_balanced ? 1 : 0;
+    if (most) {
+        *most = c->mc_coop;
+        for (const auto &pl : c->plans)
+            if (c->mc_balanced && pl.coop == 0 && pl.block == c->mc_block) *most = pl.most;
+    }
     return REMC_OK;
 }
 

@@ -181,6 +181,16 @@ class Engine:
         self._chk(self.lib.remc_get_mc_coop(self.ctx, ctypes.byref(b)), "remc_get_mc_coop")
         return b.value
 
+    def set_mc_by_cost(self, enable=True):
+        """MC workgroups by the systems' cost (remc_set_mc_by_cost)."""
+        self._chk(self.lib.remc_set_mc_by_cost(self.ctx, 1 if enable else 0), "remc_set_mc_by_cost")
+
+    def mc_by_cost(self):
+        """Whether the MC workgroups follow the systems' cost, and the largest number of a replica."""
+        on, most = ctypes.c_int(), ctypes.c_int()
+        self._chk(self.lib.remc_get_mc_by_cost(self.ctx, ctypes.byref(on), ctypes.byref(most)), "remc_get_mc_by_cost")
+        return bool(on.value), most.value
+
     def set_mc_tuning(self, lds_cache=True, split_min_pairs=0):
         self._chk(self.lib.remc_set_mc_tuning(self.ctx, 1 if lds_cache else 0, int(split_min_pairs)),
                   "remc_set_mc_tuning")
