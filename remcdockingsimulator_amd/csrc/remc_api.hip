@@ -318,8 +318,10 @@ std::mutex g_split_mu;
 // 32-bit words of an adjoint of all replicas that comes back in pinned memory, at most
 constexpr size_t PIN_ADJ_WORDS = 1 << 18;
 
-// Grows the pinned memory to at least `bytes`.  Every call that uses it waits
-// for the device before it returns, so nothing in flight refers to it here.
+// Grows the pinned memory to at least `bytes`.  Coherent: results are read as
+// soon as their flag is seen, before the kernel that stored them has ended.
+// Every call that uses it waits for its results before it returns, so nothing in
+// flight refers to it here.
 int pin_reserve(remc_ctx *c, size_t bytes)
 {
     const size_t words = (bytes + 3) / 4;
@@ -327,7 +329,7 @@ int pin_reserve(remc_ctx *c, size_t bytes)
     if (c->h_pin) HIP_TRY(hipHostFree(c->h_pin));
     c->h_pin = nullptr;
     c->pin_words = 0;
-    HIP_TRY(hipHostMalloc((void **)&c->h_pin, 4 * words, hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void **)&c->h_pin, 4 * words, hipHostMallocCoherent));
     c->pin_words = words;
     return REMC_OK;
 }
@@ -535,7 +537,7 @@ int finalize(remc_ctx *c)
     c->slot_row = REMC_MAX_COOP;
     HIP_TRY(dalloc(&c->d_err, (size_t)1));
     HIP_TRY(dalloc(&c->d_count, (size_t)1));
-    HIP_TRY(hipHostMalloc((void **)&c->h_flag, sizeof(uint32_t), hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void **)&c->h_flag, sizeof(uint32_t), hipHostMallocCoherent));
     *c->h_flag = 0;
     HIP_TRY(dalloc(&c->d_E, (size_t)R));
     HIP_TRY(dalloc(&c->d_T, (size_t)R));
