@@ -880,17 +880,19 @@ int max_coop(remc_ctx *c, int block, int *out)
 // chains and few crowders (most of its moves are chains') costs a hundred times
 // the pair terms of a light one's: with as many workgroups for every replica a
 // few replicas held the launch while the rest of the device idled.  64 systems
-// of 500-4000 beads, 512 replicas, 500 steps: 27.8 ms with one workgroup each
-// (the most that fits), 6.9 ms with 1-16 members on 1024 workgroups.  The
-// estimate of a step is its moves' mean pair terms, those of windows and split
-// moves over the members, at MC_TERMS_US terms a microsecond and 256 threads,
-// and MC_EXCHANGE_US for each split move's exchange; the slowest system's
-// replicas take one member more while the grid stays co-resident and the copies
-// fit.  (0.5, 2 and 8 us an exchange: 6.9, 7.3 and 7.2 ms; doubling instead of
+// of 500-4000 beads, 512 replicas, 500 steps: 20.4 ms with one workgroup each
+// (the most that fits), 6.9 ms with 1-16 members on 1024 workgroups (7.1-8.2 from
+// pass to pass of a longer run).  The estimate of a step is its moves' mean pair
+// terms, those of windows and split moves over the members, at MC_TERMS_US terms
+// a microsecond and 256 threads, and MC_EXCHANGE_US for each split move's
+// exchange; the slowest system's replicas take one member more while the grid
+// stays co-resident and the copies fit.  (0.5, 2 and 8 us an exchange: 6.9, 7.3 and 7.2 ms; doubling instead of
 // one more: 7.35 ms.)  Members of a replica are placed on one XCD (workgroup b
 // runs on XCD b mod 8), each XCD's in order of cost, so that the costly ones
 // start first and on different CUs.  No plan (grid 0) where that leaves one
-// workgroup per replica.
+// workgroup per replica.  Both constants were fitted on that one mix of systems;
+// the plan is one more candidate of the tuner, which times it, so that on another
+// mix a poor estimate costs speed at most.
 constexpr double MC_TERMS_US = 1300.0; // a quarter of a CU
 constexpr double MC_EXCHANGE_US = 0.5;
 

@@ -51,11 +51,13 @@ constexpr int TSTRIDE = REMC_NTYPES + 1; // row stride of the type tables in LDS
 // to L 2^-32, so a difference of two is off by up to that much, where the
 // difference of two near floats is exact: at 1024 A it is 2^-22 A, what a
 // difference of 4-8 A (a contact's) may be off by when rounded to 24 bits, and it
-// grows with the box.  Mean square error of (sigma/r)^6, pairs 4.5-8 A apart
+// grows with the box.  Root mean square error of (sigma/r)^6, pairs 4.5-8 A apart
 // anywhere in the box (emulated, reciprocals off by half a unit): 2.2e-7 at
 // 150 A, 2.3e-7 at 600, 2.5e-7 at 1000, 5.1e-7 at 5000, 9.5e-5 at 1e6 A; float
 // differences 1.8e-7 in any box, and 3.0e-7 with a squared reciprocal root, as
-// the moves' terms have.
+// the general form of a term has (pair_lj_dh).  Fractions take two instructions
+// less an axis: 64 x 11000 beads 1.74 ms an energy launch and 5.04 an adjoint's,
+// 1.84 and 5.25 with float differences; 32 x 1300 beads 43.4 and 83 us with both.
 enum CoordForm {
     FRACTION, // fractions of the box
     IMAGE,    // float differences, nearest image
@@ -306,15 +308,19 @@ static void launch_fix(const KParams &p, int rep_first, int n_rep, int max_beads
 // T; the last only for a < T/2 when T is even), so every unordered tile pair is
 // visited once and every row tile has the same work.  A workgroup takes an even
 // share of the T (T/2 + 1) column tiles and writes one FP64 partial.
-// 32 x 1300 beads: 55 -> 33 us; 64 x 11000 beads: 2.64 -> 1.77 ms (40.5M contact
-// pairs a replica at 24 VALU instructions a wave's 64 of them, 92% of the issue
-// slots; 256-bead tiles staged in LDS took 35 and lost a quarter to padding).
+// 32 x 1300 beads: 55 -> 34 us; 64 x 11000 beads: 2.64 -> 1.74 ms (39.8M contact
+// pairs a replica at 25.7 VALU instructions a wave's 64 of them, one every 3.9
+// cycles of a SIMD, where one takes four; 256-bead tiles staged in LDS lost a
+// quarter to padding).
 // A system of up to FULL_SMALL beads forms its contact pairs from float
-// differences, as the MC kernels form their energies.  A few dilute chains'
-// energy is what is left of terms that nearly cancel, so that a total of other
-// terms than the moves' would show as much of its rounding as of the energy.
-// Such a launch is all latency: 8 replicas of 100 beads take 16.0 us in this form
-// and 15.7 in the other, of 250 beads 17.4 and 17.7.
+// differences by the moves' own operations (pair_lj_dh), so that its total and
+// the sums of its moves' dE are made of the same terms: a few chains that are
+// apart have an energy that is what is left of terms that nearly cancel, and in
+// other terms it would differ by their rounding.  The terms are no more exact,
+// and it can happen at any size; the line is where that form stops being cheap.
+// A launch of 8 or 32 replicas, in us, this form and the walk: 100 beads 17.9 and
+// 17.4, 200 beads 18.4 and 17.5, 256 beads 19 and 16, 320 beads 19 and 16, 1300
+// beads 32-70 and 26-44.
 constexpr int FULL_SMALL = 256;
 
 template <bool TAB, CoordForm FORM, bool SMALL>
@@ -582,7 +588,8 @@ hipError_t launch_energy_full(const KParams &p, int n_rep, int max_beads, int *f
 // wave of each replica adds the parameter partials.  The result does not
 // depend on scheduling.  Sub-ranges are only cut when the launch holds fewer
 // than ADJ_TARGET_WG (row tile, replica) workgroups.
-// 32 x 1300 beads: 87 + 14 -> 66 + 6 us; 64 x 11000 beads: 8.15 + 0.06 -> 4.7 ms.
+// 32 x 1300 beads: 87 + 14 -> 70 + 6 us; 64 x 11000 beads: 8.15 + 0.06 -> 5.0 ms
+// (39 VALU instructions a wave's 64 ordered pairs, one every 3.7 cycles).
 // --------------------------------------------------------------------------
 struct AdjFF {
     float t0[REMC_NTYPES * REMC_NTYPES]; // T_ij - e0

@@ -139,8 +139,6 @@ hipError_t launch_mc_fb(const KParams &p, int n_rep, int nsteps, int block, int 
 hipError_t mc_fb_max_active_per_cu(const KParams &p, int block, int *out);
 size_t mc_fb_dynamic_lds(const KParams &p);
 hipError_t mc_max_active_per_cu(const KParams &p, int block, int *out);
-// full energies of n_rep replicas of at most max_beads beads: fix holds
-// fix_ints(...) ints (scratch), partials n_rep x full_units(...) doubles
 // How the host learns that a kernel's results are in pinned memory: the last workgroup
 // (counted in *count, which is left at 0) writes ticket to *flag.
 struct Signal {
@@ -171,6 +169,8 @@ __device__ __forceinline__ void signal_done(const Signal &sig)
     }
 }
 
+// full energies of n_rep replicas of at most max_beads beads: fix holds
+// fix_ints(...) ints (scratch), partials n_rep x full_units(...) doubles
 hipError_t launch_energy_full(const KParams &p, int n_rep, int max_beads, int *fix, double *partials, double *out,
                               int noncrowder_only, int write_E, hipStream_t s, const Signal &sig = Signal{});
 int full_units(int n_rep, int max_beads);
